@@ -50,7 +50,8 @@ else:  # run as a script
 # Candidate values per knob, searched one knob at a time in this order.
 KNOB_SPACE = {
     "sssp": {
-        "sssp.alpha": [2, 4, 8, 16],
+        "sssp.sorted": [0, 2],
+        "sssp.alpha": [2, 4, 8, 16, 32],
         "sssp.filter": [0, 1],
         "sssp.dist16": [0, 1],
         "sssp.push_dedup": [0, 1],

@@ -358,6 +358,9 @@ __device__ void bu_list_sweep(const GraphView<OffT> &g, int32_t *__restrict__ de
     }
 }
 
+// Frontier vertices above this degree are expanded by a wavefront.
+constexpr int32_t kBfsMid = 16;
+
 // Top-down expansion of one frontier row slice.
 template <int G, typename OffT>
 __device__ __forceinline__ void td_range(const GraphView<OffT> &g,
@@ -373,19 +376,20 @@ __device__ __forceinline__ void td_range(const GraphView<OffT> &g,
     for (OffT i = b + OffT(lane); i < e; i += OffT(G)) {
         int32_t v = g.adj[i];
         scanned++;
-        bool app = false;
+        const int32_t vs[1] = {v};
+        bool app[1] = {false};
         // The neighbour's bounds are read with its depth (one round trip
         // before the claim instead of one after it).
         const int32_t dv = depth[v];
         const OffT vb = g.rbeg(v), ve = g.rend(v);
         if (dv < 0 && atomicCAS(&depth[v], -1, level) == -1) {
-            app = true;
+            app[0] = true;
             if (parents) parents[v] = u;
             atomicOr(&next[v >> 5], 1u << (v & 31));
             cnt++;
             edges_acc += (unsigned long long)(ve - vb);
         }
-        push_out_append(out, g, fb, ctl, nxt, app, v, cnt, edges_acc);
+        push_out_append(out, g, fb, ctl, nxt, app, vs, cnt, edges_acc);
     }
 }
 
@@ -406,7 +410,7 @@ __device__ void td_sweep(const GraphView<OffT> &g, int32_t *__restrict__ depth,
     // for room only when the next unit could overfill the buffer.
     uint32_t staged = 0;
     for (uint32_t unit = blockIdx.x; unit < total; unit += gridDim.x) {
-        const uint32_t umax = push_unit_max(unit, nch, ctl->chunk);
+        const uint32_t umax = push_unit_max(unit, nch, u2, ctl);
         if (staged + umax > out.cap)
             staged = push_out_make_room(out, g, fb, ctl, nxt, umax, cnt, edges_acc);
         staged += umax;
@@ -629,6 +633,7 @@ __global__ __launch_bounds__(kBlock) void bfs_init_kernel(
         ctl->rem_valid = 0;
         ctl->rem_knob = rem_knob;
         ctl->chunk = chunk;
+        ctl->mid = kBfsMid;
         ctl->n = g.n;
         ctl->grid = grid;
         ctl->m = m;
@@ -640,7 +645,7 @@ __global__ __launch_bounds__(kBlock) void bfs_init_kernel(
         ctl->plan_rows = plan_rows;
         OffT b = g.rbeg(src), e = g.rend(src);
         int64_t d = int64_t(e - b);
-        int cls = degree_class(d);
+        int cls = degree_class(d, kBfsMid);
         if (cls == 3) {  // chunk descriptors: written by workgroup 0 below
             fb.cnt[0][3] = (uint32_t)((d + chunk - 1) / chunk);
             fb.cnt[0][4] = 1;

@@ -110,12 +110,14 @@ constexpr int kManyHeavyCapMax = 1024;
 
 struct Tuning {
     int grid_per_cu = 8;   // workgroups per CU of the fused / step launches
-    int sssp_alpha = 0;    // SSSP goes pull when frontier edges > m / alpha (0: by
-                           // graph shape, 4 skewed / 2 flat)
+    int sssp_alpha = 0;    // SSSP goes pull when frontier edges > m / alpha (0: 16 on
+                           // the sorted adjacency, else 4 skewed / 2 flat)
     int sssp_grid_per_cu = 4;  // workgroups per CU of the SSSP loop (at most)
     int sssp_dist16 = 2;   // SSSP pulls gather a 16-bit mirror of the distances
                            // (0 off, 1 on, 2: on for flat graphs)
     int sssp_filter = 0;   // SSSP pulls gather only neighbours changed last epoch
+    int sssp_sorted = 1;   // SSSP runs on the weight-sorted adjacency (0: never, 1: graphs
+                           // of kSortedMinEdges edges, 2: always)
     int sssp_push_dedup = 2;  // SSSP pushes deduplicate improved vertices when staging
                               // them (1) or on the spot (0); 2: by graph shape
     int sssp_stage = 0;    // per-vertex entries staged in LDS by SSSP pull sweeps
@@ -137,9 +139,9 @@ struct Tuning {
     int multi_graph = 1;   // batched SSSP/BFS: relaunch an epoch hipGraph
     int multi_grid_per_cu = 16;  // workgroups per CU of the batched sweep
     int multi_block = 256;       // threads per workgroup of the batched sweep (128-1024)
-    int sssp_delta = -1;         // single-source SSSP: bucket width (push epochs only;
-                                 // 0 off; -1: 2 x max weight / mean degree on flat
-                                 // graphs, off on skewed ones)
+    int sssp_delta = -1;         // single-source SSSP: bucket width on the sorted
+                                 // adjacency (0 off; -1: 4 x max weight / mean
+                                 // degree on flat graphs, off on skewed ones)
     int multi_push_div = 16;     // batched sweep: an epoch pushes from the flagged
                                  // vertices when they hold <= m / this edges (0: never)
     int multi_delta = -1;        // batched SSSP: improvements at or above a threshold
@@ -198,6 +200,20 @@ inline PlanConfig sssp_plan_config() {
     c.g4_threshold = std::min<int64_t>(tuning().sssp_g4_threshold, c.g16_threshold);
     c.block_threshold = std::max<int64_t>(tuning().sssp_block_threshold, c.wave_threshold);
     if (c.hub_threshold < c.block_threshold) c.hub_threshold = c.block_threshold;
+    return c;
+}
+
+// Degree classes of the sorted sweeps: rows end after a few edges, so a row
+// takes fewer lanes than in a sweep that reads all of it, and a chunk is short
+// enough that the sweeps that do read all of it end together.
+inline PlanConfig sorted_plan_config() {
+    PlanConfig c;
+    c.hub_threshold = c.block_threshold = 2048;
+    c.hub_chunk = 2048;
+    c.wave_threshold = 512;
+    c.g16_threshold = 64;
+    c.g4_threshold = 4;
+    c.min_degree = 1;
     return c;
 }
 
@@ -489,6 +505,34 @@ struct ColBlocks {
     void *dmem = nullptr;
     size_t bytes = 0;
 };
+// Edges of a whole weighted graph as (id, weight) pairs, each row in order of
+// rising weight key (see sorted.hip); rows lie where the CSR's offsets say.
+struct SortedAdj {
+    int2 *e = nullptr;  // nullptr: not built (no memory)
+    int32_t shift = 0;
+};
+constexpr int kSortKeys = 64;
+// Smaller graphs relax from the plain CSR: their epochs wait for launches, not
+// for edges, and a first query would pay for the copy (Kronecker, 1.8 M edges:
+// 0.40 -> 0.33 ms a query, but 0.53 -> 0.98 ms the first; 31 M edges: 1.13 ->
+// 0.50 ms, the first 1.83 -> 1.85 ms).
+constexpr int64_t kSortedMinEdges = int64_t(1) << 23;
+struct SortedView {
+    const int2 *e;
+    int32_t shift;
+    // Lower bound of the weights at and after an edge of weight w in its row.
+    __device__ __forceinline__ int32_t floor(int32_t w) const {
+        const int32_t k = w >> shift;
+        return (k < kSortKeys - 1 ? k : kSortKeys - 1) << shift;
+    }
+};
+// One copy for a graph and every share of it, built on first use.
+struct SortedSlot {
+    std::mutex mu;
+    bool tried = false;
+    SortedAdj adj;
+    ~SortedSlot();
+};
 // Knobs set on one graph (and every share of it): key/value pairs applied
 // over the process-wide set for the duration of each call on the graph.
 struct GraphTuning {
@@ -532,6 +576,7 @@ struct hc_graph_s {
     void *ws_multi = nullptr;
     void *ws_msbfs = nullptr;
     std::shared_ptr<hc::ColBlockSlot> cbslot = std::make_shared<hc::ColBlockSlot>();
+    std::shared_ptr<hc::SortedSlot> sortslot = std::make_shared<hc::SortedSlot>();
     std::shared_ptr<hc::GraphTuning> tune = std::make_shared<hc::GraphTuning>();
 };
 
@@ -577,6 +622,10 @@ inline GraphView<OffT> view(const hc_graph_s *g) {
 // stream s and waited for on first use); *out is NULL when the graph has
 // fewer than two blocks.
 int get_col_blocks(hc_graph_s *g, int shift, hipStream_t s, const ColBlocks **out);
+// Weight-sorted adjacency of a whole-graph handle (built on stream s and
+// waited for on first use); out->e is NULL when the graph is unweighted or
+// the copy does not fit the device.
+int get_sorted(hc_graph_s *g, hipStream_t s, SortedView *out);
 // Block shift a pull sweep of g uses under the current tuning (0: plain
 // sweep); flat: g has no hub rows (top 1% of rows hold < 5% of the edges).
 int col_shift_for(const hc_graph_s *g, bool flat);

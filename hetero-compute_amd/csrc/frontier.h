@@ -25,7 +25,7 @@
 // lane counts when expanded:
 //   chunk: deg > kHubDeg      -> one workgroup per chunk of StepCtl::chunk edges
 //   q[0] : deg > kBigDeg      -> one workgroup per vertex
-//   q[1] : deg > kMidDeg      -> one wavefront per vertex
+//   q[1] : deg > StepCtl::mid -> one wavefront per vertex
 //   q[2] : otherwise          -> kSmallLanes lanes per vertex
 // Chunks are small because a push epoch is latency-bound (each edge is a
 // dependent gather + atomic): many short chunks keep all CUs busy when the
@@ -40,7 +40,6 @@ namespace hc {
 constexpr int64_t kHubDeg = 1024;
 constexpr int64_t kMinChunkEdges = 128;  // smallest push chunk (sizes the chunk lists)
 constexpr int64_t kBigDeg = 256;
-constexpr int64_t kMidDeg = 16;
 constexpr int kSmallLanes = 8;
 constexpr int kSmallPerUnit = kBlock / kSmallLanes;
 constexpr int kTraceLen = 128;
@@ -76,16 +75,28 @@ struct StepCtl {
     int32_t rem_valid;             // BFS: the next pull reads the unvisited lists
     int32_t rem_knob;              // BFS: lanes per listed vertex, 0: no lists
     int32_t chunk;                 // edges per hub chunk of push epochs
-    // SSSP buckets (delta > 0, push epochs only): a vertex lowered to a value
-    // at or above thresh goes to the far bitmap instead of the next
-    // frontier; when a frontier comes out empty the threshold rises (by
-    // delta, doubled after a promotion that found nothing) and a promotion
-    // epoch moves the far vertices now below it into the frontier.
+    int32_t mid;                   // degree above which a push gives a vertex a wavefront
+    int32_t pad;
+    // SSSP on the weight-sorted adjacency: a lower bound of every distance
+    // that changed in the epoch before (rows at or below it, and edges that
+    // cannot beat the row's distance from it, are not looked at).
+    int32_t low;
+    int32_t sorted;                // SSSP: sweeps run on the weight-sorted adjacency
+    // SSSP buckets (delta > 0): the current bucket holds the distances in
+    // [base, thresh).  Its push epochs (or, from a heavy frontier, sweeps over
+    // the rows: a promotion epoch with settle 3) relax the edges that land in
+    // it; when a frontier comes out empty, the bucket's distances are final
+    // and its remaining edges are settled, by a push from its vertices
+    // (settle 2) or by a sweep over the rows above it (a promotion epoch with
+    // settle 1), and a promotion epoch makes the vertices of the next bucket
+    // the frontier.
+    int32_t base;
     int32_t thresh;
     int32_t delta;
-    int32_t far_step;              // the last rise of thresh
+    int32_t settle;
     int32_t promotions;            // promotion epochs run
-    long long far_live;            // upper bound of the far vertices
+    long long bucket_e;            // degree sum of this bucket's frontiers
+    long long done_e;              // and of the buckets before it
     // Device wall clock (constant rate): start of the loop, end of the last
     // epoch, and end of each traced epoch.
     long long t_start;
@@ -102,10 +113,12 @@ struct StepCtl {
 // groups (kSumStride words apart, each in its own cache line), so no counter
 // takes more than grid / kSumGroups same-address atomics; the controller
 // reads and clears them.  Slots: frontier vertices produced, their degree
-// sum, edges examined, and two algorithm-specific counts.
+// sum, edges examined, two algorithm-specific counts, and one value whose
+// maximum is taken.
 constexpr int kSumGroups = 64;
 constexpr int kSumStride = 16;
-constexpr int kSumSlots = 5;
+constexpr int kSumSlots = 6;
+constexpr int kMaxSlot = 5;
 static_assert(kSumGroups <= kWave, "one wavefront reads the counter groups");
 
 constexpr int kSumSets = 3;
@@ -124,7 +137,6 @@ struct FrontierBufs {
     int32_t *q[2][3];
     HubChunk *ch[2];
     uint32_t *bm[3];
-    uint32_t *far;             // SSSP buckets: vertices waiting for a higher threshold
     uint32_t (*cnt)[5];        // queue fill [parity][q0, q1, q2, chunks, hubs]
     int32_t words;             // bitmap words
     Partials part;             // counter set of the current epoch
@@ -151,8 +163,8 @@ struct FrontierWs {
 int frontier_ws_alloc(hc_graph_s *g, FrontierWs *ws);
 void frontier_ws_free(FrontierWs *ws);
 
-__device__ __forceinline__ int degree_class(int64_t d) {
-    return d > kHubDeg ? 3 : (d > kBigDeg ? 0 : (d > kMidDeg ? 1 : 2));
+__device__ __forceinline__ int degree_class(int64_t d, int32_t mid) {
+    return d > kHubDeg ? 3 : (d > kBigDeg ? 0 : (d > mid ? 1 : 2));
 }
 
 // Appends v (when pred) to the degree-classed queues of parity p.
@@ -168,7 +180,7 @@ __device__ __forceinline__ void frontier_append(const GraphView<OffT> &g,
     if (pred) {
         b = g.rbeg(v);
         e = g.rend(v);
-        cls = degree_class(int64_t(e - b));
+        cls = degree_class(int64_t(e - b), ctl->mid);
     }
     wave_append(fb.q[p][0], &fb.cnt[p][0], cls == 0, v);
     wave_append(fb.q[p][1], &fb.cnt[p][1], cls == 1, v);
@@ -234,37 +246,65 @@ struct PushKept {
     unsigned long long e;
 };
 
-template <typename OffT>
+// Appends v[r] where pred[r], for the N edges of a trip (one or four): one
+// slot reservation per wavefront and trip.
+template <int N, typename OffT>
 __device__ __forceinline__ void push_out_append(const PushOut &o, const GraphView<OffT> &g,
                                                 const FrontierBufs &fb, StepCtl *ctl, int p,
-                                                bool pred, int32_t v, uint32_t &kept_n,
+                                                const bool (&pred)[N],
+                                                const int32_t (&v)[N], uint32_t &kept_n,
                                                 unsigned long long &kept_e) {
-    const uint64_t m = __ballot(pred);
-    if (m == 0) return;
-    const int leader = __ffsll((unsigned long long)m) - 1;
-    uint32_t base = 0;
-    if (lane_id() == leader) base = atomicAdd(o.count, (uint32_t)__popcll(m));
-    base = __shfl(base, leader);
-    const uint32_t pos = base + (uint32_t)__popcll(m & lanemask_lt());
-    const bool fits = pos < o.cap;
-    if (pred && fits) o.buf[pos] = v;
-    bool direct = pred && !fits;
-    if (o.dedup && direct) {
-        const uint32_t bit = 1u << (v & 31);
-        direct = !(atomicOr(&o.dedup[v >> 5], bit) & bit);
-        if (direct) {
-            kept_n++;
-            kept_e += (unsigned long long)(g.rend(v) - g.rbeg(v));
-        }
+    uint64_t m[N];
+    uint32_t total = 0;
+#pragma unroll
+    for (int r = 0; r < N; r++) {
+        m[r] = __ballot(pred[r]);
+        total += (uint32_t)__popcll(m[r]);
     }
-    frontier_append(g, fb, ctl, p, direct, v);
+    if (total == 0) return;
+    const int leader = __ffsll((unsigned long long)__ballot(true)) - 1;
+    uint32_t base = 0;
+    if (lane_id() == leader) base = atomicAdd(o.count, total);
+    base = __shfl(base, leader);
+    uint32_t at = base;
+    uint32_t over = 0;  // entries past the buffer, a bit each
+#pragma unroll
+    for (int r = 0; r < N; r++) {
+        const uint32_t pos = at + (uint32_t)__popcll(m[r] & lanemask_lt());
+        if (pred[r]) {
+            if (pos < o.cap) o.buf[pos] = v[r];
+            else over |= 1u << r;
+        }
+        at += (uint32_t)__popcll(m[r]);
+    }
+    if (base + total <= o.cap) return;  // (the same in every lane)
+    // One copy of the queue append: the entries move up a register a round.
+    static_assert(N == 1 || N == 4, "entries of a trip");
+    int32_t x = v[0], x1 = v[1 % N], x2 = v[2 % N];
+    const int32_t x3 = v[3 % N];
+#pragma unroll 1
+    for (int r = 0; r < N; r++) {
+        bool direct = (over >> r) & 1u;
+        if (o.dedup && direct) {
+            const uint32_t bit = 1u << (x & 31);
+            direct = !(atomicOr(&o.dedup[x >> 5], bit) & bit);
+            if (direct) {
+                kept_n++;
+                kept_e += (unsigned long long)(g.rend(x) - g.rbeg(x));
+            }
+        }
+        frontier_append(g, fb, ctl, p, direct, x);
+        x = x1;
+        x1 = x2;
+        x2 = x3;
+    }
 }
 
 // Moves the staged entries into the queues of parity p (all threads of the
 // workgroup; after the sweep, or earlier to make room).  Returns this
 // thread's share of the kept counts when deduplicating (zero otherwise).
 template <typename OffT>
-__device__ PushKept push_out_flush(const PushOut &o, const GraphView<OffT> &g,
+__device__ __forceinline__ PushKept push_out_flush(const PushOut &o, const GraphView<OffT> &g,
                                    const FrontierBufs &fb, StepCtl *ctl, int p) {
     __shared__ uint32_t s_n[5], s_base[5];
     PushKept kept{0u, 0ull};
@@ -285,7 +325,7 @@ __device__ PushKept push_out_flush(const PushOut &o, const GraphView<OffT> &g,
             kept.n++;
             kept.e += (unsigned long long)d;
         }
-        const int c = degree_class(d);
+        const int c = degree_class(d, ctl->mid);
         if (c < 3) {
             atomicAdd(&s_n[c], 1u);
         } else {
@@ -311,7 +351,7 @@ __device__ PushKept push_out_flush(const PushOut &o, const GraphView<OffT> &g,
             v = o.buf[i];
             b = g.rbeg(v);
             e = g.rend(v);
-            c = degree_class(int64_t(e - b));
+            c = degree_class(int64_t(e - b), ctl->mid);
         }
         if (c >= 0 && c < 3) fb.q[p][c][s_base[c] + atomicAdd(&s_n[c], 1u)] = v;
         const uint32_t nch = c == 3 ? (uint32_t)((int64_t(e - b) + ck - 1) / ck) : 0u;
@@ -356,11 +396,13 @@ __device__ __forceinline__ uint32_t push_out_make_room(const PushOut &o, const G
     return 0;
 }
 
-// Entries a push unit can append: a hub chunk's edges, or at most kHubDeg
-// (a workgroup row, four wavefront rows of at most kBigDeg, or 32 small rows
-// of at most kMidDeg).
-__device__ __forceinline__ uint32_t push_unit_max(uint32_t unit, uint32_t nch, int64_t chunk) {
-    return unit < nch ? (uint32_t)chunk : (uint32_t)kHubDeg;
+// Entries a push unit can append: a hub chunk's edges, or at most kHubDeg (a
+// workgroup row, four wavefront rows of at most kBigDeg), or kSmallPerUnit
+// small rows of at most ctl->mid (units from u2 on).
+__device__ __forceinline__ uint32_t push_unit_max(uint32_t unit, uint32_t nch, uint32_t u2,
+                                                  const StepCtl *ctl) {
+    return unit < nch ? (uint32_t)ctl->chunk
+                      : (unit < u2 ? (uint32_t)kHubDeg : (uint32_t)(kSmallPerUnit * ctl->mid));
 }
 
 // Chunk descriptors of a hub source (parity 0), written by one workgroup.
@@ -369,7 +411,7 @@ __device__ __forceinline__ void write_source_chunks(const GraphView<OffT> &g,
                                                     const FrontierBufs &fb, int32_t src,
                                                     int64_t chunk) {
     const int64_t b = int64_t(g.rbeg(src)), e = int64_t(g.rend(src));
-    if (degree_class(e - b) != 3) return;
+    if (e - b <= kHubDeg) return;
     const int64_t nch = (e - b + chunk - 1) / chunk;
     for (int64_t j = threadIdx.x; j < nch; j += blockDim.x) {
         const int64_t cb = b + j * chunk;
@@ -377,13 +419,15 @@ __device__ __forceinline__ void write_source_chunks(const GraphView<OffT> &g,
     }
 }
 
-// Workgroup sums of three per-thread counters plus two per-workgroup values
-// (x, y: taken from thread 0), added into this workgroup's counter group.
+// Workgroup sums of three per-thread counters plus three per-workgroup values
+// (x, y: added, z: maximum; taken from thread 0), put into this workgroup's
+// counter group.
 __device__ __forceinline__ void write_partials(const Partials &part, uint32_t n,
                                                unsigned long long e,
                                                unsigned long long s,
                                                unsigned long long x = 0,
-                                               unsigned long long y = 0) {
+                                               unsigned long long y = 0,
+                                               unsigned long long z = 0) {
     __shared__ uint32_t s_n[kWavesPerBlock];
     __shared__ unsigned long long s_e[kWavesPerBlock], s_s[kWavesPerBlock];
 #pragma unroll
@@ -400,15 +444,16 @@ __device__ __forceinline__ void write_partials(const Partials &part, uint32_t n,
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        unsigned long long v[kSumSlots] = {0, 0, 0, x, y};
+        unsigned long long v[kSumSlots] = {0, 0, 0, x, y, z};
         for (int i = 0; i < kWavesPerBlock; i++) {
             v[0] += s_n[i];
             v[1] += s_e[i];
             v[2] += s_s[i];
         }
         unsigned long long *g = part.acc + (blockIdx.x % kSumGroups) * kSumStride;
-        for (int k = 0; k < kSumSlots; k++)
+        for (int k = 0; k < kMaxSlot; k++)
             if (v[k]) atomicAdd(&g[k], v[k]);
+        if (v[kMaxSlot]) atomicMax(&g[kMaxSlot], v[kMaxSlot]);
     }
 }
 
@@ -424,7 +469,10 @@ __device__ __forceinline__ void sum_partials(const Partials &part,
         for (int k = 0; k < kSumSlots; k++) v[k] = threadIdx.x < kSumGroups ? g[k] : 0ull;
         for (int k = 0; k < kSumSlots; k++) {
 #pragma unroll
-            for (int sh = 32; sh > 0; sh >>= 1) v[k] += __shfl_xor(v[k], sh, 64);
+            for (int sh = 32; sh > 0; sh >>= 1) {
+                const unsigned long long o = __shfl_xor(v[k], sh, 64);
+                v[k] = k == kMaxSlot ? (v[k] > o ? v[k] : o) : v[k] + o;
+            }
         }
         if (threadIdx.x == 0)
             for (int k = 0; k < kSumSlots; k++) r[k] = v[k];
@@ -550,7 +598,7 @@ __device__ void compact_body(const GraphView<OffT> &g, const FrontierBufs &fb,
         for (uint32_t x = bits; x; x &= x - 1) {
             int32_t v = w * 32 + __ffs(x) - 1;
             int64_t d = int64_t(g.rend(v) - g.rbeg(v));
-            int c = degree_class(d);
+            int c = degree_class(d, ctl->mid);
             if (c < 3) {
                 my[c]++;
             } else {
@@ -573,7 +621,7 @@ __device__ void compact_body(const GraphView<OffT> &g, const FrontierBufs &fb,
             int32_t v = w * 32 + __ffs(x) - 1;
             OffT b = g.rbeg(v), e = g.rend(v);
             int64_t d = int64_t(e - b);
-            int c = degree_class(d);
+            int c = degree_class(d, ctl->mid);
             if (c < 3) {
                 fb.q[p][c][s_base[c] + off[c]++] = v;
             } else {

@@ -117,6 +117,7 @@ int64_t *knob_ref(Tuning &t, const char *key, bool *is_int, int **iref) {
     } i32[] = {{"grid_per_cu", &t.grid_per_cu},
                {"sssp.alpha", &t.sssp_alpha},
                {"sssp.filter", &t.sssp_filter},
+               {"sssp.sorted", &t.sssp_sorted},
                {"sssp.dist16", &t.sssp_dist16},
                {"sssp.push_dedup", &t.sssp_push_dedup},
                {"sssp.stage", &t.sssp_stage},
@@ -607,6 +608,7 @@ int hc_graph_share(hc_graph_t g, hc_graph_t *out) {
     h->h_off = g->h_off;
     h->shared = true;
     h->cbslot = g->cbslot;  // one column-blocked copy for the graph and its shares
+    h->sortslot = g->sortslot;  // one weight-sorted copy
     h->tune = g->tune;      // and one set of per-graph knobs
     *out = h;
     return HC_OK;
@@ -628,6 +630,8 @@ int set_knob(Tuning &t, const char *key, int64_t value) {
                           !strcmp(key, "msbfs.on");
         if (!strcmp(key, "sssp.dist16"))
             HC_CHECK_ARG(value >= 0 && value <= 2, "sssp.dist16 must be 0, 1 or 2");
+        if (!strcmp(key, "sssp.sorted"))
+            HC_CHECK_ARG(value >= 0 && value <= 2, "sssp.sorted must be 0, 1 or 2");
         if (!strcmp(key, "sssp.push_dedup"))
             HC_CHECK_ARG(value >= 0 && value <= 2, "sssp.push_dedup must be 0, 1 or 2");
         if (!strcmp(key, "bu.first"))
@@ -684,7 +688,7 @@ int set_knob(Tuning &t, const char *key, int64_t value) {
                              !strcmp(key, "pull.col_shift") ||
                              !strcmp(key, "bu.first") || !strcmp(key, "sssp.alpha") ||
                              !strcmp(key, "sssp.dist16") || !strcmp(key, "sssp.push_dedup") ||
-                             !strcmp(key, "bu.stage_min");
+                             !strcmp(key, "sssp.sorted") || !strcmp(key, "bu.stage_min");
         HC_CHECK_ARG(value >= (zero_ok ? 0 : 1) && value <= (flag ? 1 : 1 << 20),
                      "%s out of range", key);
         if (stage)

@@ -191,7 +191,7 @@ __device__ __forceinline__ void pull_group(const PlanDev &p, int c, int k,
 // FILTER: gather only neighbours in `changed` (see row_min); `gathered`
 // counts the gathers.
 template <bool LOOP, bool FILTER, typename DR, typename OffT>
-__device__ void sssp_pull_sweep(const PlanDev &p, const GraphView<OffT> &g,
+__device__ __forceinline__ void sssp_pull_sweep(const PlanDev &p, const GraphView<OffT> &g,
                                 const DR &rd, const Staged<uint32_t> &changed,
                                 int32_t *__restrict__ dist, uint16_t *d16, uint32_t *next_bm,
                                 uint32_t &cnt, unsigned long long &edges_acc,
@@ -270,7 +270,7 @@ __device__ void sssp_pull_sweep(const PlanDev &p, const GraphView<OffT> &g,
 // next-frontier bitmap, or the epoch API's seen bitmap) counts it once;
 // edges_acc adds its full degree.
 template <typename DR, typename OffT>
-__device__ void sssp_pull_sweep_cb(const PlanDev &p, const GraphView<OffT> &g,
+__device__ __forceinline__ void sssp_pull_sweep_cb(const PlanDev &p, const GraphView<OffT> &g,
                                    const GraphView<OffT> &cb, int K, const DR &rd,
                                    int32_t *__restrict__ dist, uint16_t *d16,
                                    uint32_t *counted, uint32_t &cnt,
@@ -318,36 +318,77 @@ __device__ void sssp_pull_sweep_cb(const PlanDev &p, const GraphView<OffT> &g,
 // Push expansion of the frontier
 // ---------------------------------------------------------------------------
 
-// Relaxes the out-edges [b, e) of u (G lanes); a lowered neighbour joins
-// the next frontier, or, when its new value is at or above `thresh`
-// (buckets), the far bitmap (`nfar` counts those settings).
-template <int G, typename OffT>
-__device__ __forceinline__ void push_range(const GraphView<OffT> &g,
+constexpr int kPushTrip = 4;  // edges a lane of a push epoch has in flight
+// Rows up to this degree take kSmallLanes lanes (two trips at most); with one
+// edge in flight per lane they would want a wavefront from 17 edges on.
+constexpr int32_t kPushMid = 64;
+
+// Edges of a push epoch: the CSR's two arrays, or the weight-sorted pairs.
+template <typename OffT>
+struct CsrEdges {
+    static constexpr bool kSorted = false;
+    const int32_t *adj, *wt;
+    __device__ __forceinline__ int2 get(OffT i) const { return int2{adj[i], wt[i]}; }
+    __device__ __forceinline__ int32_t floor(int32_t) const { return 0; }
+};
+template <typename OffT>
+struct SortedEdges {
+    static constexpr bool kSorted = true;
+    SortedView v;
+    __device__ __forceinline__ int2 get(OffT i) const { return v.e[i]; }
+    __device__ __forceinline__ int32_t floor(int32_t w) const { return v.floor(w); }
+};
+
+// Relaxes the out-edges [b, e) of u (G lanes, kPushTrip edges a lane in
+// flight: a trip is a chain of dependent accesses -- pair, distance, minimum,
+// staging slot -- and its latency bounds the epoch); a lowered neighbour joins
+// the next frontier.  Sorted edges: only those that land below `thresh` are
+// relaxed (buckets; HC_INF_DIST: all), and the scan stops at the first key
+// that cannot.  `lowest` is the smallest value written.
+template <int G, typename ER, typename OffT>
+__device__ __forceinline__ void push_range(const GraphView<OffT> &g, const ER &er,
                                            int32_t *__restrict__ dist,
                                            const FrontierBufs &fb, StepCtl *ctl,
                                            const PushOut &out,
                                            int nxt, uint32_t *wbm, int32_t u, OffT b,
                                            OffT e, int lane, uint32_t &cnt,
                                            unsigned long long &edges_acc, int32_t thresh,
-                                           uint32_t &nfar) {
+                                           int32_t &lowest) {
     const int32_t du = dist[u];
-    for (OffT i = b + OffT(lane); i < e; i += OffT(G)) {
-        int32_t v = g.adj[i];
-        int32_t nd = relax(du, g.wt[i]);
-        bool lowered = false;
-        if (nd < dist[v]) lowered = nd < atomicMin(&dist[v], nd);
-        if (lowered && nd >= thresh) {
-            atomicOr(&fb.far[v >> 5], 1u << (v & 31));
-            nfar++;
-            lowered = false;
+    for (OffT i = b + OffT(lane); i < e; i += OffT(kPushTrip * G)) {
+        int2 x[kPushTrip];
+        bool in[kPushTrip];
+#pragma unroll
+        for (int r = 0; r < kPushTrip; r++) {
+            const OffT k = i + OffT(r * G);
+            in[r] = k < e;
+            x[r] = in[r] ? er.get(k) : int2{0, 0};
         }
-        if (!out.dedup && lowered) {
-            // The first edge to set v's bit appends v, now.
-            const uint32_t bit = 1u << (v & 31);
-            lowered = !(atomicOr(&wbm[v >> 5], bit) & bit);
-            if (lowered) {
-                cnt++;
-                edges_acc += (unsigned long long)(g.rend(v) - g.rbeg(v));
+        if (ER::kSorted && relax(du, er.floor(x[0].y)) >= thresh) break;
+        int32_t nd[kPushTrip], d[kPushTrip], old[kPushTrip];
+#pragma unroll
+        for (int r = 0; r < kPushTrip; r++) {
+            nd[r] = in[r] ? relax(du, x[r].y) : HC_INF_DIST;
+            d[r] = nd[r] < thresh ? dist[x[r].x] : 0;
+        }
+#pragma unroll
+        for (int r = 0; r < kPushTrip; r++)
+            old[r] = nd[r] < d[r] ? atomicMin(&dist[x[r].x], nd[r]) : 0;
+        int32_t v[kPushTrip];
+        bool lowered[kPushTrip];
+#pragma unroll
+        for (int r = 0; r < kPushTrip; r++) {
+            v[r] = x[r].x;
+            lowered[r] = nd[r] < old[r];
+            if (lowered[r]) lowest = min(lowest, nd[r]);
+            if (!out.dedup && lowered[r]) {
+                // The first edge to set v's bit appends v, now.
+                const uint32_t bit = 1u << (v[r] & 31);
+                lowered[r] = !(atomicOr(&wbm[v[r] >> 5], bit) & bit);
+                if (lowered[r]) {
+                    cnt++;
+                    edges_acc += (unsigned long long)(g.rend(v[r]) - g.rbeg(v[r]));
+                }
             }
         }
         // Deferred: a lowered neighbour is a candidate; the staging keeps
@@ -356,14 +397,14 @@ __device__ __forceinline__ void push_range(const GraphView<OffT> &g,
     }
 }
 
-template <typename OffT>
-__device__ void sssp_push_sweep(const GraphView<OffT> &g,
+template <typename ER, typename OffT>
+__device__ __forceinline__ void sssp_push_sweep(const GraphView<OffT> &g, const ER &er,
                                 int32_t *__restrict__ dist,
                                 const FrontierBufs &fb, StepCtl *ctl,
                                 const PushOut &out, int cur,
                                 int nxt, uint32_t *wbm, uint32_t &cnt,
-                                unsigned long long &edges_acc, uint32_t &nfar) {
-    const int32_t thresh = ctl->thresh;
+                                unsigned long long &edges_acc, int32_t &lowest) {
+    const int32_t thresh = ER::kSorted ? ctl->thresh : HC_INF_DIST;
     const uint32_t nch = fb.cnt[cur][3], n0 = fb.cnt[cur][0],
                    n1 = fb.cnt[cur][1], n2 = fb.cnt[cur][2];
     const uint32_t u1 = nch + n0;
@@ -373,65 +414,397 @@ __device__ void sssp_push_sweep(const GraphView<OffT> &g,
     // for room only when the next unit could overfill the buffer.
     uint32_t staged = 0;
     for (uint32_t unit = blockIdx.x; unit < total; unit += gridDim.x) {
-        const uint32_t umax = push_unit_max(unit, nch, ctl->chunk);
+        const uint32_t umax = push_unit_max(unit, nch, u2, ctl);
         if (staged + umax > out.cap)
             staged = push_out_make_room(out, g, fb, ctl, nxt, umax, cnt, edges_acc);
         staged += umax;
         if (unit < nch) {
             HubChunk h = fb.ch[cur][unit];
-            push_range<kBlock>(g, dist, fb, ctl, out, nxt, wbm, h.u, OffT(h.b), OffT(h.e),
-                               threadIdx.x, cnt, edges_acc, thresh, nfar);
+            push_range<kBlock>(g, er, dist, fb, ctl, out, nxt, wbm, h.u, OffT(h.b), OffT(h.e),
+                               threadIdx.x, cnt, edges_acc, thresh, lowest);
         } else if (unit < u1) {
             int32_t u = fb.q[cur][0][unit - nch];
-            push_range<kBlock>(g, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u), g.rend(u),
-                               threadIdx.x, cnt, edges_acc, thresh, nfar);
+            push_range<kBlock>(g, er, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u), g.rend(u),
+                               threadIdx.x, cnt, edges_acc, thresh, lowest);
         } else if (unit < u2) {
             uint32_t idx = (unit - u1) * kWavesPerBlock + threadIdx.x / kWave;
             if (idx < n1) {
                 int32_t u = fb.q[cur][1][idx];
-                push_range<kWave>(g, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u), g.rend(u),
-                                  lane_id(), cnt, edges_acc, thresh, nfar);
+                push_range<kWave>(g, er, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u), g.rend(u),
+                                  lane_id(), cnt, edges_acc, thresh, lowest);
             }
         } else {
             uint32_t idx = (unit - u2) * kSmallPerUnit + threadIdx.x / kSmallLanes;
             if (idx < n2) {
                 int32_t u = fb.q[cur][2][idx];
-                push_range<kSmallLanes>(g, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u),
+                push_range<kSmallLanes>(g, er, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u),
                                         g.rend(u), threadIdx.x % kSmallLanes, cnt,
-                                        edges_acc, thresh, nfar);
+                                        edges_acc, thresh, lowest);
             }
         }
     }
 }
 
-// Promotion epoch of the buckets: every far vertex whose distance is now
-// below `thresh` leaves the far bitmap and is set in the changed bitmap
-// `wbm` (compacted into the next frontier's queues by the launch after);
-// `cnt` / `edges_acc` count those, `left` the vertices still far.  A thread
-// owns one word of both bitmaps.
+// ---------------------------------------------------------------------------
+// Sweeps over the weight-sorted adjacency
+// ---------------------------------------------------------------------------
+
+// Distances that bound a sorted sweep (fields of the control block).
+struct RowBounds {
+    int32_t low, base, thresh;
+};
+
+// A settling sweep is taken when the bucket's degree sum times this exceeds
+// the edges not yet done.
+constexpr long long kSettleShare = 2;
+// Within a bucket, a frontier of more than m / kBucketSweep edges is relaxed
+// by a sweep over the rows instead of a push.
+constexpr long long kBucketSweep = 8;
+
+// What a sorted sweep does with a row.
+enum RowJob {
+    kRowPull,    // lower the row; a lowered row is changed
+    kRowBucket,  // buckets: lower the row to a value below thresh; a lowered row is changed
+    kRowSettle,  // buckets: lower a row at or above base; below thresh it joins the frontier
+    kRowScatter  // buckets: push the edges of a row in [low, thresh) that leave the bucket
+};
+
+// Per-thread results of a sweep.
+struct RowSums {
+    uint32_t cnt = 0;                  // rows put into the next frontier
+    unsigned long long edges = 0;      // and their degree sum
+    uint32_t gathered = 0;             // edges relaxed
+    uint32_t left = 0;                 // kRowSettle: rows reached and left at or above thresh
+    int32_t lowest = HC_INF_DIST;      // smallest value written (kRowSettle: left at or above thresh)
+};
+
+// One trip of sorted_row_min: R edges a lane from edge i.  False when the
+// scan is over.
+template <int G, int R, typename OffT>
+__device__ __forceinline__ bool sorted_trip(const SortedView &sv, const int32_t *dist, OffT i,
+                                            OffT e, int lane, int32_t low, int32_t &best,
+                                            int32_t &m, uint32_t &gathered) {
+    int2 x[R];
+    bool in[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const OffT k = i + OffT(r * G + lane);
+        in[r] = k < e;
+        x[r] = in[r] ? sv.e[k] : int2{0, 0};
+    }
+    int32_t d[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const bool use = in[r] && low + x[r].y < best;
+        d[r] = use ? dist[x[r].x] : HC_INF_DIST;
+        gathered += use ? 1u : 0u;
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) m = min(m, relax(d[r], x[r].y));
+    if (G > 1) m = group_min<G>(m);
+    best = min(best, m);
+    // The last lane's last edge has the trip's heaviest key.
+    bool more = in[R - 1] && low + sv.floor(x[R - 1].y) < best;
+    if (G > 1) more = __shfl(more ? 1 : 0, G - 1, G) != 0;
+    return more;
+}
+
+// Smallest candidate over the sorted edges [b, e) of a row of distance cur,
+// by a group of G lanes; every lane returns the group's minimum.  `low` is a
+// lower bound of the distances that can still lower the row, so an edge is
+// gathered only where low + w is below the best value so far, and the scan
+// ends with the first trip that reaches a key where it is not.  Most rows end
+// after a trip of two edges a lane; those that go on (unreached rows, above
+// all) take longer trips, since the latency of a trip is what they wait for.
+template <int G, typename OffT>
+__device__ __forceinline__ int32_t sorted_row_min(const SortedView &sv, const int32_t *dist,
+                                                  OffT b, OffT e, int lane, int32_t cur,
+                                                  int32_t low, uint32_t &gathered) {
+    int32_t best = cur, m = HC_INF_DIST;
+    if (!sorted_trip<G, 2>(sv, dist, b, e, lane, low, best, m, gathered)) return m;
+    // (8-byte offsets take the registers of the longer trip)
+    constexpr int R = sizeof(OffT) == 8 ? 2 : 4;
+    for (OffT i = b + OffT(2 * G); i < e; i += OffT(R * G))
+        if (!sorted_trip<G, R>(sv, dist, i, e, lane, low, best, m, gathered)) break;
+    return m;
+}
+
+// Pushes the sorted edges [b, e) of a row of distance du that reach thresh or
+// more (the lighter ones were relaxed by the bucket's push epochs).
+template <int G, typename OffT>
+__device__ __forceinline__ void scatter_row(const SortedView &sv, int32_t *dist, OffT b, OffT e,
+                                            int lane, int32_t du, int32_t thresh,
+                                            uint32_t &gathered) {
+    for (OffT i = b + OffT(lane); i < e; i += OffT(G)) {
+        const int2 x = sv.e[i];
+        const int32_t nd = relax(du, x.y);
+        if (nd < thresh || nd >= HC_INF_DIST) continue;
+        gathered++;
+        if (nd < dist[x.x]) atomicMin(&dist[x.x], nd);
+    }
+}
+
+// The bound of a row's scan, and whether the row is swept at all.
+template <int JOB>
+__device__ __forceinline__ bool row_wanted(const RowBounds &c, int32_t cur) {
+    if (JOB == kRowPull || JOB == kRowBucket) return cur > c.low;
+    if (JOB == kRowSettle) return cur >= c.base;
+    return cur >= c.low && cur < c.thresh;
+}
+
+// A row of a wavefront's block, one per lane.
 template <typename OffT>
-__device__ void sssp_promote_sweep(const GraphView<OffT> &g, const int32_t *dist,
-                                   const FrontierBufs &fb, int32_t thresh, uint32_t *wbm,
-                                   uint32_t &cnt, unsigned long long &edges_acc, uint32_t &left) {
-    for (int w = blockIdx.x * kBlock + threadIdx.x; w < fb.words; w += gridDim.x * kBlock) {
-        const uint32_t word = fb.far[w];
-        if (!word) continue;
-        uint32_t now = 0;
-        for (uint32_t x = word; x; x &= x - 1) {
-            const int b = __ffs(x) - 1;
-            const int32_t v = w * 32 + b;
-            if (dist[v] < thresh) {
-                now |= 1u << b;
-                cnt++;
-                edges_acc += (unsigned long long)(g.rend(v) - g.rbeg(v));
+struct RowHead {
+    int32_t u, cur;
+    OffT b, e;
+    bool ok;
+};
+
+// Outcome of a row: its new value is min(cur, m); `hit` puts it into the next
+// frontier.
+template <int JOB>
+__device__ __forceinline__ bool row_done(const RowBounds &ct, int32_t cur, int32_t top, int32_t m,
+                                         unsigned long long deg, RowSums &s) {
+    bool hit = m < top;
+    if (JOB != kRowSettle) {
+        if (hit) s.lowest = min(s.lowest, m);
+    } else {
+        const int32_t d = min(cur, m);
+        hit = d < ct.thresh;
+        if (!hit && d < HC_INF_DIST) {
+            s.left++;
+            s.lowest = min(s.lowest, d);
+        }
+    }
+    if (hit) {
+        s.cnt++;
+        s.edges += deg;
+    }
+    return hit;
+}
+
+// The same for a chunk of a shared row (one lane).
+template <int JOB, typename OffT>
+__device__ __forceinline__ void shared_done(const RowBounds &ct, const GraphView<OffT> &g,
+                                            int32_t *dist, uint32_t *wbm, int32_t u, int32_t cur,
+                                            int32_t top, int32_t m, RowSums &s) {
+    int32_t d = cur;
+    bool hit = false;
+    if (m < top) {
+        const int32_t old = atomicMin(&dist[u], m);
+        hit = m < old;
+        d = min(old, m);
+    }
+    if (JOB != kRowSettle) {
+        if (hit) s.lowest = min(s.lowest, m);
+    } else {
+        hit = d < ct.thresh;
+        if (!hit && d < HC_INF_DIST) {
+            s.left++;
+            s.lowest = min(s.lowest, d);
+        }
+    }
+    if (hit) {
+        const uint32_t bit = 1u << (u & 31);
+        if (!(atomicOr(&wbm[u >> 5], bit) & bit)) {
+            s.cnt++;
+            s.edges += (unsigned long long)(g.rend(u) - g.rbeg(u));
+        }
+    }
+}
+
+template <int JOB>
+__device__ __forceinline__ int32_t row_top(const RowBounds &ct, int32_t cur) {
+    return JOB == kRowBucket ? min(cur, ct.thresh) : cur;
+}
+
+// The wanted rows of a wavefront's block (one row head per lane), those of
+// lanes j0, j0 + jstep, ... (several wavefronts may share a block; a row's
+// wavefront must not depend on distances, which they read at different
+// times), G lanes per row.  A row's distance and bounds are read by one lane,
+// coalesced over the block, so a block without wanted rows costs its heads
+// only; the wanted ones are packed together.
+// SHARED: heads are chunks of hub rows, which several wavefronts lower: with
+// atomicMin, the row's bit counted by the chunk that sets it, and a chunk of a
+// settling sweep that finds the row below thresh sets the bit whoever lowered
+// it; `left` then counts a hub by each chunk's view, which matters only when
+// no row at all is below thresh.
+template <int JOB, int G, bool SHARED, typename OffT>
+__device__ __forceinline__ void sorted_block(const RowHead<OffT> &h, int j0, int jstep,
+                                             const RowBounds &ct, const GraphView<OffT> &g,
+                                             const SortedView &sv, int32_t *dist, uint32_t *wbm,
+                                             RowSums &s) {
+    const int lane = lane_id();
+    const bool want = h.ok && lane % jstep == j0 && row_wanted<JOB>(ct, h.cur);
+    bool hit = false;  // of this lane's row
+    if (G == 1) {
+        if (want) {
+            if (JOB == kRowScatter) {
+                scatter_row<1>(sv, dist, h.b, h.e, 0, h.cur, ct.thresh, s.gathered);
             } else {
-                left++;
+                const int32_t top = row_top<JOB>(ct, h.cur);
+                const int32_t m =
+                    sorted_row_min<1>(sv, dist, h.b, h.e, 0, top, ct.low, s.gathered);
+                if (m < top) dist[h.u] = m;
+                hit = row_done<JOB>(ct, h.cur, top, m, (unsigned long long)(h.e - h.b), s);
             }
         }
-        if (now) {
-            fb.far[w] = word & ~now;
-            wbm[w] = now;  // cleared by the launch before; no other writer
+    } else {
+        constexpr int PER = kWave / G;
+        const uint64_t mask = __ballot(want);
+        const int n = __popcll(mask);
+        // Lane r learns the lane of the r-th wanted row (the others fill the
+        // places after them).
+        const int rank = __popcll(mask & lanemask_lt());
+        const int src =
+            __builtin_amdgcn_ds_permute((want ? rank : n + lane - rank) << 2, lane);
+        for (int j = 0; j * PER < n; j++) {
+            const int gi = j * PER + lane / G;
+            const bool have = gi < n;
+            const int sl = __shfl(src, gi & (kWave - 1));
+            const int32_t cur = __shfl(h.cur, sl);
+            const int32_t u = __shfl(h.u, sl);
+            const OffT b = __shfl(h.b, sl), e = __shfl(h.e, sl);
+            bool ghit = false;
+            if (have) {
+                if (JOB == kRowScatter) {
+                    scatter_row<G>(sv, dist, b, e, lane % G, cur, ct.thresh, s.gathered);
+                } else {
+                    const int32_t top = row_top<JOB>(ct, cur);
+                    const int32_t m = sorted_row_min<G>(sv, dist, b, e, lane % G, top, ct.low,
+                                                        s.gathered);
+                    if (SHARED) {
+                        if (lane == 0) shared_done<JOB>(ct, g, dist, wbm, u, cur, top, m, s);
+                    } else if (lane % G == 0) {
+                        if (m < top) dist[u] = m;
+                        ghit = row_done<JOB>(ct, cur, top, m, (unsigned long long)(e - b), s);
+                    }
+                }
+            }
+            if (JOB != kRowScatter && !SHARED) {
+                // The groups' outcomes back to their rows' lanes.
+                for (uint64_t gm = __ballot(ghit); gm; gm &= gm - 1) {
+                    const int l = __ffsll((unsigned long long)gm) - 1;
+                    hit = hit || lane == __builtin_amdgcn_readlane(sl, l);
+                }
+            }
         }
+    }
+    if (JOB != kRowScatter && !SHARED) wave_or_bits(wbm, h.u, hit);
+}
+
+// Wavefronts that share a block of 64 heads: 16 for hub chunks
+// and heavy rows (64 lanes a row), and while the plan has fewer blocks than
+// the grid wavefronts, four for the lighter ones.
+constexpr int kHeavySplit = 16;
+
+// One sweep over the plan (grid-stride, wavefront units), the next unit's
+// heads read ahead of this unit's rows.
+template <int JOB, typename OffT>
+__device__ __forceinline__ void sorted_sweep(const PlanDev &p, const RowBounds &ct,
+                                             const GraphView<OffT> &g, const SortedView &sv,
+                                             int32_t *dist, uint32_t *wbm, RowSums &s) {
+    const int b0 = (p.cnt[0] + 63) / 64, b2 = (p.cnt[2] + 63) / 64;
+    const int b3 = (p.cnt[3] + 63) / 64, b4 = (p.cnt[4] + 63) / 64, b5 = (p.cnt[5] + 63) / 64;
+    const int stride = gridDim.x * kWavesPerBlock;
+    const int split = b3 + b4 < stride ? 4 : 1;
+    const int t0 = b0 * kHeavySplit, t2 = t0 + b2 * kHeavySplit;
+    const int t3 = t2 + b3 * 4 * split, t4 = t3 + b4 * split, total = t4 + b5;
+    const int lane = lane_id();
+    // The lane's row of a unit (class indexes are constants: an indexed plan
+    // would be copied to scratch).
+    auto head = [&](int unit) {
+        RowHead<OffT> h{0, 0, OffT(0), OffT(0), false};
+        int i = 0, beg = 0;
+        const int32_t *list = nullptr;
+        if (unit < t0) {
+            i = unit / kHeavySplit * 64 + lane;
+            if (i < p.cnt[0]) {
+                const HubChunk c = p.chunks[i];
+                h.u = c.u;
+                h.b = OffT(c.b);
+                h.e = OffT(c.e);
+                h.cur = dist[c.u];
+                // The chunk's first key rules out the rest of it.
+                h.ok = JOB == kRowScatter ||
+                       ct.low + sv.floor(sv.e[c.b].y) < row_top<JOB>(ct, h.cur) ||
+                       (JOB == kRowSettle && h.cur >= ct.base);
+            }
+            return h;
+        } else if (unit < t2) {
+            i = (unit - t0) / kHeavySplit * 64 + lane;
+            h.ok = i < p.cnt[2];
+            beg = p.beg[2];
+            list = p.list[2];
+        } else if (unit < t3) {
+            i = (unit - t2) / (4 * split) * 64 + lane;
+            h.ok = i < p.cnt[3];
+            beg = p.beg[3];
+            list = p.list[3];
+        } else if (unit < t4) {
+            i = (unit - t3) / split * 64 + lane;
+            h.ok = i < p.cnt[4];
+            beg = p.beg[4];
+            list = p.list[4];
+        } else if (unit < total) {
+            i = (unit - t4) * 64 + lane;
+            h.ok = i < p.cnt[5];
+            beg = p.beg[5];
+            list = p.list[5];
+        }
+        if (h.ok) {
+            h.u = list ? list[i] : beg + i;
+            h.cur = dist[h.u];
+            h.b = g.rbeg(h.u);
+            h.e = g.rend(h.u);
+        }
+        return h;
+    };
+    int unit = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
+    RowHead<OffT> h = head(unit);
+    while (unit < total) {
+        const RowHead<OffT> nx = head(unit + stride);
+        if (unit < t0)
+            sorted_block<JOB, 64, true>(h, unit % kHeavySplit, kHeavySplit, ct, g, sv, dist, wbm,
+                                        s);
+        else if (unit < t2)
+            sorted_block<JOB, 64, false>(h, (unit - t0) % kHeavySplit, kHeavySplit, ct, g, sv,
+                                         dist, wbm, s);
+        else if (unit < t3)
+            sorted_block<JOB, 16, false>(h, (unit - t2) % (4 * split), 4 * split, ct, g, sv, dist,
+                                         wbm, s);
+        else if (unit < t4)
+            sorted_block<JOB, 4, false>(h, (unit - t3) % split, split, ct, g, sv, dist, wbm, s);
+        else
+            sorted_block<JOB, 1, false>(h, 0, 1, ct, g, sv, dist, wbm, s);
+        unit += stride;
+        h = nx;
+    }
+}
+
+// Promotion without a settling sweep: the vertices in [base, thresh) become
+// the frontier.  A wavefront owns two words of the bitmap.
+template <typename OffT>
+__device__ __forceinline__ void promote_scan(const RowBounds &ct, const GraphView<OffT> &g, const int32_t *dist,
+                             uint32_t *wbm, RowSums &s) {
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    for (int64_t i0 = (int64_t)blockIdx.x * kBlock; i0 < g.n; i0 += stride) {
+        const int64_t i = i0 + threadIdx.x;
+        const bool in = i < g.n;
+        const int32_t u = (int32_t)(in ? i : 0);
+        const int32_t d = in ? dist[u] : HC_INF_DIST;
+        const bool hit = in && d >= ct.base && d < ct.thresh;
+        const uint64_t m = __ballot(hit);
+        if (hit) {
+            s.cnt++;
+            s.edges += (unsigned long long)(g.rend(u) - g.rbeg(u));
+        } else if (d >= ct.thresh && d < HC_INF_DIST) {
+            s.left++;
+            s.lowest = min(s.lowest, d);
+        }
+        // (the epoch before cleared the bitmap)
+        if (lane_id() == 0 && uint32_t(m)) wbm[u >> 5] = uint32_t(m);
+        if (lane_id() == 32 && uint32_t(m >> 32)) wbm[u >> 5] = uint32_t(m >> 32);
     }
 }
 
@@ -499,17 +872,15 @@ __global__ __launch_bounds__(kBlock) void sssp_step_kernel(
                 sssp_pull_sweep<true, false>(p, g, rd, unstaged(rbm), dist, nullptr, wbm, cnt,
                                              eacc, gathered);
         }
-    } else if (mode == kPromote) {
-        // (`gathered` carries the vertices left far)
-        sssp_promote_sweep(g, dist, fb, ctl->thresh, wbm, cnt, eacc, gathered);
     } else {
         // Output staged in the dynamic LDS (unused by push epochs).
         __shared__ uint32_t s_out;
         if (threadIdx.x == 0) s_out = 0;
         __syncthreads();
         const PushOut out{s_stage, &s_out, (uint32_t)push_cap, defer_dedup ? wbm : nullptr};
-        // (`gathered` carries the far settings)
-        sssp_push_sweep(g, dist, fb, ctl, out, cur, nxt, wbm, cnt, eacc, gathered);
+        int32_t lowest = HC_INF_DIST;
+        sssp_push_sweep(g, CsrEdges<OffT>{g.adj, g.wt}, dist, fb, ctl, out, cur, nxt, wbm, cnt,
+                        eacc, lowest);
         const PushKept k = push_out_flush(out, g, fb, ctl, nxt);
         cnt += k.n;
         eacc += k.e;
@@ -517,26 +888,104 @@ __global__ __launch_bounds__(kBlock) void sssp_step_kernel(
     write_partials(fb.part, cnt, eacc, gathered);
 }
 
+// The step on the weight-sorted adjacency (the default): pull epochs or, with
+// buckets, settling sweeps look only at the edges that can lower a row (see
+// sorted.hip), push epochs only at those that land in the bucket.
+// Kronecker 23: a pull epoch gathers 4-35 M distances instead of 259 M and
+// takes 160-340 us instead of 1600, a source 1.36 ms instead of 5.15; what is
+// left is the lines of the row heads and starts and, in the push that meets
+// most of the graph, the atomics (27 G/s at any size and locality on this
+// GPU, where random loads reach 65 G/s from 33 MB and 262 G/s from L2).
+// Uniform 23: 4.06 ms a source instead of 10.6.
+template <typename OffT, bool BUCKETS>
+__global__ __launch_bounds__(kBlock) void sssp_sorted_step_kernel(
+    PlanDev p, GraphView<OffT> g, SortedView sv, int32_t *__restrict__ dist, FrontierBufs fb,
+    StepCtl *ctl, int32_t push_cap, int defer_dedup) {
+    extern __shared__ int32_t s_stage[];
+    __shared__ uint32_t s_out, s_left;
+    __shared__ int32_t s_lowest;
+    if (ctl->done) return;
+    const int mode = ctl->mode;
+    const int k = ctl->epoch;
+    const int cur = k & 1, nxt = cur ^ 1;
+    uint32_t *wbm = fb.bm[(k + 1) % 3];
+    uint32_t *cbm = fb.bm[(k + 2) % 3];
+    for (int w = blockIdx.x * kBlock + threadIdx.x; w < fb.words; w += gridDim.x * kBlock)
+        cbm[w] = 0;
+    if (threadIdx.x == 0) {
+        s_out = 0;
+        s_left = 0;
+        s_lowest = HC_INF_DIST;
+    }
+    __syncthreads();
+    RowSums s;
+    const RowBounds rb{ctl->low, ctl->base, ctl->thresh};
+    if (mode == kPush && !(BUCKETS && ctl->settle)) {
+        const PushOut out{s_stage, &s_out, (uint32_t)push_cap, defer_dedup ? wbm : nullptr};
+        sssp_push_sweep(g, SortedEdges<OffT>{sv}, dist, fb, ctl, out, cur, nxt, wbm, s.cnt,
+                        s.edges, s.lowest);
+        const PushKept kept = push_out_flush(out, g, fb, ctl, nxt);
+        s.cnt += kept.n;
+        s.edges += kept.e;
+    } else if (!BUCKETS) {
+        sorted_sweep<kRowPull>(p, rb, g, sv, dist, wbm, s);
+    } else if (mode == kPush) {
+        sorted_sweep<kRowScatter>(p, rb, g, sv, dist, wbm, s);
+    } else if (ctl->settle == 3) {
+        sorted_sweep<kRowBucket>(p, rb, g, sv, dist, wbm, s);
+    } else if (ctl->settle) {
+        sorted_sweep<kRowSettle>(p, rb, g, sv, dist, wbm, s);
+    } else {
+        promote_scan(rb, g, dist, wbm, s);
+    }
+    if (s.left) atomicAdd(&s_left, s.left);
+    if (s.lowest < HC_INF_DIST) atomicMin(&s_lowest, s.lowest);
+    __syncthreads();
+    write_partials(fb.part, s.cnt, s.edges, s.gathered, s_left, 0,
+                   (unsigned long long)(HC_INF_DIST - s_lowest));
+}
+
+// Next bucket: the vertices in [base, base + delta) at least.
+__device__ __forceinline__ void next_bucket(StepCtl *c, int32_t base) {
+    c->base = base;
+    c->thresh = (int32_t)min((long long)base + c->delta, (long long)HC_INF_DIST);
+    c->bucket_e = 0;
+}
+
 // Epoch controller (one thread, on the header copy c), from the step sums
 // of the epoch that ran.
 __device__ void sssp_decide(StepCtl *c, StepCtl *trace,
                             const unsigned long long (&sums)[kSumSlots]) {
     const unsigned long long out_n = sums[0], out_e = sums[1], gathered = sums[2];
+    const unsigned long long left = sums[3];
+    const int32_t lowest = HC_INF_DIST - (int32_t)sums[kMaxSlot];
     const int k = c->epoch;
     const int ran = c->mode;
+    const int settled = c->settle;
     if (ran == kPromote) {
-        // far bitmap words, plus dist[v] and a bitmap entry per far vertex
-        c->alg_bytes += 4ull * (unsigned long long)((c->n + 31) / 32) + 8ull * (out_n + gathered);
+        // dist per vertex; pair + gathered distance per relaxed edge and
+        // offsets per row of a settling sweep; a bit per frontier vertex
+        c->alg_bytes += (settled ? 8ull : 4ull) * (unsigned long long)c->n + 12ull * gathered +
+                        8ull * out_n;
         c->promotions++;
-        c->far_live = (long long)gathered;
-        trace_epoch(c, trace, k, ran, out_n, out_e, 0);
+        trace_epoch(c, trace, k, ran, out_n, out_e, gathered);
     } else if (ran == kPush) {
         // offsets + dist[u] per frontier vertex; id + weight + dist[v] per
         // edge; dist write + bitmap/queue entry per improved vertex.
-        c->alg_bytes += 12ull * c->in_n + 12ull * c->in_e + 8ull * out_n;
+        if (settled) {
+            c->alg_bytes += 8ull * (unsigned long long)c->n + 12ull * gathered;
+            trace_epoch(c, trace, k, ran, out_n, out_e, gathered);
+        } else {
+            c->alg_bytes += 12ull * c->in_n + 12ull * c->in_e + 8ull * out_n;
+            trace_epoch(c, trace, k, ran, out_n, out_e, c->in_e);
+        }
         c->push_epochs++;
-        c->far_live += (long long)gathered;  // far settings (may repeat a vertex)
-        trace_epoch(c, trace, k, ran, out_n, out_e, c->in_e);
+    } else if (c->sorted) {
+        // Offsets and own distances; id + weight + distance per edge relaxed.
+        c->alg_bytes += (unsigned long long)c->sweep_bytes - 12ull * (unsigned long long)c->m +
+                        12ull * gathered + 8ull * out_n;
+        c->pull_epochs++;
+        trace_epoch(c, trace, k, ran, out_n, out_e, gathered);
     } else {
         // Offsets, ids and own distances always; weight + distance per
         // gathered edge; one bit per tested neighbour when filtering.
@@ -546,6 +995,7 @@ __device__ void sssp_decide(StepCtl *c, StepCtl *trace,
         c->pull_epochs++;
         trace_epoch(c, trace, k, ran, out_n, out_e, (unsigned long long)c->m);
     }
+    if ((ran == kPush && !settled) || settled == 3) c->bucket_e += c->in_e;
     c->epoch = k + 1;
     c->in_n = (long long)out_n;
     c->in_e = (long long)out_e;
@@ -557,23 +1007,49 @@ __device__ void sssp_decide(StepCtl *c, StepCtl *trace,
     int next = ran;
     if (c->max_epochs > 0 && k + 1 >= c->max_epochs) {
         c->done = 1;
-    } else if (out_n == 0) {
-        if (c->delta > 0 && c->far_live > 0) {
-            // Raise the threshold and promote; after a promotion that found
-            // nothing below it, rise twice as far.
-            const long long step = ran == kPromote ? 2ll * c->far_step : (long long)c->delta;
-            c->far_step = (int32_t)min(step, (long long)HC_INF_DIST);
-            c->thresh = (int32_t)min((long long)c->thresh + step, (long long)HC_INF_DIST);
+    } else if (c->delta > 0) {
+        c->settle = 0;
+        if (out_n != 0) {
+            // The bucket goes on: by a sweep of the rows above its lowest
+            // pending value while the frontier is heavy, else by a push.
+            c->low = ran == kPromote && settled != 3 ? c->base : lowest;
+            next = kPush;
+            if (c->direction != 2 && (long long)out_e > c->m / kBucketSweep) {
+                c->settle = 3;
+                next = kPromote;
+            }
+        } else if ((ran == kPush && !settled) || settled == 3) {
+            // The bucket is complete.  A sweep over the rows above it costs
+            // a few edges of each, a push from its vertices most of theirs:
+            // the sweep, once the bucket holds a fair share of the edges not
+            // yet done (and always the push while most rows are unreached,
+            // whose scans find no bound).
+            const long long rest = c->m - c->done_e - c->bucket_e;
+            c->done_e += c->bucket_e;
+            c->low = c->base;
+            if (c->direction != 2 && c->bucket_e * kSettleShare > rest) {
+                c->settle = 1;
+                next = kPromote;
+                next_bucket(c, c->thresh);
+            } else {
+                c->settle = 2;
+                next = kPush;
+            }
+        } else if (ran == kPush) {
             next = kPromote;
+            next_bucket(c, c->thresh);
+        } else if (left != 0) {
+            // An empty bucket: on to the smallest distance above it.
+            next = kPromote;
+            next_bucket(c, lowest);
         } else {
             c->done = 1;
         }
-    } else if (c->delta > 0 || c->direction == 2) {
-        next = kPush;
-    } else if (c->direction == 1) {
-        next = kPull;
     } else {
-        next = (long long)out_e > c->m / c->alpha ? kPull : kPush;
+        c->low = lowest;
+        if (out_n == 0) c->done = 1;
+        else if (c->direction != 0) next = c->direction == 1 ? kPull : kPush;
+        else next = (long long)out_e > c->m / c->alpha ? kPull : kPush;
     }
     c->need_compact = (!c->done && ran != kPush && next == kPush) ? 1 : 0;
     c->mode = next;
@@ -597,6 +1073,16 @@ __global__ __launch_bounds__(kBlock) void sssp_between_kernel(GraphView<OffT> g,
     compact_body(g, fb, &s_c, 1, dist, d16);
 }
 
+// Smallest initial distance seen by each workgroup, for sssp_init_kernel.
+__global__ __launch_bounds__(kBlock) void sssp_init_low_kernel(const int32_t *__restrict__ init,
+                                                               int32_t n, Partials part) {
+    int32_t m = HC_INF_DIST;
+    for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
+        m = min(m, init[i]);
+    m = block_min(m);
+    if (threadIdx.x == 0) part.acc[blockIdx.x] = (unsigned long long)(long long)m;
+}
+
 // Initialises distances, bitmaps and the control block for one run.
 // init_dist == nullptr: single source `src`; otherwise copy init_dist and
 // start in pull mode with an empty frontier (sssp_pull_gpu semantics).
@@ -605,7 +1091,8 @@ __global__ __launch_bounds__(kBlock) void sssp_init_kernel(
     GraphView<OffT> g, int32_t *__restrict__ dist,
     const int32_t *__restrict__ init_dist, FrontierBufs fb, StepCtl *ctl,
     int32_t src, int direction, int alpha, int max_epochs, long long m,
-    long long sweep_bytes, int grid, int filter, int chunk, uint16_t *d16, int delta) {
+    long long sweep_bytes, int grid, int filter, int chunk, uint16_t *d16, int delta, int sorted,
+    int low_parts) {
     const int stride = gridDim.x * kBlock;
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < g.n; i += stride) {
         const int32_t d = init_dist ? init_dist[i] : (i == src ? 0 : HC_INF_DIST);
@@ -617,11 +1104,24 @@ __global__ __launch_bounds__(kBlock) void sssp_init_kernel(
         fb.bm[0][w] = (!init_dist && w == (src >> 5)) ? (1u << (src & 31)) : 0u;
         fb.bm[1][w] = 0;
         fb.bm[2][w] = 0;
-        fb.far[w] = 0;
     }
-    if (blockIdx.x == 0)
+    // Smallest initial distance (sssp_init_low_kernel's results lie in the
+    // counter sets, one per workgroup of that launch).
+    __shared__ int32_t s_low;
+    if (blockIdx.x == 0) {
+        if (threadIdx.x == 0) s_low = HC_INF_DIST;
+        __syncthreads();
+        for (int i = threadIdx.x; i < low_parts; i += kBlock)
+            atomicMin(&s_low, (int32_t)(long long)fb.part.acc[i]);
+        __syncthreads();
         for (int j = 0; j < kSumSets; j++) clear_partials(sum_set(fb.part, j));
+    }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ctl->sorted = sorted;
+        // Every candidate of epoch 0 comes from the source, or from an
+        // initial distance; where one of those is negative (relax() reads
+        // it as unsigned) no edge is left out.
+        ctl->low = !init_dist ? 0 : (s_low < 0 ? -HC_INF_DIST - 1 : s_low);
         // With initial distances the changed set before epoch 0 is unknown:
         // that epoch gathers every neighbour.
         ctl->filter_knob = filter;
@@ -635,16 +1135,19 @@ __global__ __launch_bounds__(kBlock) void sssp_init_kernel(
         ctl->alpha = alpha;
         ctl->need_compact = 0;
         ctl->chunk = chunk;
+        ctl->mid = kPushMid;
         ctl->n = g.n;
         ctl->grid = grid;
         ctl->m = m;
         ctl->sweep_bytes = sweep_bytes;
         ctl->push_epochs = ctl->pull_epochs = 0;
         ctl->delta = delta;
+        ctl->base = 0;
         ctl->thresh = delta > 0 ? delta : HC_INF_DIST;
-        ctl->far_step = delta;
+        ctl->settle = 0;
         ctl->promotions = 0;
-        ctl->far_live = 0;
+        ctl->bucket_e = 0;
+        ctl->done_e = 0;
         ctl->reached = 0;
         ctl->alg_bytes = 0;
         ctl->t_start = wall_clock64();
@@ -656,7 +1159,7 @@ __global__ __launch_bounds__(kBlock) void sssp_init_kernel(
         } else {
             OffT b = g.rbeg(src), e = g.rend(src);
             int64_t d = int64_t(e - b);
-            int cls = degree_class(d);
+            int cls = degree_class(d, kPushMid);
             if (cls == 3) {  // chunk descriptors: written by workgroup 0 below
                 fb.cnt[0][3] = (uint32_t)((d + chunk - 1) / chunk);
                 fb.cnt[0][4] = 1;
@@ -917,11 +1420,19 @@ struct SsspLaunch {
     PlanDev cbplan;          // column-blocked pull sweeps (cbk > 0)
     GraphView<OffT> cbv;
     int cbk;
+    SortedView sv;           // weight-sorted adjacency (e: not nullptr)
+    bool buckets;
     template <bool D16, bool CB>
     void step(FrontierBufs fb, StepCtl *cur) {
         timed_launch(kt, sssp_step_kernel<OffT, D16, CB>, dim3(grid), dim3(kBlock),
                      uint32_t(lds_entries * sizeof(int32_t)), s, plan, g, dist, d16, fb, cur,
                      nstage, push_cap, defer_dedup, cbplan, cbv, cbk);
+    }
+    template <bool BUCKETS>
+    void sorted_step(FrontierBufs fb, StepCtl *cur) {
+        timed_launch(kt, sssp_sorted_step_kernel<OffT, BUCKETS>, dim3(grid), dim3(kBlock),
+                     uint32_t(lds_entries * sizeof(int32_t)), s, plan, g, sv, dist, fb, cur,
+                     push_cap, defer_dedup);
     }
     // Epoch k: header slot k & 1, counter set k % 3.
     static int launch(void *arg, long long k) {
@@ -929,7 +1440,10 @@ struct SsspLaunch {
         FrontierBufs fb = a->fb;
         fb.part = sum_set(a->fb.part, k);
         StepCtl *cur = a->ctl + (k & 1), *nxt = a->ctl + ((k + 1) & 1);
-        if (a->d16) {
+        if (a->sv.e) {
+            if (a->buckets) a->template sorted_step<true>(fb, cur);
+            else a->template sorted_step<false>(fb, cur);
+        } else if (a->d16) {
             if (a->cbk) a->template step<true, true>(fb, cur);
             else a->template step<true, false>(fb, cur);
         } else {
@@ -944,16 +1458,17 @@ struct SsspLaunch {
 };
 
 
-// Bucket width of the single-source loop (knob sssp.delta): 2 x the sampled
+// Bucket width of the single-source loop (knob sssp.delta): 4 x the sampled
 // largest weight / mean degree on flat graphs (uniform 23, weights 1..255,
-// degree 32: 16; 8 and 16 measured best, 20.7 -> 10.5 ms), off on skewed
-// ones (Kronecker 23: 5.1 -> 8.3..9.2 ms with widths 16..256).
+// degree 32: widths 24 / 32 / 48 / 64 / 96 4.41 / 4.06 / 4.41 / 4.56 / 4.70
+// ms), off on skewed ones, whose pull sweeps win (Kronecker 23: 1.36 ms
+// against 2.4 / 1.8 ms with widths 32 / 96).
 static int sssp_delta(hc_graph_s *g) {
     const int d = tuning().sssp_delta;
     if (d >= 0) return d;
     if (!g->weighted || g->m == 0 || g->max_weight <= 0 || !flat_graph(g)) return 0;
     const double mean_deg = (double)g->m / std::max(1, g->rows);
-    return (int)std::max(1.0, std::ceil(2.0 * g->max_weight / mean_deg));
+    return (int)std::max(1.0, std::ceil(4.0 * g->max_weight / mean_deg));
 }
 
 template <typename OffT>
@@ -962,12 +1477,24 @@ static int run_sssp_loop(hc_graph_s *g, int32_t src, const int32_t *init_dist,
                          int max_epochs, hc_run_stats_t *stats, hipStream_t s) {
     SsspWs *ws = nullptr;
     HC_TRY(get_sssp_ws(g, &ws));
-    const PlanHost *ph = nullptr;
-    HC_TRY(get_plan(g, 0, g->n, sssp_plan_config(), &ph));
     GraphView<OffT> v = view<OffT>(g);
-    if (alpha <= 0) alpha = tuning().sssp_alpha > 0 ? tuning().sssp_alpha : (flat_graph(g) ? 2 : 4);
+    // The weight-sorted adjacency (buckets set by a knob need it on any graph),
+    // unless a knob asks for one of the plain sweeps' variants or there is no
+    // memory for the copy.
+    const Tuning &t = tuning();
+    SortedView sv{nullptr, 0};
+    const bool want = t.sssp_sorted == 2 ||
+                      (t.sssp_sorted == 1 && (g->m >= kSortedMinEdges || t.sssp_delta > 0));
+    if (want && t.sssp_filter == 0 && t.sssp_dist16 != 1 && t.pull_col_shift <= 0)
+        HC_TRY(get_sorted(g, s, &sv));
+    const bool sorted = sv.e != nullptr;
+    const PlanHost *ph = nullptr;
+    HC_TRY(get_plan(g, 0, g->n, sorted ? sorted_plan_config() : sssp_plan_config(), &ph));
+    // A pruned pull costs little more than its row heads: pull early
+    // (Kronecker 23: alpha 4 / 8 / 16 / 32 1.72 / 1.39 / 1.36 / 1.35 ms).
+    if (alpha <= 0) alpha = t.sssp_alpha > 0 ? t.sssp_alpha : (sorted ? 16 : flat_graph(g) ? 2 : 4);
     uint16_t *d16 = nullptr;
-    if (tuning().sssp_dist16 == 1 || (tuning().sssp_dist16 == 2 && flat_graph(g))) {
+    if (!sorted && (t.sssp_dist16 == 1 || (t.sssp_dist16 == 2 && flat_graph(g)))) {
         if (!ws->d16 && hipMalloc(&ws->d16, sizeof(uint16_t) * std::max(g->n, 1)) != hipSuccess)
             return fail(HC_ERR_OOM, "16-bit distance mirror allocation failed");
         d16 = ws->d16;
@@ -978,11 +1505,11 @@ static int run_sssp_loop(hc_graph_s *g, int32_t src, const int32_t *init_dist,
     const int32_t lds_entries = std::max<int32_t>(nstage, push_cap);
     // Pull epochs gather column block by column block (not with filtering,
     // which tests a changed bit per neighbour before its gather).
-    // Buckets (sssp.delta): push epochs only.
-    const int delta = init_dist || direction == 1 ? 0 : sssp_delta(g);
+    // Buckets (sssp.delta): on the sorted adjacency.
+    const int delta = init_dist || direction == 1 || !sorted ? 0 : sssp_delta(g);
     const ColBlocks *cb = nullptr;
     const PlanHost *phb = nullptr;
-    if (direction != 2 && delta == 0 && tuning().sssp_filter != 1) {
+    if (!sorted && direction != 2 && tuning().sssp_filter != 1) {
         HC_TRY(get_col_blocks(g, col_shift_for(g, flat_graph(g)), s, &cb));
         if (cb) {
             // Plain sweep for the light rows only.
@@ -991,7 +1518,9 @@ static int run_sssp_loop(hc_graph_s *g, int32_t src, const int32_t *init_dist,
         }
     }
     const void *step_fn =
-        d16 ? (cb ? reinterpret_cast<const void *>(&sssp_step_kernel<OffT, true, true>)
+        sorted ? (delta > 0 ? reinterpret_cast<const void *>(&sssp_sorted_step_kernel<OffT, true>)
+                            : reinterpret_cast<const void *>(&sssp_sorted_step_kernel<OffT, false>))
+        : d16 ? (cb ? reinterpret_cast<const void *>(&sssp_step_kernel<OffT, true, true>)
                   : reinterpret_cast<const void *>(&sssp_step_kernel<OffT, true, false>))
             : (cb ? reinterpret_cast<const void *>(&sssp_step_kernel<OffT, false, true>)
                   : reinterpret_cast<const void *>(&sssp_step_kernel<OffT, false, false>));
@@ -999,10 +1528,13 @@ static int run_sssp_loop(hc_graph_s *g, int32_t src, const int32_t *init_dist,
                                    kBlock, lds_entries * sizeof(int32_t),
                                    std::min(ws->f.grid, grid_blocks(tuning().sssp_grid_per_cu)));
     const int init_grid = std::max(1, std::min(grid, (g->n + kBlock - 1) / kBlock));
+    const int low_parts = init_dist && sorted ? std::min(init_grid, kSumWords * kSumSets) : 0;
+    if (low_parts)
+        sssp_init_low_kernel<<<low_parts, kBlock, 0, s>>>(init_dist, g->n, ws->f.fb.part);
     sssp_init_kernel<OffT><<<init_grid, kBlock, 0, s>>>(
         v, dist, init_dist, ws->f.fb, ws->f.ctl, src, direction, alpha,
         max_epochs, (long long)g->m, sweep, grid, tuning().sssp_filter, tuning().push_chunk, d16,
-        delta);
+        delta, sorted ? 1 : 0, low_parts);
     HC_HIP(hipGetLastError());
     ws->f.kt.reset();
     // Push epochs deduplicate improved vertices when staging them (flat
@@ -1015,7 +1547,7 @@ static int run_sssp_loop(hc_graph_s *g, int32_t src, const int32_t *init_dist,
                        cb ? GraphView<OffT>{static_cast<const OffT *>(cb->off), cb->adj, cb->wt,
                                             0, g->n}
                           : GraphView<OffT>{},
-                       cb ? cb->K : 0};
+                       cb ? cb->K : 0, sv, delta > 0};
     // Bellman-Ford needs at most n epochs (buckets add promotion epochs and
     // re-pushes: a generous bound); the cap bounds a faulty loop.
     const long long bound = delta > 0 ? 64LL * (g->n + 1) + 4096 : (long long)g->n;

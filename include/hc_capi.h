@@ -214,9 +214,20 @@ int hc_graph_get_info(hc_graph_t g, hc_graph_info_t *out);
  * src/kernels/heterogeneous/sssp.cuh:180-278).  Keys:
  *   grid_per_cu            workgroups per CU of full-device launches (8); the
  *                          loops launch at most as many as fit at once
- *   sssp.alpha             SSSP pull when frontier edges > m/alpha; 0: by graph
- *                          shape, 4 when the top 1% rows hold >= 5% of the
- *                          edges (skewed), else 2 (0)
+ *   sssp.alpha             SSSP pull when frontier edges > m/alpha; 0: 16 on
+ *                          the weight-sorted adjacency, on the plain CSR 4
+ *                          when the top 1% rows hold >= 5% of the edges
+ *                          (skewed), else 2 (0)
+ *   sssp.sorted            hc_sssp and hc_sssp_pull (bucketed mapping) relax
+ *                          from a copy of the edges with each row in order of
+ *                          rising weight (8 bytes per edge, built on first use
+ *                          and shared by the graph's shares), whose scans end
+ *                          where no later edge can lower the row: 1 on graphs
+ *                          of at least 2^23 edges (or where sssp.delta sets
+ *                          buckets), 2 on all, 0 on none.  The plain CSR is
+ *                          used all the same when there is no memory for the
+ *                          copy, and when sssp.filter, sssp.dist16 = 1 or
+ *                          pull.col_shift > 0 asks for another sweep (1)
  *   sssp.grid_per_cu       cap on workgroups per CU of the SSSP loop (4)
  *   sssp.filter            1: SSSP pull epochs gather only neighbours whose
  *                          distance changed in the previous epoch; k >= 2:
@@ -278,14 +289,12 @@ int hc_graph_get_info(hc_graph_t g, hc_graph_info_t *out);
  *                          0 off; -1 (default) 12 x the graph's sampled
  *                          largest weight / mean degree on flat graphs, off
  *                          on skewed ones.  Results do not depend on it
- *   sssp.delta             hc_sssp: a vertex lowered to a value at or above
- *                          a threshold waits in a far set instead of the next
- *                          frontier; when a frontier comes out empty the
- *                          threshold rises by this much (doubling after a
- *                          promotion that found nothing) and the far
- *                          vertices below it become the frontier (near-far
- *                          buckets; push epochs only, no pulls); 0 off; -1
- *                          (default) 2 x the graph's sampled largest weight
+ *   sssp.delta             hc_sssp on the weight-sorted adjacency: distances
+ *                          become final in buckets of this width; push epochs
+ *                          relax only the edges that land in the current
+ *                          bucket, and a promotion epoch settles the bucket's
+ *                          other edges and starts the next one; 0 off; -1
+ *                          (default) 4 x the graph's sampled largest weight
  *                          / mean degree on flat graphs, off on skewed ones
  *                          and with direction 1.  Results do not depend on it
  *   multi.push_div         batched sweep: an epoch whose flagged vertices

@@ -1,0 +1,123 @@
+"""GPU tests of the SSSP sweeps on the weight-sorted adjacency: rows at the
+edges of the sort's classes (4, 16, 64, 512 and 2048 edges, hub chunks), weights
+that one key holds exactly (up to 63) and that share keys (up to 2^30), zero
+weights, unsorted vertex orders, 8-byte offsets, shares, and initial distances
+of every kind.  Distances are the unique fixpoint: equality with the oracle."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _stars(hc, degrees, max_weight, seed, extra=4000):
+    """A graph with one hub of each given degree over a common pool of leaves,
+    and random edges among the leaves."""
+    rng = np.random.default_rng(seed)
+    hubs = len(degrees)
+    leaves = max(degrees) + 8
+    src, dst = [], []
+    for h, d in enumerate(degrees):
+        src.append(np.full(d, h))
+        dst.append(hubs + rng.choice(leaves, d, replace=False))
+    src.append(hubs + rng.integers(0, leaves, extra))
+    dst.append(hubs + rng.integers(0, leaves, extra))
+    src, dst = np.concatenate(src), np.concatenate(dst)
+    w = rng.integers(0, max_weight + 1, src.size).astype(np.int32)
+    return hc.HostGraph.from_edges(src.astype(np.int32), dst.astype(np.int32), hubs + leaves,
+                                   weights=w, relabel=bool(seed % 2))
+
+
+@pytest.fixture(autouse=True)
+def always_sorted(hc):
+    """These graphs are below the size from which the copy is built."""
+    hc.set_tuning("sssp.sorted", 2)
+    yield
+    hc.reset_tuning()
+
+
+DEGREES = [1, 3, 4, 5, 15, 16, 17, 63, 64, 65, 511, 512, 513, 2047, 2048, 2049, 4095, 4096, 4097,
+           20000, 40001]
+
+
+@pytest.mark.parametrize("max_weight", [0, 1, 63, 64, 255, 70000, (1 << 30) - 2])
+@pytest.mark.parametrize("seed", [0, 1])
+def test_sorted_rows_exact(hc, gpu, oracle, max_weight, seed):
+    g = _stars(hc, DEGREES, max_weight, seed)
+    with hc.DeviceGraph(g) as dg:
+        for s in (0, 7, g.num_nodes - 5):
+            ref = oracle.sssp_dijkstra(g.index, g.neighbors, g.weights, s)
+            for direction in (0, 1, 2):
+                assert np.array_equal(hc.sssp(dg, s, direction=direction).values, ref), direction
+            for delta in (max(1, max_weight // 16), max(1, max_weight)):
+                dg.set_tuning("sssp.delta", delta)
+                for direction in (0, 2):
+                    assert np.array_equal(hc.sssp(dg, s, direction=direction).values, ref), delta
+                dg.reset_tuning()
+
+
+def test_sorted_matches_plain_wide_offsets_and_shares(hc, gpu, oracle, monkeypatch):
+    monkeypatch.setenv("HC_FORCE_OFF64", "1")
+    g = _stars(hc, DEGREES, 1000, 3)
+    u = hc.HostGraph.generate("uniform", 12, 6, weighted=True, seed=4)
+    for gg in (g, u):
+        with hc.DeviceGraph(gg) as dg:
+            assert dg.info()["offset_bytes"] == 8
+            s = int(gg.pick_sources(1)[0])
+            ref = oracle.sssp_dijkstra(gg.index, gg.neighbors, gg.weights, s)
+            share = dg.share()
+            for h in (dg, share):
+                assert np.array_equal(hc.sssp(h, s).values, ref)
+            share.set_tuning("sssp.sorted", 0)
+            assert np.array_equal(hc.sssp(share, s).values, ref)
+            share.free()
+
+
+@pytest.mark.parametrize("init", ["one", "many", "low", "negative", "above"])
+def test_sorted_pull_initial_distances(hc, gpu, oracle, init):
+    """hc_sssp_pull from initial distances: the sorted sweeps give what the
+    plain ones give, also for values outside the sentinel's range."""
+    g = hc.HostGraph.generate("kron", 11, 8, weighted=True, seed=9)
+    rng = np.random.default_rng(2)
+    d0 = np.full(g.num_nodes, hc.INF_DIST, np.int32)
+    some = rng.choice(g.num_nodes, 40, replace=False)
+    if init == "one":
+        d0[some[0]] = 0
+    elif init == "many":
+        d0[some] = rng.integers(0, 500, 40)
+    elif init == "low":
+        d0[:] = rng.integers(1000, 2000, g.num_nodes)
+        d0[some] = 990
+    elif init == "negative":
+        d0[some] = rng.integers(-300, 300, 40)
+    else:
+        d0[some[:20]] = 5
+        d0[some[20:]] = hc.INF_DIST + 77
+    with hc.DeviceGraph(g) as dg:
+        got = hc.sssp_pull(dg, d0).values
+        dg.set_tuning("sssp.sorted", 0)
+        assert np.array_equal(got, hc.sssp_pull(dg, d0).values)
+
+
+def test_flat_buckets_cover_every_settling_path(hc, gpu, oracle):
+    """A flat graph whose buckets are settled by pushes (few vertices done) and
+    by sweeps (most done), with sweeps inside heavy buckets; narrow and wide
+    weights, and parts that the source does not reach."""
+    rng = np.random.default_rng(5)
+    n = 30000
+    src, dst = rng.integers(0, n - 500, 8 * n), rng.integers(0, n - 500, 8 * n)
+    for top in (3, 255, 100000):
+        w = rng.integers(1, top + 1, src.size).astype(np.int32)
+        g = hc.HostGraph.from_edges(src.astype(np.int32), dst.astype(np.int32), n, weights=w)
+        with hc.DeviceGraph(g) as dg:
+            for s in (0, 123):
+                ref = oracle.sssp_dijkstra(g.index, g.neighbors, g.weights, s)
+                for delta in (-1, 1, max(1, top // 8), top, 4 * top):
+                    if delta == 1 and top > 255:
+                        continue  # tens of thousands of buckets
+                    dg.set_tuning("sssp.delta", delta)
+                    r = hc.sssp(dg, s)
+                    assert np.array_equal(r.values, ref), (top, delta)
+                    assert r.stats["pull_epochs"] == 0
+                    assert np.array_equal(hc.sssp(dg, s, direction=2).values, ref), (top, delta)
