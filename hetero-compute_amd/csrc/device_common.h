@@ -150,11 +150,13 @@ struct Tuning {
                                  // on flat graphs, off on skewed ones)
     int msbfs = 1;               // batched BFS: bit-parallel levels (1) or the batched
                                  // sweep with unit weights (0)
-    int msbfs_alpha = 32;        // bit-parallel BFS pushes a level while its frontier's
-                                 // edges < m / this, else pulls
+    int msbfs_alpha = 16;        // bit-parallel BFS pushes a level while its frontier's
+                                 // edges < m / this, else pulls (Kronecker 22: 8 / 16 /
+                                 // 32 2.80 / 2.79 / 3.1 ms; uniform: 16 = 8)
     int msbfs_col_shift = -1;    // its pulls gather column blocks of 2^this vertices
-                                 // (0: off; -1: four blocks on flat graphs, sixteen
-                                 // on skewed ones, at least 2^16 vertices each)
+                                 // (0 and -1: off; the copy takes 10-90 ms to build, and
+                                 // pulls with it are slower on Kronecker 22, 2.8 -> 3.4
+                                 // ms, and 6% faster on uniform 23)
     int many_block = 512;        // many-graph BFS: threads per workgroup (256, 512, 1024)
     int many_per_cu = 2;         // ... workgroups per CU (0: as many as the device holds)
     int many_light_deg = 32;     // ... top-down: a thread expands vertices up to this degree

@@ -36,8 +36,6 @@
 namespace hc {
 
 constexpr int kMsQ = 64;
-constexpr int kMsLight = 32;      // push: a thread expands frontier vertices up to this degree
-constexpr int kMsHeavyCap = 512;  // heavier ones (per workgroup pass) go to whole wavefronts
 
 // Per-level counters of one rotation slot: list length, its edge count
 // (sum of degrees), edges examined, depth entries written.
@@ -129,47 +127,67 @@ __device__ __forceinline__ void ms_clear_old(const MsBufs &b, int L) {
         f[q[i]] = 0;
 }
 
-// Edges [i0, e) with stride `step` of a frontier vertex with mask fu: four
-// targets per trip, their ids, then their seen and next masks, loaded
-// before any is used.
-template <typename OffT>
-__device__ __forceinline__ void ms_push_edges(const MsBufs &b, const GraphView<OffT> &g,
-                                              uint64_t *nxt, int32_t *nq, MsCount &c,
-                                              uint64_t fu, OffT i0, OffT e, OffT step,
-                                              unsigned long long &deg_acc,
-                                              unsigned long long &edges) {
-    for (OffT i = i0; i < e; i += 4 * step) {
-        int32_t v[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const OffT k = i + OffT(r) * step;
-            v[r] = k < e ? ldnt(&g.adj[k]) : -1;
-        }
-        uint64_t bits[4], have[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            bits[r] = v[r] >= 0 ? fu & ~b.seen[v[r]] : 0;
-            have[r] = v[r] >= 0 ? nxt[v[r]] : 0;
-        }
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            edges += v[r] >= 0;
-            bool first = false;
-            // An atomic only when it adds a bit the next mask lacks.
-            if (bits[r] & ~have[r])
-                first = atomicOr((unsigned long long *)&nxt[v[r]],
-                                 (unsigned long long)bits[r]) == 0;
-            if (first) deg_acc += (unsigned long long)(g.rend(v[r]) - g.rbeg(v[r]));
-            wave_append(nq, &c.len, first, v[r]);
-        }
-    }
+// A wavefront's part of the next list, collected in LDS and sent with one
+// reservation per kMsStage / 2 entries: appends straight to the list take
+// same-address atomics, which serialize at 12 ns each on this GPU.
+constexpr int kMsStage = 512;
+
+struct MsStage {
+    int32_t *buf;  // kMsStage entries of LDS, this wavefront's
+    int n;         // entries held (the same in every lane)
+};
+
+__device__ __forceinline__ void ms_stage_flush(MsStage &st, int32_t *nq, MsCount &c) {
+    if (st.n == 0) return;
+    // The entries were written by other lanes of this wavefront.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    uint32_t base = 0;
+    if (lane_id() == 0) base = atomicAdd(&c.len, (uint32_t)st.n);
+    base = __shfl(base, 0);
+    for (int i = lane_id(); i < st.n; i += kWave) nq[base + i] = st.buf[i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    st.n = 0;
 }
 
-// Push level L over the list of level L-1.
+__device__ __forceinline__ void ms_stage_append(MsStage &st, bool pred, int32_t v) {
+    const uint64_t m = __ballot(pred);
+    if (pred) st.buf[st.n + __popcll(m & lanemask_lt())] = v;
+    st.n += __popcll(m);
+}
+
+// Push level L over the list of level L-1.  The list is cut into windows of
+// kMsWindow vertices, each taken by as many workgroups as its edges warrant;
+// every one of them sums the window's chunk counts in LDS (kMsChunk edges a
+// chunk, a group of kMsGroup lanes each) and takes its share of the chunks, so
+// a short list of hubs fills the GPU as well as a long one of leaves.
+// (Measured, Kronecker 22, 64 sources: with the list's vertices dealt whole, a
+// wavefront per heavy one, levels of a few thousand hub-rich vertices took
+// 3-14 ms on a handful of workgroups.)
+constexpr int kMsWindow = 4096;
+constexpr int kMsGroup = 16;
+constexpr int kMsTrip = 4;                      // edges a lane has in flight
+constexpr int kMsChunk = kMsGroup * kMsTrip;
+constexpr int kMsPer = kMsWindow / kBlock;
+
+// Workgroups per window of a push from `len` vertices with `deg` edges.
+__host__ __device__ inline int ms_push_share(unsigned long long len, unsigned long long deg,
+                                             int grid) {
+    const unsigned long long wins = (len + kMsWindow - 1) / kMsWindow;
+    if (wins == 0) return 1;
+    // About four chunks (at least one a vertex) for each group of lanes.
+    const unsigned long long want = (deg / kMsChunk + len) / (4ull * kBlock / kMsGroup) + 1;
+    const unsigned long long per = (want + wins - 1) / wins;
+    const unsigned long long most = (unsigned long long)grid / wins;
+    return (int)(per < most ? per : (most ? most : 1));
+}
+
 template <typename OffT>
 __global__ __launch_bounds__(kBlock) void ms_push_kernel(MsBufs b, GraphView<OffT> g, int L) {
-    __shared__ int32_t heavy[kMsHeavyCap];
-    __shared__ int s_nheavy;
+    __shared__ uint32_t s_pre[kMsWindow];
+    __shared__ uint32_t s_wave[kWavesPerBlock];
+    __shared__ int32_t s_stage[kWavesPerBlock][kMsStage];
     const int cu = (L + 2) % 3, nx = L % 3;
     const uint64_t *cur = b.fr[cu];
     uint64_t *nxt = b.fr[nx];
@@ -180,38 +198,99 @@ __global__ __launch_bounds__(kBlock) void ms_push_kernel(MsBufs b, GraphView<Off
     // Counters of buffer nx were reset by the previous commit; the list
     // length read here is level L-1's, final since its commit.
     const unsigned long long len = b.cnt[cu].len;
+    const int per = ms_push_share(len, b.cnt[cu].deg, gridDim.x);
+    const unsigned long long wins = (len + kMsWindow - 1) / kMsWindow;
+    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    MsStage st{s_stage[wave], 0};
     unsigned long long deg_acc = 0, edges = 0;
-    const unsigned long long stride = (unsigned long long)gridDim.x * kBlock;
-    // Rounds of kBlock list entries per workgroup, so the heavy list is
-    // per round and every thread reaches each barrier.
-    for (unsigned long long base = blockIdx.x * (unsigned long long)kBlock; base < len;
-         base += stride) {
-        if (threadIdx.x == 0) s_nheavy = 0;
-        __syncthreads();
-        const unsigned long long i = base + threadIdx.x;
-        if (i < len) {
-            const int32_t u = list[i];
-            const OffT ub = g.rbeg(u), ue = g.rend(u);
-            bool self = true;
-            if (ue - ub > OffT(kMsLight)) {
-                const int slot = atomicAdd(&s_nheavy, 1);
-                if (slot < kMsHeavyCap) {
-                    heavy[slot] = u;
-                    self = false;
-                }
+    const int sub = blockIdx.x % per;
+    for (unsigned long long win = blockIdx.x / per; win < wins; win += gridDim.x / per) {
+        if (blockIdx.x / per >= gridDim.x / per) break;  // past the last full share
+        const int n = (int)min((unsigned long long)kMsWindow, len - win * kMsWindow);
+        const int32_t *wl = list + win * kMsWindow;
+        // Exclusive chunk offsets of the window's vertices, kMsPer per thread.
+        uint32_t mine[kMsPer], t = 0;
+#pragma unroll
+        for (int k = 0; k < kMsPer; k++) {
+            const int i = threadIdx.x * kMsPer + k;
+            uint32_t ch = 0;
+            if (i < n) {
+                const int32_t u = wl[i];
+                ch = (uint32_t)((g.rend(u) - g.rbeg(u) + OffT(kMsChunk - 1)) / OffT(kMsChunk));
             }
-            if (self)
-                ms_push_edges<OffT>(b, g, nxt, nq, c, cur[u], ub, ue, OffT(1), deg_acc, edges);
+            mine[k] = t;
+            t += ch;
         }
-        __syncthreads();
-        const int nh = min(s_nheavy, kMsHeavyCap);
-        for (int h = threadIdx.x / kWave; h < nh; h += kWavesPerBlock) {
-            const int32_t u = heavy[h];
-            ms_push_edges<OffT>(b, g, nxt, nq, c, cur[u], g.rbeg(u) + OffT(lane_id()), g.rend(u),
-                                OffT(kWave), deg_acc, edges);
+        uint32_t incl = t;
+#pragma unroll
+        for (int s = 1; s < kWave; s <<= 1) {
+            const uint32_t o = __shfl_up(incl, s, kWave);
+            if (lane >= s) incl += o;
         }
+        __syncthreads();  // the window before is done with s_pre
+        if (lane == kWave - 1) s_wave[wave] = incl;
         __syncthreads();
+        uint32_t before = incl - t, total = 0;
+        for (int w = 0; w < kWavesPerBlock; w++) {
+            if (w < wave) before += s_wave[w];
+            total += s_wave[w];
+        }
+#pragma unroll
+        for (int k = 0; k < kMsPer; k++) s_pre[threadIdx.x * kMsPer + k] = before + mine[k];
+        __syncthreads();
+        // Chunks in rounds of the wavefront's groups (the same count in all
+        // its lanes).
+        constexpr int kGroups = kWave / kMsGroup;
+        const uint32_t first = (uint32_t)(sub * kWavesPerBlock + wave) * kGroups;
+        const uint32_t step = (uint32_t)per * kWavesPerBlock * kGroups;
+        for (uint32_t q0 = first; q0 < total; q0 += step) {
+            const uint32_t q = q0 + lane / kMsGroup;
+            int32_t v[kMsTrip];
+            uint64_t fu = 0;
+            if (q < total) {
+                int lo = 0, hi = n;
+                while (hi - lo > 1) {
+                    const int mid = (lo + hi) / 2;
+                    if (s_pre[mid] <= q) lo = mid; else hi = mid;
+                }
+                const int32_t u = wl[lo];
+                const OffT e = g.rend(u);
+                const OffT i0 = g.rbeg(u) + OffT(q - s_pre[lo]) * OffT(kMsChunk) +
+                                OffT(lane % kMsGroup);
+                fu = cur[u];
+#pragma unroll
+                for (int r = 0; r < kMsTrip; r++) {
+                    const OffT k = i0 + OffT(r * kMsGroup);
+                    v[r] = k < e ? ldnt(&g.adj[k]) : -1;
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < kMsTrip; r++) v[r] = -1;
+            }
+            uint64_t bits[kMsTrip], have[kMsTrip];
+#pragma unroll
+            for (int r = 0; r < kMsTrip; r++) {
+                bits[r] = v[r] >= 0 ? fu & ~b.seen[v[r]] : 0;
+                have[r] = v[r] >= 0 ? nxt[v[r]] : 0;
+            }
+            bool fresh[kMsTrip];
+#pragma unroll
+            for (int r = 0; r < kMsTrip; r++) {
+                edges += v[r] >= 0;
+                // An atomic only when it adds a bit the next mask lacks.
+                fresh[r] = (bits[r] & ~have[r]) != 0 &&
+                           atomicOr((unsigned long long *)&nxt[v[r]],
+                                    (unsigned long long)bits[r]) == 0;
+            }
+#pragma unroll
+            for (int r = 0; r < kMsTrip; r++) {
+                if (fresh[r]) deg_acc += (unsigned long long)(g.rend(v[r]) - g.rbeg(v[r]));
+                ms_stage_append(st, fresh[r], v[r]);
+            }
+            if (st.n > kMsStage - kMsTrip * kWave) ms_stage_flush(st, nq, c);
+        }
     }
+    ms_stage_flush(st, nq, c);
     const unsigned long long d = block_sum_u64(deg_acc);
     const unsigned long long ed = block_sum_u64(edges);
     if (threadIdx.x == 0) {
@@ -249,11 +328,78 @@ __device__ __forceinline__ uint64_t ms_row_or(const GraphView<OffT> &g, const ui
     return acc;
 }
 
-// Pull level L over the plan (all rows of the graph).
+// A row of a wavefront's block, one per lane.
+template <typename OffT>
+struct MsHead {
+    int32_t v;
+    uint64_t need;  // sources that have not reached it (0: nothing to do)
+    OffT b, e;
+};
+
+// The wanted rows among a wavefront's heads (those of lanes j0, j0 + jstep,
+// ...; which wavefront takes a row must not depend on masks that change), G
+// lanes per row.  SHARED: the heads are chunks of hub rows, whose bits are
+// added with atomicOr.
+template <int G, bool SHARED, typename OffT>
+__device__ __forceinline__ void ms_pull_block(const MsHead<OffT> &h, int j0, int jstep,
+                                              const GraphView<OffT> &g, const uint64_t *cur,
+                                              uint64_t *nxt, int32_t *nq, MsCount &c, MsStage &st,
+                                              unsigned long long &deg_acc,
+                                              unsigned long long &edges) {
+    constexpr int PER = kWave / G;
+    const int lane = lane_id();
+    const bool want = h.need != 0 && lane % jstep == j0;
+    const uint64_t mask = __ballot(want);
+    const int n = __popcll(mask);
+    // Lane r learns the lane of the r-th wanted row.
+    const int rank = __popcll(mask & lanemask_lt());
+    const int src = __builtin_amdgcn_ds_permute((want ? rank : n + lane - rank) << 2, lane);
+    for (int j = 0; j * PER < n; j++) {
+        const int gi = j * PER + lane / G;
+        const bool have = gi < n;
+        const int sl = __shfl(src, gi & (kWave - 1));
+        const int32_t v = __shfl(h.v, sl);
+        const uint64_t need = (uint64_t)__shfl((unsigned long long)h.need, sl);
+        const OffT b = __shfl(h.b, sl), e = __shfl(h.e, sl);
+        uint64_t got = 0;
+        if (have) {
+            got = ms_row_or<G, OffT>(g, cur, b, e, lane % G, need, edges);
+            if (G > 1) got = group_or<G>(got);
+            got &= need;
+        }
+        bool first = false;
+        if (have && lane % G == 0 && got != 0) {
+            if (SHARED) {
+                first = atomicOr((unsigned long long *)&nxt[v], (unsigned long long)got) == 0;
+                if (first) deg_acc += (unsigned long long)(g.rend(v) - g.rbeg(v));
+            } else {
+                nxt[v] = got;  // the only group on this row
+                first = true;
+                deg_acc += (unsigned long long)(e - b);
+            }
+        }
+        ms_stage_append(st, first, v);
+        if (st.n > kMsStage - kWave) ms_stage_flush(st, nq, c);
+    }
+}
+
+// Wavefronts that share a block of 64 heads of hub chunks and heavy rows (64
+// lanes a row), and of 16-lane rows.
+constexpr int kMsSplit = 16;
+constexpr int kMsSplit16 = 4;
+
+// Pull level L over the plan (all rows of the graph; sorted_plan_config), in
+// wavefront units: a block of 64 rows' masks and bounds is read at once, the
+// next block's ahead of this one's edges, and only rows that miss a source
+// get lanes.  (Measured, Kronecker 22, 64 sources, three pull levels: 4.8 ms
+// in column blocks with an append per wavefront straight to the list, 2.5 ms
+// with staged appends, 1.6 ms here without the column blocks, whose copy took
+// 90 ms to build.)
 template <typename OffT>
 __global__ __launch_bounds__(kBlock) void ms_pull_kernel(MsBufs b, GraphView<OffT> g, PlanDev p,
                                                          int L) {
-    __shared__ uint64_t s_or[kWavesPerBlock];
+    __shared__ int32_t s_stage[kWavesPerBlock][kMsStage];
+    MsStage st{s_stage[threadIdx.x / kWave], 0};
     const int cu = (L + 2) % 3, nx = L % 3;
     const uint64_t *cur = b.fr[cu];
     uint64_t *nxt = b.fr[nx];
@@ -261,81 +407,76 @@ __global__ __launch_bounds__(kBlock) void ms_pull_kernel(MsBufs b, GraphView<Off
     MsCount &c = b.cnt[nx];
     ms_clear_old(b, L);
     unsigned long long deg_acc = 0, edges = 0;
-    const int total = p.unit_start[kNumClasses];
-    for (int unit = blockIdx.x; unit < total; unit += gridDim.x) {
-        int cls = 0;
-        while (unit >= p.unit_start[cls + 1]) cls++;
-        const int k = unit - p.unit_start[cls];
-        if (cls <= 1) {
-            // A hub chunk or a whole row per workgroup (unit-uniform).
-            int32_t v;
-            OffT rb, re;
-            if (cls == 0) {
-                const HubChunk h = p.chunks[k];
-                v = h.u;
-                rb = OffT(h.b);
-                re = OffT(h.e);
-            } else {
-                v = p.list[1] ? p.list[1][k] : p.beg[1] + k;
-                rb = g.rbeg(v);
-                re = g.rend(v);
+    const int b0 = (p.cnt[0] + 63) / 64, b2 = (p.cnt[2] + 63) / 64;
+    const int b3 = (p.cnt[3] + 63) / 64, b4 = (p.cnt[4] + 63) / 64, b5 = (p.cnt[5] + 63) / 64;
+    const int stride = gridDim.x * kWavesPerBlock;
+    const int t0 = b0 * kMsSplit, t2 = t0 + b2 * kMsSplit, t3 = t2 + b3 * kMsSplit16;
+    const int t4 = t3 + b4, total = t4 + b5;
+    const int lane = lane_id();
+    auto head = [&](int unit) {
+        MsHead<OffT> h{0, 0, OffT(0), OffT(0)};
+        int i = 0, beg = 0, cnt = 0;
+        const int32_t *list = nullptr;
+        if (unit < t0) {
+            i = unit / kMsSplit * 64 + lane;
+            if (i < p.cnt[0]) {
+                const HubChunk ch = p.chunks[i];
+                h.v = ch.u;
+                h.b = OffT(ch.b);
+                h.e = OffT(ch.e);
+                h.need = b.full & ~b.seen[ch.u];
             }
-            const uint64_t sv = b.seen[v];
-            const uint64_t need = b.full & ~sv;
-            uint64_t acc = 0;
-            if (need) acc = ms_row_or<kBlock, OffT>(g, cur, rb, re, threadIdx.x, need, edges);
-            const uint64_t got = block_or(acc, s_or) & need;
-            bool first = false;
-            if (threadIdx.x == 0 && got) {
-                if (cls == 0) {
-                    first = atomicOr((unsigned long long *)&nxt[v], (unsigned long long)got) == 0;
-                } else {
-                    nxt[v] = got;
-                    first = true;
-                }
-                if (first) deg_acc += (unsigned long long)(g.rend(v) - g.rbeg(v));
-            }
-            if (threadIdx.x < kWave) wave_append(nq, &c.len, first, v);
-            __syncthreads();
-            continue;
+            return h;
+        } else if (unit < t2) {
+            i = (unit - t0) / kMsSplit * 64 + lane;
+            cnt = p.cnt[2];
+            beg = p.beg[2];
+            list = p.list[2];
+        } else if (unit < t3) {
+            i = (unit - t2) / kMsSplit16 * 64 + lane;
+            cnt = p.cnt[3];
+            beg = p.beg[3];
+            list = p.list[3];
+        } else if (unit < t4) {
+            i = (unit - t3) * 64 + lane;
+            cnt = p.cnt[4];
+            beg = p.beg[4];
+            list = p.list[4];
+        } else if (unit < total) {
+            i = (unit - t4) * 64 + lane;
+            cnt = p.cnt[5];
+            beg = p.beg[5];
+            list = p.list[5];
         }
-        // Rows of classes 2-5: G lanes per row, kBlock / G rows per unit.
-        int G = cls == 2 ? 64 : cls == 3 ? 16 : cls == 4 ? 4 : 1;
-        const int per = kBlock / G;
-        const int idx = k * per + (int)threadIdx.x / G;
-        const int li = (int)threadIdx.x % G;
-        const bool ok = idx < p.cnt[cls];
-        int32_t v = 0;
-        uint64_t need = 0, acc = 0;
-        if (ok) {
-            v = p.list[cls] ? p.list[cls][idx] : p.beg[cls] + idx;
-            need = b.full & ~b.seen[v];
-            if (need) {
-                const OffT rb = g.rbeg(v), re = g.rend(v);
-                if (cls == 2)
-                    acc = ms_row_or<64, OffT>(g, cur, rb, re, li, need, edges);
-                else if (cls == 3)
-                    acc = ms_row_or<16, OffT>(g, cur, rb, re, li, need, edges);
-                else if (cls == 4)
-                    acc = ms_row_or<4, OffT>(g, cur, rb, re, li, need, edges);
-                else
-                    acc = ms_row_or<1, OffT>(g, cur, rb, re, li, need, edges);
-            }
+        if (i < cnt) {
+            h.v = list ? list[i] : beg + i;
+            h.need = b.full & ~b.seen[h.v];
+            h.b = g.rbeg(h.v);
+            h.e = g.rend(h.v);
         }
-        if (cls == 2)
-            acc = group_or<64>(acc);
-        else if (cls == 3)
-            acc = group_or<16>(acc);
-        else if (cls == 4)
-            acc = group_or<4>(acc);
-        const uint64_t got = acc & need;
-        const bool first = ok && li == 0 && got != 0;
-        if (first) {
-            nxt[v] = got;  // the only group on this row
-            deg_acc += (unsigned long long)(g.rend(v) - g.rbeg(v));
-        }
-        wave_append(nq, &c.len, first, v);
+        return h;
+    };
+    int unit = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
+    MsHead<OffT> h = head(unit);
+    while (unit < total) {
+        const MsHead<OffT> ahead = head(unit + stride);
+        if (unit < t0)
+            ms_pull_block<64, true>(h, unit % kMsSplit, kMsSplit, g, cur, nxt, nq, c, st, deg_acc,
+                                    edges);
+        else if (unit < t2)
+            ms_pull_block<64, false>(h, (unit - t0) % kMsSplit, kMsSplit, g, cur, nxt, nq, c, st,
+                                     deg_acc, edges);
+        else if (unit < t3)
+            ms_pull_block<16, false>(h, (unit - t2) % kMsSplit16, kMsSplit16, g, cur, nxt, nq, c,
+                                     st, deg_acc, edges);
+        else if (unit < t4)
+            ms_pull_block<4, false>(h, 0, 1, g, cur, nxt, nq, c, st, deg_acc, edges);
+        else
+            ms_pull_block<1, false>(h, 0, 1, g, cur, nxt, nq, c, st, deg_acc, edges);
+        unit += stride;
+        h = ahead;
     }
+    ms_stage_flush(st, nq, c);
     const unsigned long long d = block_sum_u64(deg_acc);
     const unsigned long long ed = block_sum_u64(edges);
     if (threadIdx.x == 0) {
@@ -355,6 +496,8 @@ __global__ __launch_bounds__(kBlock) void ms_pull_cb_kernel(MsBufs b, GraphView<
                                                             GraphView<OffT> cb, int K,
                                                             PlanDev p, int L) {
     __shared__ uint64_t s_or[kWavesPerBlock];
+    __shared__ int32_t s_stage[kWavesPerBlock][kMsStage];
+    MsStage st{s_stage[threadIdx.x / kWave], 0};
     const int cu = (L + 2) % 3, nx = L % 3;
     const uint64_t *cur = b.fr[cu];
     uint64_t *nxt = b.fr[nx];
@@ -386,7 +529,10 @@ __global__ __launch_bounds__(kBlock) void ms_pull_cb_kernel(MsBufs b, GraphView<
                 first = atomicOr((unsigned long long *)&nxt[v], (unsigned long long)got) == 0;
                 if (first) deg_acc += (unsigned long long)(g.rend(v) - g.rbeg(v));
             }
-            if (threadIdx.x < kWave) wave_append(nq, &c.len, first, v);
+            if (threadIdx.x < kWave) {
+                ms_stage_append(st, first, v);
+                if (st.n > kMsStage - kWave) ms_stage_flush(st, nq, c);
+            }
             __syncthreads();
             continue;
         }
@@ -424,8 +570,10 @@ __global__ __launch_bounds__(kBlock) void ms_pull_cb_kernel(MsBufs b, GraphView<
             first = atomicOr((unsigned long long *)&nxt[v], (unsigned long long)got) == 0;
             if (first) deg_acc += (unsigned long long)(g.rend(v) - g.rbeg(v));
         }
-        wave_append(nq, &c.len, first, v);
+        ms_stage_append(st, first, v);
+        if (st.n > kMsStage - kWave) ms_stage_flush(st, nq, c);
     }
+    ms_stage_flush(st, nq, c);
     const unsigned long long d = block_sum_u64(deg_acc);
     const unsigned long long ed = block_sum_u64(edges);
     if (threadIdx.x == 0) {
@@ -434,9 +582,12 @@ __global__ __launch_bounds__(kBlock) void ms_pull_cb_kernel(MsBufs b, GraphView<
     }
 }
 
-// Commit of level L: depth entries of the new bits, seen updated; one
-// wavefront per listed vertex (lane q writes source q's entry).  Resets the
-// counters of buffer (L+1) % 3, which level L+1 fills.
+// Commit of level L: depth entries of the new bits, seen updated.  A
+// wavefront takes 64 listed vertices: their masks are read at once, a lane
+// each, then their rows are written one after another, lane q source q's
+// entry (with a vertex per wavefront the chain list, mask, row bounded the
+// level: 420 us for 2.3 M vertices of Kronecker 22).  Resets the counters of
+// buffer (L+1) % 3, which level L+1 fills.
 __global__ __launch_bounds__(kBlock) void ms_commit_kernel(MsBufs b, int L) {
     const int nx = L % 3;
     const uint64_t *nxt = b.fr[nx];
@@ -444,16 +595,25 @@ __global__ __launch_bounds__(kBlock) void ms_commit_kernel(MsBufs b, int L) {
     const unsigned long long len = b.cnt[nx].len;
     const int lane = lane_id();
     unsigned long long bits = 0;
-    const unsigned long long waves = (unsigned long long)gridDim.x * kWavesPerBlock;
-    for (unsigned long long i = blockIdx.x * (unsigned long long)kWavesPerBlock +
-                                threadIdx.x / kWave;
-         i < len; i += waves) {
-        const int32_t v = q[i];
-        const uint64_t nb = nxt[v];
-        if ((nb >> lane) & 1) b.depth[(size_t)v * kMsQ + lane] = L;
-        if (lane == 0) {
+    const unsigned long long step = (unsigned long long)gridDim.x * kBlock;
+    for (unsigned long long i0 = blockIdx.x * (unsigned long long)kBlock +
+                                 (threadIdx.x / kWave) * kWave;
+         i0 < len; i0 += step) {
+        const int n = (int)min((unsigned long long)kWave, len - i0);
+        int32_t v = 0;
+        uint64_t nb = 0;
+        if (lane < n) {
+            v = q[i0 + lane];
+            nb = nxt[v];
             b.seen[v] |= nb;
             bits += (unsigned long long)__popcll(nb);
+        }
+        const uint32_t lo = (uint32_t)nb, hi = (uint32_t)(nb >> 32);
+        for (int j = 0; j < n; j++) {
+            const int32_t vj = __builtin_amdgcn_readlane(v, j);
+            const uint32_t lj = __builtin_amdgcn_readlane(lo, j);
+            const uint32_t hj = __builtin_amdgcn_readlane(hi, j);
+            if (((lane < 32 ? lj : hj) >> (lane & 31)) & 1u) b.depth[(size_t)vj * kMsQ + lane] = L;
         }
     }
     const unsigned long long t = block_sum_u64(bits);
@@ -520,19 +680,10 @@ static int run_msbfs(hc_graph_s *g, const int32_t *sources, int num, int32_t *de
     MsBfsWs *ws = nullptr;
     HC_TRY(get_msbfs_ws(g, &ws));
     const PlanHost *ph = nullptr;
-    HC_TRY(get_plan(g, 0, g->n, sssp_plan_config(), &ph));
-    // Pull levels gather column block by column block: four blocks on flat
-    // graphs (the copy the SSSP sweeps use), sixteen on skewed ones, whose
-    // hub rows would otherwise gather from the whole mask array (measured,
-    // 64 sources: uniform 23 75 -> 36 ms, Kronecker 24 42 -> 29 ms).
+    HC_TRY(get_plan(g, 0, g->n, sorted_plan_config(), &ph));
     const ColBlocks *cb = nullptr;
     const PlanHost *pcb = nullptr;
-    int shift = tuning().msbfs_col_shift;
-    if (shift < 0) {
-        int lg = 0;
-        while ((int64_t(1) << lg) < (int64_t)g->n) lg++;
-        shift = std::max(16, lg - (flat_graph(g) ? 2 : 4));
-    }
+    const int shift = tuning().msbfs_col_shift;
     if (shift > 0) HC_TRY(get_col_blocks(g, shift, s, &cb));
     if (cb) {
         PlanConfig c = cb_plan_config(cb->K);

@@ -304,10 +304,9 @@ int hc_graph_get_info(hc_graph_t g, hc_graph_info_t *out);
  *   msbfs.on               hc_bfs_multi runs bit-parallel levels (1, default)
  *                          or the batched sweep with unit weights (0)
  *   msbfs.alpha            ... a bit-parallel level pushes while its frontier
- *                          holds fewer than m / this edges, else pulls (32)
+ *                          holds fewer than m / this edges, else pulls (16)
  *   msbfs.col_shift        ... its pulls gather column blocks of 2^this
- *                          vertices (0 off; -1 default: four blocks on flat
- *                          graphs, sixteen on skewed ones, >= 2^16 each)
+ *                          vertices (0, and -1, the default: off)
  *   multi.hub_threshold / multi.hub_chunk / multi.wave_threshold /
  *   multi.g16_threshold    degree classes of the batched sweep
  *   pull.col_shift         pull sweeps of whole graphs with at least two
