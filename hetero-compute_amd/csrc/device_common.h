@@ -519,6 +519,7 @@ constexpr int kSortKeys = 64;
 // 0.40 -> 0.33 ms a query, but 0.53 -> 0.98 ms the first; 31 M edges: 1.13 ->
 // 0.50 ms, the first 1.83 -> 1.85 ms).
 constexpr int64_t kSortedMinEdges = int64_t(1) << 23;
+constexpr int64_t kSortedMinBatchEdges = int64_t(1) << 20;  // batched sweeps
 struct SortedView {
     const int2 *e;
     int32_t shift;

@@ -121,3 +121,25 @@ def test_flat_buckets_cover_every_settling_path(hc, gpu, oracle):
                     assert np.array_equal(r.values, ref), (top, delta)
                     assert r.stats["pull_epochs"] == 0
                     assert np.array_equal(hc.sssp(dg, s, direction=2).values, ref), (top, delta)
+
+
+@pytest.mark.parametrize("max_weight,delta", [(0, -1), (255, -1), (255, 40), (70000, 9000)])
+@pytest.mark.parametrize("seed", [0, 1])
+def test_batched_sweeps_exact(hc, gpu, oracle, max_weight, delta, seed):
+    """The batched sweep on the sorted adjacency, with and without buckets and
+    push epochs: every column is the oracle's, and the plain sweep's."""
+    g = _stars(hc, DEGREES, max_weight, seed)
+    rng = np.random.default_rng(seed)
+    for count, push_div in ((1, 16), (40, 0), (64, 4)):
+        sources = rng.integers(0, g.num_nodes, count)
+        with hc.DeviceGraph(g) as dg:
+            dg.set_tuning("multi.delta", delta)
+            dg.set_tuning("multi.push_div", push_div)
+            r = hc.sssp_multi(dg, sources).values
+            again = hc.sssp_multi(dg, sources).values
+            dg.set_tuning("sssp.sorted", 0)
+            assert np.array_equal(r, hc.sssp_multi(dg, sources).values)
+        assert np.array_equal(r, again)
+        for q in (0, count // 2, count - 1):
+            ref = oracle.sssp_dijkstra(g.index, g.neighbors, g.weights, int(sources[q]))
+            assert np.array_equal(r[q], ref), (count, q)
