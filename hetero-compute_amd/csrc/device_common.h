@@ -107,6 +107,11 @@ struct PlanConfig {
 // vertices are listed per level.
 constexpr int kManyLdsNodesMax = 1 << 17;
 constexpr int kManyHeavyCapMax = 1024;
+// A launch ends with its largest graphs, which want a wide workgroup (512
+// graphs of up to 2^16 vertices: 388 us at 512 threads, 308 at 1024); among
+// small ones its barriers cost more than its width gains (up to 4000
+// vertices: 102 against 123 us).
+constexpr int kManyWideNodes = 8192;
 
 struct Tuning {
     int grid_per_cu = 8;   // workgroups per CU of the fused / step launches
@@ -157,10 +162,12 @@ struct Tuning {
                                  // (0 and -1: off; the copy takes 10-90 ms to build, and
                                  // pulls with it are slower on Kronecker 22, 2.8 -> 3.4
                                  // ms, and 6% faster on uniform 23)
-    int many_block = 512;        // many-graph BFS: threads per workgroup (256, 512, 1024)
+    int many_block = 1024;       // many-graph BFS: threads per workgroup, at most (256, 512,
+                                 // 1024; batches of graphs below kManyWideNodes
+                                 // vertices take at most 512)
     int many_per_cu = 2;         // ... workgroups per CU (0: as many as the device holds)
-    int many_light_deg = 32;     // ... top-down: a thread expands vertices up to this degree
-    int many_heavy_cap = 512;    // ... heavier ones, up to this many per level, by wavefronts
+    int many_light_deg = 8;      // ... top-down: a thread expands vertices up to this degree
+    int many_heavy_cap = 1024;    // ... heavier ones, up to this many per level, by wavefronts
     int many_lds_nodes = 1 << 17;  // ... graphs up to this many vertices keep bitmaps in LDS
     int pull_col_shift = -1;     // pull sweeps gather column blocks of 2^this vertices
                                  // (0: off; -1: automatic, flat graphs only; used

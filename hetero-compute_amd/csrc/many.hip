@@ -112,6 +112,31 @@ __device__ __forceinline__ long long many_block_sum(long long v, long long *s_re
     return t;
 }
 
+// Top-down expansion of u's edges [b, e), G lanes (this one is `lane`), four
+// edges a lane in flight.
+template <int G, bool Global>
+__device__ __forceinline__ void expand(const uint32_t *__restrict__ off,
+                                       const int32_t *__restrict__ adj,
+                                       int32_t *__restrict__ depth, int32_t *__restrict__ parents,
+                                       uint32_t *vis, uint32_t *next, int level, int32_t u,
+                                       uint32_t b, uint32_t e, int lane, long long &cnt,
+                                       long long &sc) {
+    for (uint32_t i = b + lane; i < e; i += 4 * G) {
+        int32_t v[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] = i + r * G < e ? adj[i + r * G] : -1;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            if (v[r] < 0 || !bm_claim<Global>(vis, v[r])) continue;
+            atomicOr(&next[v[r] >> 5], 1u << (v[r] & 31));
+            depth[v[r]] = level;
+            if (parents) parents[v[r]] = u;
+            cnt++;
+            sc += off[v[r] + 1] - off[v[r]];
+        }
+    }
+}
+
 // One direction-optimizing BFS of graph d from src by the whole workgroup;
 // bm holds three bitmaps of `words` words (LDS, or a global slot when
 // Global).  Frontier vertices of degree above light_deg are expanded by
@@ -175,16 +200,8 @@ __device__ __forceinline__ void bfs_one_graph(const Desc &d, int32_t src,
                         }
                     }
                     scanned += e - b;
-                    for (uint32_t i = b; i < e; i++) {
-                        const int32_t v = adj[i];
-                        if (bm_claim<Global>(vis, v)) {
-                            atomicOr(&next[v >> 5], 1u << (v & 31));
-                            depth[v] = level;
-                            if (parents) parents[v] = u;
-                            cnt++;
-                            sc += off[v + 1] - off[v];
-                        }
-                    }
+                    expand<1, Global>(off, adj, depth, parents, vis, next, level, u, b, e, 0, cnt,
+                                      sc);
                 }
             }
             __syncthreads();
@@ -194,34 +211,54 @@ __device__ __forceinline__ void bfs_one_graph(const Desc &d, int32_t src,
                 const int32_t u = heavy[h];
                 const uint32_t b = off[u], e = off[u + 1];
                 if (lane == 0) scanned += e - b;
-                for (uint32_t i = b + lane; i < e; i += kWave) {
-                    const int32_t v = adj[i];
-                    if (bm_claim<Global>(vis, v)) {
-                        atomicOr(&next[v >> 5], 1u << (v & 31));
-                        depth[v] = level;
-                        if (parents) parents[v] = u;
-                        cnt++;
-                        sc += off[v + 1] - off[v];
-                    }
-                }
+                expand<kWave, Global>(off, adj, depth, parents, vis, next, level, u, b, e, lane,
+                                      cnt, sc);
             }
             st.pushes += (tid == 0);
         } else {
             // Bottom-up: every unvisited vertex takes its first neighbour
             // (CSR order) in the frontier.
-            for (int u = tid; u < n; u += BLOCK) {
-                if (bm_get<Global>(vis, u)) continue;
-                const uint32_t b = off[u], e = off[u + 1];
-                for (uint32_t i = b; i < e; i++) {
-                    const int32_t v = adj[i];
+            // kRows vertices a thread at once: their bounds, then their first
+            // neighbours, are in flight together (one workgroup runs the
+            // graph, so the level waits on these chains: 512 graphs, 507 ->
+            // 388 us with this and four edges in flight below).
+            constexpr int kRows = 8;
+            for (int u0 = tid; u0 < n; u0 += kRows * BLOCK) {
+                uint32_t rb[kRows], re[kRows];
+                int32_t f[kRows];
+#pragma unroll
+                for (int k = 0; k < kRows; k++) {
+                    const int u = u0 + k * BLOCK;
+                    const bool open = u < n && !bm_get<Global>(vis, u);
+                    rb[k] = open ? off[u] : 0u;
+                    re[k] = open ? off[u + 1] : 0u;
+                }
+#pragma unroll
+                for (int k = 0; k < kRows; k++) f[k] = rb[k] < re[k] ? adj[rb[k]] : -1;
+#pragma unroll
+                for (int k = 0; k < kRows; k++) {
+                    if (f[k] < 0) continue;
+                    const int u = u0 + k * BLOCK;
+                    int32_t par = -1;
                     scanned++;
-                    if (bm_get<Global>(front, v)) {
+                    if (bm_get<Global>(front, f[k])) par = f[k];
+                    for (uint32_t i = rb[k] + 1; par < 0 && i < re[k]; i += 4) {
+                        int32_t v[4];
+#pragma unroll
+                        for (int r = 0; r < 4; r++) v[r] = i + r < re[k] ? adj[i + r] : -1;
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            if (par >= 0 || v[r] < 0) continue;
+                            scanned++;
+                            if (bm_get<Global>(front, v[r])) par = v[r];
+                        }
+                    }
+                    if (par >= 0) {
                         atomicOr(&vis[u >> 5], 1u << (u & 31));
                         atomicOr(&next[u >> 5], 1u << (u & 31));
                         depth[u] = level;
-                        if (parents) parents[u] = v;
+                        if (parents) parents[u] = par;
                         cnt++;
-                        break;
                     }
                 }
             }
@@ -339,7 +376,8 @@ struct ManyLaunch {
 // that LDS, or many.per_cu per CU when set.
 ManyShape many_shape(const hc_graph_batch_s *b, int *grid, int *slot_words) {
     const Tuning &t = tuning();
-    ManyShape sh{t.many_block, t.many_light_deg, t.many_heavy_cap, 0};
+    const int block = b->max_nodes < kManyWideNodes ? std::min(t.many_block, 512) : t.many_block;
+    ManyShape sh{block, t.many_light_deg, t.many_heavy_cap, 0};
     const int limit = std::min(t.many_lds_nodes, kManyLdsNodesMax);
     int fit = 0;
     for (int i = 0; i < b->num_graphs; i++) {

@@ -323,14 +323,15 @@ int hc_graph_get_info(hc_graph_t g, hc_graph_info_t *out);
  *                          lanes, a wavefront, a workgroup take a row's slice
  *                          in column-blocked sweeps (2 / 12 / 48 / 512)
  *   many.block             threads per workgroup of hc_bfs_many (256, 512
- *                          or 1024; 512)
+ *                          or 1024; 1024), at most 512 where the largest
+ *                          graph has under 8192 vertices
  *   many.per_cu            its workgroups per CU (at most one per graph; 0:
  *                          as many as the device holds with the launch's
  *                          LDS; 2)
  *   many.light_deg         its top-down levels: a thread expands frontier
- *                          vertices up to this degree (32) ...
+ *                          vertices up to this degree (8) ...
  *   many.heavy_cap         ... heavier ones, up to this many per level (at
- *                          most 1024; 512), by whole wavefronts
+ *                          most 1024; 1024), by whole wavefronts
  *   many.lds_nodes         graphs of up to this many vertices (at most 2^17)
  *                          keep their bitmaps in LDS, sized to the largest
  *                          of them in the batch; larger ones use global
