@@ -172,41 +172,106 @@ __device__ __forceinline__ void bu_vertex(const GraphView<OffT> &g,
 // A one-lane row of the plan's last class read ahead of its use (visited
 // flag, first neighbour, bounds), and its bottom-up step once resolved:
 // the same probe and scan as bu_vertex<1> with first-neighbour probes.
-template <typename OffT>
+// HEAD4: the first four neighbours instead of the first (flat graphs).
+template <typename OffT, bool HEAD4>
 struct RowAhead {
-    int32_t u, vis, f;
+    int32_t u, vis;
+    int32_t f[HEAD4 ? 4 : 1];
     OffT b, e;
     bool ok;
 };
 
-template <typename OffT>
-__device__ __forceinline__ RowAhead<OffT> row_ahead(const PlanDev &p, int k,
-                                                    const GraphView<OffT> &g,
-                                                    const int32_t *__restrict__ visited,
-                                                    const int32_t *__restrict__ first) {
-    RowAhead<OffT> r;
+template <bool HEAD4, typename OffT>
+__device__ __forceinline__ RowAhead<OffT, HEAD4> row_ahead(const PlanDev &p, int k,
+                                                           const GraphView<OffT> &g,
+                                                           const int32_t *__restrict__ visited,
+                                                           const int32_t *__restrict__ first) {
+    RowAhead<OffT, HEAD4> r;
     const int idx = k * kBlock + threadIdx.x;
     r.ok = idx < p.cnt[5];
     r.u = r.ok ? (p.list[5] ? p.list[5][idx] : p.beg[5] + idx) : 0;
     r.vis = r.ok ? visited[r.u] : 0;
-    r.f = r.ok ? first[r.u] : -1;
+    if constexpr (HEAD4) {
+        const int4 h = r.ok ? reinterpret_cast<const int4 *>(first)[r.u] : int4{-1, -1, -1, -1};
+        r.f[0] = h.x;
+        r.f[1] = h.y;
+        r.f[2] = h.z;
+        r.f[3] = h.w;
+    } else {
+        r.f[0] = r.ok ? first[r.u] : -1;
+    }
     r.b = r.ok ? g.rbeg(r.u) : OffT(0);
     r.e = r.ok ? g.rend(r.u) : OffT(0);
     return r;
 }
 
-template <typename OffT>
-__device__ __forceinline__ void row_resolve(const RowAhead<OffT> &r, const GraphView<OffT> &g,
+template <bool HEAD4, typename OffT>
+__device__ __forceinline__ void row_resolve(const RowAhead<OffT, HEAD4> &r,
+                                            const GraphView<OffT> &g,
                                             const Staged<uint32_t> &frontier, bool &found,
                                             bool &open, int32_t &par, uint32_t &scanned,
                                             int64_t &deg) {
     deg = int64_t(r.e - r.b);
     if (!r.ok || r.vis >= 0) return;
     int32_t pr = -1;
-    const bool fnd = bu_scan<1, true>(g, frontier, r.b, r.e, 0, 0, pr, scanned, r.f);
+    bool fnd = false;
+    if constexpr (HEAD4) {
+        bool h[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) h[k] = r.f[k] >= 0 && bit_test(frontier, r.f[k]);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (fnd || r.f[k] < 0) continue;
+            scanned++;
+            fnd = h[k];
+            pr = h[k] ? r.f[k] : pr;
+        }
+    } else {
+        if (r.f[0] >= 0) {
+            scanned++;
+            fnd = bit_test(frontier, r.f[0]);
+            pr = fnd ? r.f[0] : -1;
+        }
+    }
+    // (the caller scans on: row_scan_packed)
     found = fnd;
     open = !fnd;
     par = pr;
+}
+
+// The rows of a wavefront that are still open after the neighbours read ahead,
+// scanned on by groups of four lanes: one lane a row, the
+// wavefront would wait for its longest scan (uniform graph of 5 M vertices,
+// the first bottom-up level: 360 us so, 310 with the first four neighbours
+// from their array).
+template <bool HEAD4, typename OffT>
+__device__ __forceinline__ void row_scan_packed(const RowAhead<OffT, HEAD4> &r,
+                                                const GraphView<OffT> &g,
+                                                const Staged<uint32_t> &frontier, bool &found,
+                                                bool &open, int32_t &par, uint32_t &scanned) {
+    constexpr int G = 4, PER = kWave / G, SEEN = HEAD4 ? 4 : 1;
+    const int lane = lane_id();
+    const bool want = open && r.e - r.b > OffT(SEEN);
+    const uint64_t mask = __ballot(want);
+    const int n = __popcll(mask);
+    const int rank = __popcll(mask & lanemask_lt());
+    // Lane k learns the lane of the k-th wanted row.
+    const int src = __builtin_amdgcn_ds_permute((want ? rank : n + lane - rank) << 2, lane);
+    for (int j = 0; j * PER < n; j++) {
+        const int gi = j * PER + lane / G;
+        const int sl = __shfl(src, gi & (kWave - 1));
+        const OffT b = __shfl(r.b, sl) + OffT(SEEN), e = __shfl(r.e, sl);
+        int32_t pr = -1;
+        bool f = false;
+        if (gi < n) f = bu_scan<G>(g, frontier, b, e, lane % G, lane - lane % G, pr, scanned);
+        // Each row's lane reads its group's outcome.
+        const int32_t got = __shfl(f ? pr : -1, (rank % PER) * G);
+        if (want && rank / PER == j && got >= 0) {
+            found = true;
+            open = false;
+            par = got;
+        }
+    }
 }
 
 template <int G, typename OffT>
@@ -265,11 +330,12 @@ __device__ __forceinline__ void bu_commit(const GraphView<OffT> &g,
 // and a bit in the next-frontier bitmap, counted with their degree; with
 // `rem`, vertices that stay unvisited are listed for the next sweep.
 // Epoch API: visited is parents.
-template <bool LOOP, typename OffT>
-__device__ void bu_sweep(const PlanDev &p, const GraphView<OffT> &g,
+template <bool LOOP, bool HEAD4, typename OffT>
+__device__ __forceinline__ void bu_sweep(const PlanDev &p, const GraphView<OffT> &g,
                          int32_t *__restrict__ visited, int32_t *__restrict__ parents,
                          const int32_t *__restrict__ first, const int32_t *__restrict__ first_g,
-                         int32_t level, const Staged<uint32_t> &frontier,
+                         const int32_t *__restrict__ head, int32_t level,
+                         const Staged<uint32_t> &frontier,
                          uint32_t *__restrict__ next, int32_t *rem, uint32_t *rem_cnt,
                          uint32_t &cnt, unsigned long long &edges_acc, uint32_t &scanned) {
     const int total = p.unit_start[kNumClasses];
@@ -277,21 +343,22 @@ __device__ void bu_sweep(const PlanDev &p, const GraphView<OffT> &g,
         int c = 0;
         while (unit >= p.unit_start[c + 1]) c++;
         const int k = unit - p.unit_start[c];
-        if (LOOP && c == 5 && first) {
+        if (LOOP && c == 5 && head) {
             // One-lane rows, the last class: this workgroup's remaining
             // units in a pipeline that reads the next unit's rows before
             // committing this unit's, so the commit's stores and atomics
             // are not waited for before the next loads are in flight.
-            RowAhead<OffT> cur = row_ahead(p, k, g, visited, first);
+            RowAhead<OffT, HEAD4> cur = row_ahead<HEAD4>(p, k, g, visited, head);
             for (;;) {
                 const int nunit = unit + (int)gridDim.x;
                 const bool more = nunit < total;
-                RowAhead<OffT> nx{0, 0, -1, OffT(0), OffT(0), false};
-                if (more) nx = row_ahead(p, nunit - p.unit_start[5], g, visited, first);
+                RowAhead<OffT, HEAD4> nx{};
+                if (more) nx = row_ahead<HEAD4>(p, nunit - p.unit_start[5], g, visited, head);
                 bool found = false, open = false;
                 int32_t par = -1;
                 int64_t deg = -1;
-                row_resolve(cur, g, frontier, found, open, par, scanned, deg);
+                row_resolve<HEAD4>(cur, g, frontier, found, open, par, scanned, deg);
+                row_scan_packed<HEAD4>(cur, g, frontier, found, open, par, scanned);
                 bu_commit<LOOP>(g, visited, parents, level, next, rem, rem_cnt, found, open,
                                 cur.u, par, deg, cnt, edges_acc);
                 if (!more) return;
@@ -441,13 +508,107 @@ __device__ void td_sweep(const GraphView<OffT> &g, int32_t *__restrict__ depth,
     }
 }
 
+// Stage 1 of a heavy top-down epoch: unvisited neighbours get their depth by
+// plain stores (every writer of a vertex writes the same value, and any of the
+// writers' parents is one of the level before).  Edges as in td_sweep, four a
+// lane in flight.
+template <int G, typename OffT>
+__device__ __forceinline__ void mark_range(const GraphView<OffT> &g, int32_t *depth,
+                                           int32_t *parents, int32_t level, int32_t u, OffT b,
+                                           OffT e, int lane, uint32_t &scanned) {
+    constexpr int R = 4;
+    for (OffT i = b + OffT(lane); i < e; i += OffT(R * G)) {
+        int32_t v[R], d[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const OffT k = i + OffT(r * G);
+            v[r] = k < e ? g.adj[k] : -1;
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) d[r] = v[r] >= 0 ? depth[v[r]] : 0;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            scanned += v[r] >= 0 ? 1u : 0u;
+            if (d[r] < 0) {
+                depth[v[r]] = level;
+                if (parents) parents[v[r]] = u;
+            }
+        }
+    }
+}
+
+template <typename OffT>
+__device__ __forceinline__ void mark_sweep(const GraphView<OffT> &g, int32_t *depth,
+                                           int32_t *parents, int32_t level,
+                                           const FrontierBufs &fb, int cur, uint32_t &scanned) {
+    const uint32_t nch = fb.cnt[cur][3], n0 = fb.cnt[cur][0],
+                   n1 = fb.cnt[cur][1], n2 = fb.cnt[cur][2];
+    const uint32_t u1 = nch + n0;
+    const uint32_t u2 = u1 + (n1 + kWavesPerBlock - 1) / kWavesPerBlock;
+    const uint32_t total = u2 + (n2 + kSmallPerUnit - 1) / kSmallPerUnit;
+    for (uint32_t unit = blockIdx.x; unit < total; unit += gridDim.x) {
+        if (unit < nch) {
+            const HubChunk h = fb.ch[cur][unit];
+            mark_range<kBlock>(g, depth, parents, level, h.u, OffT(h.b), OffT(h.e), threadIdx.x,
+                               scanned);
+        } else if (unit < u1) {
+            const int32_t u = fb.q[cur][0][unit - nch];
+            mark_range<kBlock>(g, depth, parents, level, u, g.rbeg(u), g.rend(u), threadIdx.x,
+                               scanned);
+        } else if (unit < u2) {
+            const uint32_t idx = (unit - u1) * kWavesPerBlock + threadIdx.x / kWave;
+            if (idx < n1) {
+                const int32_t u = fb.q[cur][1][idx];
+                mark_range<kWave>(g, depth, parents, level, u, g.rbeg(u), g.rend(u), lane_id(),
+                                  scanned);
+            }
+        } else {
+            const uint32_t idx = (unit - u2) * kSmallPerUnit + threadIdx.x / kSmallLanes;
+            if (idx < n2) {
+                const int32_t u = fb.q[cur][2][idx];
+                mark_range<kSmallLanes>(g, depth, parents, level, u, g.rbeg(u), g.rend(u),
+                                        threadIdx.x % kSmallLanes, scanned);
+            }
+        }
+    }
+}
+
+// Stage 2: the vertices of depth `level` are the next frontier.  A wavefront
+// owns two words of the bitmap and writes both.
+template <typename OffT>
+__device__ __forceinline__ void collect_level(const GraphView<OffT> &g, const int32_t *depth,
+                                              int32_t level, uint32_t *next, uint32_t &cnt,
+                                              unsigned long long &edges_acc) {
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    for (int64_t i0 = (int64_t)blockIdx.x * kBlock; i0 < g.n; i0 += stride) {
+        const int64_t i = i0 + threadIdx.x;
+        const bool hit = i < g.n && depth[i] == level;
+        const uint64_t m = __ballot(hit);
+        if (hit) {
+            cnt++;
+            edges_acc += (unsigned long long)(g.rend((int32_t)i) - g.rbeg((int32_t)i));
+        }
+        if (lane_id() == 0 && i < g.n) next[i >> 5] = uint32_t(m);
+        if (lane_id() == 32 && i < g.n) next[i >> 5] = uint32_t(m >> 32);
+    }
+}
+
+// A top-down epoch is heavy when its edges outnumber this: below, its claims
+// and bits cost less than the second launch and the scan (n / 16: 4 bytes a
+// vertex against two atomics an edge; Kronecker 23, 6.1 M edges: 157 us with
+// claims).
+__device__ __forceinline__ bool heavy_push(long long edges, long long n) {
+    return edges > (1ll << 19) + n / 16;
+}
+
 // `nstage` leading frontier-bitmap words are staged in dynamic LDS for
 // bottom-up epochs; top-down epochs stage up to `push_cap` output entries
 // there.
-template <typename OffT>
+template <typename OffT, bool HEAD4>
 __global__ __launch_bounds__(kBlock) void bfs_step_kernel(
     PlanDev p, GraphView<OffT> g, int32_t *__restrict__ depth,
-    int32_t *__restrict__ parents, const int32_t *__restrict__ first, FrontierBufs fb,
+    int32_t *__restrict__ parents, const int32_t *__restrict__ first,
+    const int32_t *__restrict__ head4, FrontierBufs fb,
     StepCtl *ctl, RemLists rl, int32_t nstage, int32_t stage_min, int32_t push_cap,
     int first_all) {
     extern __shared__ uint32_t s_words[];
@@ -487,14 +648,19 @@ __global__ __launch_bounds__(kBlock) void bfs_step_kernel(
                 bu_list_sweep<1>(g, depth, parents, first, level, fr, next, list, len, rem, &s_rem,
                                  cnt, eacc, scanned);
         } else
-            bu_sweep<true>(p, g, depth, parents, first, first_all ? first : nullptr, level, fr,
-                           next, rem, &s_rem, cnt, eacc, scanned);
+            bu_sweep<true, HEAD4>(p, g, depth, parents, first, first_all ? first : nullptr,
+                                  HEAD4 ? head4 : first, level, fr, next, rem, &s_rem, cnt, eacc,
+                                  scanned);
         if (listing) {
             __syncthreads();
             if (threadIdx.x == 0) rl.len[nxt * gridDim.x + blockIdx.x] = s_rem;
             list_in = len;
             list_out = s_rem;
         }
+    } else if (ctl->stage == 1) {
+        mark_sweep(g, depth, parents, level, fb, cur, scanned);
+    } else if (ctl->stage == 2) {
+        collect_level(g, depth, level, next, cnt, eacc);
     } else {
         // Top-down: output staged in the dynamic LDS (unused by this mode).
         __shared__ uint32_t s_out;
@@ -516,7 +682,15 @@ __device__ void bfs_decide(StepCtl *c, StepCtl *trace, const unsigned long long 
                            int offb) {
     // Frontier size and degree sum, edges examined, unvisited-list lengths
     // read and written by a pull epoch.
-    const unsigned long long q = sums[0], sc = sums[1], scanned = sums[2];
+    if (c->stage == 1) {  // the epoch goes on: its frontier is still to be collected
+        c->stage = 2;
+        c->stage_edges = sums[2];
+        c->need_compact = 0;
+        return;
+    }
+    const bool collected = c->stage == 2;
+    const unsigned long long q = sums[0], sc = sums[1];
+    const unsigned long long scanned = collected ? c->stage_edges : sums[2];
     const unsigned long long lin = sums[3], lout = sums[4];
     const int k = c->epoch;
     const int ran = c->mode;
@@ -576,7 +750,8 @@ __device__ void bfs_decide(StepCtl *c, StepCtl *trace, const unsigned long long 
         }
     }
     if (c->max_epochs > 0 && k + 1 >= c->max_epochs) c->done = 1;
-    c->need_compact = (!c->done && ran == kPull && next == kPush) ? 1 : 0;
+    c->need_compact = (!c->done && (ran == kPull || collected) && next == kPush) ? 1 : 0;
+    c->stage = next == kPush && heavy_push((long long)sc, n) ? 1 : 0;
     // A pull epoch listed the vertices it left open; the next pull reads that
     // list unless the list mode is switched off.
     c->rem_valid = (c->rem_knob && ran == kPull && next == kPull) ? 1 : 0;
@@ -625,6 +800,8 @@ __global__ __launch_bounds__(kBlock) void bfs_init_kernel(
             for (int j = 0; j < 5; j++) fb.cnt[p][j] = 0;
         ctl->done = 0;
         ctl->epoch = 0;
+        ctl->steps = 0;
+        ctl->stage = 0;
         ctl->max_epochs = max_epochs;
         ctl->direction = direction;
         ctl->alpha = alpha;
@@ -686,8 +863,9 @@ __global__ __launch_bounds__(kBlock) void bfs_pull_fused_kernel(
     extern __shared__ uint32_t s_words[];
     uint32_t nnew = 0, scanned = 0;
     unsigned long long eacc = 0;
-    bu_sweep<false>(p, g, parents, nullptr, nullptr, nullptr, 0, stage(frontier, nstage, s_words), next,
-                    nullptr, nullptr, nnew, eacc, scanned);
+    bu_sweep<false, false>(p, g, parents, nullptr, nullptr, nullptr, nullptr, 0,
+                           stage(frontier, nstage, s_words), next, nullptr, nullptr, nnew, eacc,
+                           scanned);
     unsigned long long s = block_sum_u64(nnew);
     if (threadIdx.x == 0 && s) atomicAdd(num_nodes, (int32_t)s);
 }
@@ -779,10 +957,27 @@ __global__ __launch_bounds__(kBlock) void first_neighbour_kernel(GraphView<OffT>
     }
 }
 
+// The first four neighbours of each row (-1 past its end).
+template <typename OffT>
+__global__ __launch_bounds__(kBlock) void head4_kernel(GraphView<OffT> g, int4 *__restrict__ head) {
+    for (int u = blockIdx.x * kBlock + threadIdx.x; u < g.n; u += gridDim.x * kBlock) {
+        const OffT b = g.rbeg(u), e = g.rend(u);
+        int32_t v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = b + OffT(k) < e ? g.adj[b + OffT(k)] : -1;
+        head[u] = int4{v[0], v[1], v[2], v[3]};
+    }
+}
+
 struct BfsWs {
     FrontierWs f;
     int32_t *depth = nullptr;  // used when the caller passes no depth array
     int32_t *first = nullptr;  // first neighbour of each vertex (-1: no edges)
+    // First four neighbours of each vertex, on flat graphs: there a row's first
+    // neighbour is in the frontier no more often than the others, and the scan
+    // of the edge array would fetch a line per row for the next few.  (No
+    // memory for it: the rows scan on.)
+    int32_t *head4 = nullptr;
     // Unvisited-list segments: off[grid + 1] then len[2][grid] (sized for
     // f.grid workgroups), laid out for rem_plan at rem_grid workgroups.
     int32_t *rem = nullptr;
@@ -819,9 +1014,13 @@ void free_bfs_ws(hc_graph_s *g) {
     if (ws->depth) hipFree(ws->depth);
     if (ws->rem) hipFree(ws->rem);
     if (ws->first) hipFree(ws->first);
+    if (ws->head4) hipFree(ws->head4);
     delete ws;
     g->ws_bfs = nullptr;
 }
+
+// Below this the edge array stays in cache anyway.
+constexpr int32_t kHead4MinNodes = 1 << 19;
 
 static int get_bfs_ws(hc_graph_s *g, BfsWs **out, hipStream_t s) {
     // The partial slots are sized for the launch grid; re-allocate when the
@@ -845,6 +1044,18 @@ static int get_bfs_ws(hc_graph_s *g, BfsWs **out, hipStream_t s) {
         }
         if (g->n > 0) {
             const int nb = std::min((g->n + kBlock - 1) / kBlock, 65536);
+            if (flat_graph(g) && g->n >= kHead4MinNodes) {
+                if (hipMalloc(&ws->head4, sizeof(int4) * (size_t)g->n) != hipSuccess) {
+                    (void)hipGetLastError();
+                    ws->head4 = nullptr;
+                } else if (g->off64) {
+                    head4_kernel<<<nb, kBlock, 0, s>>>(view<uint64_t>(g),
+                                                       reinterpret_cast<int4 *>(ws->head4));
+                } else {
+                    head4_kernel<<<nb, kBlock, 0, s>>>(view<uint32_t>(g),
+                                                       reinterpret_cast<int4 *>(ws->head4));
+                }
+            }
             if (g->off64)
                 first_neighbour_kernel<<<nb, kBlock, 0, s>>>(view<uint64_t>(g), ws->first);
             else
@@ -868,6 +1079,7 @@ struct BfsLaunch {
     int32_t *depth;
     int32_t *parents;
     const int32_t *first;
+    const int32_t *head4;
     FrontierBufs fb;
     StepCtl *ctl;
     RemLists rl;
@@ -879,16 +1091,20 @@ struct BfsLaunch {
     int32_t push_cap;
     int first_all;
     KernelTimer *kt;
+    template <bool HEAD4>
+    void step(FrontierBufs b, StepCtl *cur) {
+        timed_launch(kt, bfs_step_kernel<OffT, HEAD4>, dim3(grid), dim3(kBlock),
+                     uint32_t(lds_words * sizeof(uint32_t)), s, plan, g, depth, parents, first,
+                     head4, b, cur, rl, nstage, stage_min, push_cap, first_all);
+    }
     // Epoch k: header slot k & 1, counter set k % 3.
     static int launch(void *arg, long long k) {
         auto *a = static_cast<BfsLaunch *>(arg);
         FrontierBufs fb = a->fb;
         fb.part = sum_set(a->fb.part, k);
         StepCtl *cur = a->ctl + (k & 1), *nxt = a->ctl + ((k + 1) & 1);
-        timed_launch(a->kt, bfs_step_kernel<OffT>, dim3(a->grid), dim3(kBlock),
-                     uint32_t(a->lds_words * sizeof(uint32_t)), a->s, a->plan, a->g, a->depth,
-                     a->parents, static_cast<const int32_t *>(a->first), fb, cur, a->rl,
-                     a->nstage, a->stage_min, a->push_cap, a->first_all);
+        if (a->head4) a->template step<true>(fb, cur);
+        else a->template step<false>(fb, cur);
         bfs_between_kernel<OffT><<<compact_grid(a->grid), kBlock, 0, a->s>>>(
             a->g, fb, cur, nxt, a->ctl, sum_set(a->fb.part, k + 1), (int)sizeof(OffT));
         if (hipGetLastError() != hipSuccess) return fail(HC_ERR_HIP, "BFS epoch launch failed");
@@ -913,8 +1129,11 @@ static int run_bfs_loop(hc_graph_s *g, int32_t src, int32_t *depth,
     // of top-down epochs, whichever is larger.
     const int32_t push_cap = tuning().push_stage;
     const int32_t lds_words = std::max<int32_t>(nstage, push_cap);
-    const int grid = resident_grid(reinterpret_cast<const void *>(&bfs_step_kernel<OffT>),
-                                   kBlock, lds_words * sizeof(uint32_t), ws->f.grid);
+    const int32_t *head4 = tuning().bu_first ? ws->head4 : nullptr;
+    const int grid =
+        resident_grid(head4 ? reinterpret_cast<const void *>(&bfs_step_kernel<OffT, true>)
+                            : reinterpret_cast<const void *>(&bfs_step_kernel<OffT, false>),
+                      kBlock, lds_words * sizeof(uint32_t), ws->f.grid);
     if (grid > ws->f.grid) return fail(HC_ERR_HIP, "BFS grid %d above its workspace", grid);
     HC_TRY(bfs_rem_layout(ws, ph, grid, s));
     const int init_grid = std::max(1, std::min(grid, (g->n + kBlock - 1) / kBlock));
@@ -925,7 +1144,7 @@ static int run_bfs_loop(hc_graph_s *g, int32_t src, int32_t *depth,
     ws->f.kt.reset();
     const RemLists rl{ws->rem, reinterpret_cast<uint32_t *>(ws->rem + grid + 1)};
     BfsLaunch<OffT> L{ph->dev, v, depth, parents, tuning().bu_first ? ws->first : nullptr,
-                      ws->f.fb, ws->f.ctl, rl, grid, s, nstage, tuning().bu_stage_min,
+                      head4, ws->f.fb, ws->f.ctl, rl, grid, s, nstage, tuning().bu_stage_min,
                       lds_words, push_cap, tuning().bu_first == 2, &ws->f.kt};
     const long long cap = (long long)g->n + 2;  // levels <= n
     float ms = 0;
@@ -946,7 +1165,7 @@ static int run_bfs_loop(hc_graph_s *g, int32_t src, int32_t *depth,
         stats->reached = (int64_t)fc.reached;
         stats->alg_bytes = (double)fc.alg_bytes;
         if (ws->f.kt.on) {
-            stats->kernel_launches = std::min(fc.epoch, ws->f.kt.pairs());
+            stats->kernel_launches = (int32_t)std::min<long long>(fc.steps, ws->f.kt.pairs());
             stats->kernel_ms = ws->f.kt.sum_ms(stats->kernel_launches);
         }
     }

@@ -186,7 +186,7 @@ struct Tuning {
         bu.block_threshold = INT64_MAX;
         bu.wave_threshold = 4096;
         bu.g16_threshold = 512;
-        bu.g4_threshold = 64;
+        bu.g4_threshold = 128;
         multi.hub_threshold = 2048;
         multi.hub_chunk = 1024;
         multi.block_threshold = INT64_MAX;

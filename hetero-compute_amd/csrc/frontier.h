@@ -76,7 +76,13 @@ struct StepCtl {
     int32_t rem_knob;              // BFS: lanes per listed vertex, 0: no lists
     int32_t chunk;                 // edges per hub chunk of push epochs
     int32_t mid;                   // degree above which a push gives a vertex a wavefront
-    int32_t pad;
+    // Heavy push epochs run in two launches, since random atomics are scarce
+    // on this GPU (27 G/s, where random stores reach 85 and more): 1, plain
+    // stores mark what the push reaches; 2, a scan of the state collects the
+    // frontier (0: a push with claims and queues, in one launch).
+    int32_t stage;
+    long long steps;                 // launch pairs that did work
+    unsigned long long stage_edges;  // edges examined by stage 1
     // SSSP on the weight-sorted adjacency: a lower bound of every distance
     // that changed in the epoch before (rows at or below it, and edges that
     // cannot beat the row's distance from it, are not looked at).
@@ -527,6 +533,7 @@ __device__ __forceinline__ bool ctl_begin(StepCtl *s_c, const StepCtl *cur, cons
     __syncthreads();
     if (s_c->done) return false;
     sum_partials(part, sums);  // ends with a barrier
+    if (threadIdx.x == 0) s_c->steps++;
     return true;
 }
 

@@ -111,7 +111,7 @@ int read_final_ctl(const StepCtl *d, StepCtl *out, hipStream_t s) {
     HC_HIP(hipMemcpyAsync(h, d, 2 * sizeof(StepCtl), hipMemcpyDeviceToHost, s));
     HC_HIP(hipStreamSynchronize(s));
     *out = h[0];
-    if (h[1].epoch > h[0].epoch)
+    if (h[1].steps > h[0].steps)
         std::memcpy(out, &h[1], sizeof(unsigned long long) * kCtlHeadWords);
     return HC_OK;
 }

@@ -1130,6 +1130,8 @@ __global__ __launch_bounds__(kBlock) void sssp_init_kernel(
             for (int j = 0; j < 5; j++) fb.cnt[p][j] = 0;
         ctl->done = 0;
         ctl->epoch = 0;
+        ctl->steps = 0;
+        ctl->stage = 0;
         ctl->max_epochs = max_epochs;
         ctl->direction = direction;
         ctl->alpha = alpha;
@@ -1571,7 +1573,7 @@ static int run_sssp_loop(hc_graph_s *g, int32_t src, const int32_t *init_dist,
         stats->reached = -1;
         stats->alg_bytes = (double)fc.alg_bytes;
         if (ws->f.kt.on) {
-            stats->kernel_launches = std::min(fc.epoch, ws->f.kt.pairs());
+            stats->kernel_launches = (int32_t)std::min<long long>(fc.steps, ws->f.kt.pairs());
             stats->kernel_ms = ws->f.kt.sum_ms(stats->kernel_launches);
         }
     }

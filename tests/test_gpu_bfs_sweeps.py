@@ -1,0 +1,60 @@
+"""GPU tests of the BFS loop where its launches divide: top-down epochs on both
+sides of the size from which they mark by plain stores and collect by a scan,
+and bottom-up rows whose scan ends at, or just past, the neighbours read ahead
+(one on skewed graphs, four on flat ones).  Depths are unique; parents are
+valid, and bottom-up the first frontier neighbour."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(hc, oracle, g, sources, directions=(0, 1, 2)):
+    with hc.DeviceGraph(g) as dg:
+        for s in sources:
+            depth = oracle.bfs_depth(g.index, g.neighbors, s)
+            for direction in directions:
+                b = hc.bfs(dg, s, direction=direction)
+                assert np.array_equal(b.values, depth), (s, direction)
+                assert oracle.verify_parents(depth, b.parents, s) == 0, (s, direction)
+            _, _, dirs = oracle.bfs_do(g.index, g.neighbors, s)
+            hc.bfs(dg, s)
+            tr = hc.epoch_trace(dg, "bfs")
+            assert [e["mode"] == "pull" for e in tr] == [bool(x) for x in dirs]
+            reached = int((depth >= 0).sum())
+            assert 1 + sum(e["frontier"] for e in tr) == reached
+
+
+@pytest.mark.parametrize("leaves", [5000, 560000, 900000])
+def test_heavy_top_down_epochs(hc, gpu, oracle, leaves):
+    """Twelve hubs over a pool of leaves and a tail behind the leaves: the
+    second epoch pushes 12 * leaves / 8 edges, many to the same leaves."""
+    rng = np.random.default_rng(leaves)
+    hubs, tail = 12, 70
+    per = leaves // 8
+    src = [np.zeros(hubs, int)] + [np.full(per, 1 + h) for h in range(hubs)]
+    dst = [1 + np.arange(hubs)] + [1 + hubs + rng.choice(leaves, per, replace=False)
+                                   for _ in range(hubs)]
+    last = hubs + leaves
+    src.append(last + np.arange(tail))
+    dst.append(last + 1 + np.arange(tail))
+    g = hc.HostGraph.from_edges(np.concatenate(src).astype(np.int32),
+                                np.concatenate(dst).astype(np.int32), 1 + hubs + leaves + tail)
+    _check(hc, oracle, g, [0, int(dst[1][0])])
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("degree", [1, 2, 3, 9])
+def test_flat_rows_read_ahead(hc, gpu, oracle, monkeypatch, degree, wide):
+    """Flat graphs above the size from which four neighbours are read ahead:
+    rows of zero to a few dozen edges, vertices the source does not reach."""
+    if wide:
+        monkeypatch.setenv("HC_FORCE_OFF64", "1")
+    rng = np.random.default_rng(degree)
+    n = (1 << 19) + 77
+    src = rng.integers(0, n - 1000, degree * n).astype(np.int32)
+    dst = rng.integers(0, n - 1000, degree * n).astype(np.int32)
+    g = hc.HostGraph.from_edges(src, dst, n)
+    _check(hc, oracle, g, [int(src[0])], directions=(0, 1))
