@@ -1112,12 +1112,35 @@ struct BfsLaunch {
     }
 };
 
+static void fill_bfs_stats(const StepCtl &fc, int32_t launches, hc_run_stats_t *stats) {
+    if (!stats) return;
+    std::memset(stats, 0, sizeof(*stats));
+    // Device wall clock from the init kernel to the controller of the
+    // last epoch (launches queued past it are not part of the loop).
+    stats->ms = double(fc.t_end - fc.t_start) / device_state().clock_khz;
+    stats->epochs = fc.epoch;
+    stats->push_epochs = fc.push_epochs;
+    stats->pull_epochs = fc.pull_epochs;
+    stats->launches = launches;
+    stats->reached = (int64_t)fc.reached;
+    stats->alg_bytes = (double)fc.alg_bytes;
+}
+
 template <typename OffT>
 static int run_bfs_loop(hc_graph_s *g, int32_t src, int32_t *depth,
                         int32_t *parents, int direction, int alpha, int beta,
                         hc_run_stats_t *stats, hipStream_t s) {
     BfsWs *ws = nullptr;
     HC_TRY(get_bfs_ws(g, &ws, s));
+    if (direction == 0 && bfs_is_small(g) && !tuning().kernel_events) {
+        HC_TRY(launch_bfs_small(g, src, depth ? depth : ws->depth, parents, alpha, beta,
+                                ws->f.ctl, s));
+        StepCtl &c = *ws->f.h_ctl;
+        HC_HIP(hipMemcpyAsync(&c, ws->f.ctl, sizeof(StepCtl), hipMemcpyDeviceToHost, s));
+        HC_HIP(hipStreamSynchronize(s));
+        fill_bfs_stats(c, 1, stats);
+        return HC_OK;
+    }
     const PlanHost *ph = nullptr;
     HC_TRY(get_plan(g, 0, g->n, tuning().bu, &ph));
     int32_t plan_rows = 0;
@@ -1153,17 +1176,8 @@ static int run_bfs_loop(hc_graph_s *g, int32_t src, int32_t *depth,
     HC_TRY(run_epoch_loop(&ws->f, s, cap, &BfsLaunch<OffT>::launch, &L, &ms,
                           &launches, &fc));
     if (!fc.done) return fail(HC_ERR_HIP, "BFS loop did not finish in %lld epochs", launches);
+    fill_bfs_stats(fc, (int32_t)(2 * launches), stats);
     if (stats) {
-        std::memset(stats, 0, sizeof(*stats));
-        // Device wall clock from the init kernel to the controller of the
-        // last epoch (launches queued past it are not part of the loop).
-        stats->ms = double(fc.t_end - fc.t_start) / device_state().clock_khz;
-        stats->epochs = fc.epoch;
-        stats->push_epochs = fc.push_epochs;
-        stats->pull_epochs = fc.pull_epochs;
-        stats->launches = (int32_t)(2 * launches);
-        stats->reached = (int64_t)fc.reached;
-        stats->alg_bytes = (double)fc.alg_bytes;
         if (ws->f.kt.on) {
             stats->kernel_launches = (int32_t)std::min<long long>(fc.steps, ws->f.kt.pairs());
             stats->kernel_ms = ws->f.kt.sum_ms(stats->kernel_launches);

@@ -675,6 +675,15 @@ __device__ void compact_body(const GraphView<OffT> &g, const FrontierBufs &fb,
     }
 }
 
+// Graphs of up to this size run a direction-optimizing BFS as one workgroup
+// (many.hip): launch_bfs_small enqueues it; ctl[0] receives the final header
+// and the trace.
+constexpr int32_t kBfsSmallNodes = 1 << 15;
+constexpr int64_t kBfsSmallEdges = int64_t(1) << 20;
+bool bfs_is_small(const hc_graph_s *g);
+int launch_bfs_small(const hc_graph_s *g, int32_t src, int32_t *depth, int32_t *parents,
+                     int alpha, int beta, StepCtl *ctl, hipStream_t s);
+
 // Host loop shared by SSSP and BFS: enqueue `launch_epoch(arg, k)` for
 // epochs k = 0, 1, ... in batches and poll the done flag of the previous
 // batch while the next one is queued.  final_ctl: the last header with the
@@ -683,7 +692,7 @@ int run_epoch_loop(FrontierWs *ws, hipStream_t s, long long cap,
                    int (*launch_epoch)(void *, long long), void *arg, float *ms,
                    long long *launches, StepCtl *final_ctl);
 
-// The newer header of the two slots at d (epoch counts differ by one) with
+// The newer header of the two slots at d (their step counts differ) with
 // the trace of slot 0.
 int read_final_ctl(const StepCtl *d, StepCtl *out, hipStream_t s);
 

@@ -22,7 +22,7 @@
 #include <vector>
 
 #include "../../include/hc_batch.h"
-#include "device_common.h"
+#include "frontier.h"
 
 struct hc_graph_batch_s {
     int32_t num_graphs = 0;
@@ -141,14 +141,20 @@ __device__ __forceinline__ void expand(const uint32_t *__restrict__ off,
 // bm holds three bitmaps of `words` words (LDS, or a global slot when
 // Global).  Frontier vertices of degree above light_deg are expanded by
 // whole wavefronts, up to heavy_cap of them per level.
-template <int BLOCK, bool Global>
+// TRACE: the levels are recorded in `trace` as the epoch loop records its
+// epochs, and its totals set (single-graph runs).
+template <int BLOCK, bool Global, bool TRACE = false>
 __device__ __forceinline__ void bfs_one_graph(const Desc &d, int32_t src,
                               const uint32_t *__restrict__ off,
                               const int32_t *__restrict__ adj, int32_t *__restrict__ depth,
                               int32_t *__restrict__ parents, uint32_t *bm, int words,
                               int alpha, int beta, int light_deg, int heavy_cap,
-                              int32_t *heavy, int *s_nheavy, long long *s_red, ManyStats &st) {
+                              int32_t *heavy, int *s_nheavy, long long *s_red, ManyStats &st,
+                              StepCtl *trace = nullptr) {
     const int tid = threadIdx.x;
+    long long t_start = 0;
+    if (TRACE) t_start = wall_clock64();
+    unsigned long long bytes = 0, reached = 1;
     const int n = d.n;
     uint32_t *vis = bm;
     uint32_t *front = bm + words;
@@ -259,6 +265,7 @@ __device__ __forceinline__ void bfs_one_graph(const Desc &d, int32_t src,
                         depth[u] = level;
                         if (parents) parents[u] = par;
                         cnt++;
+                        sc += re[k] - rb[k];
                     }
                 }
             }
@@ -267,6 +274,20 @@ __device__ __forceinline__ void bfs_one_graph(const Desc &d, int32_t src,
         const long long q = many_block_sum<BLOCK>(cnt, s_red);
         const long long scq = many_block_sum<BLOCK>(sc, s_red);
         st.scanned += (unsigned long long)scanned;
+        if (TRACE) {
+            const long long ex = many_block_sum<BLOCK>(scanned, s_red);
+            // (the epoch loop's byte counts, with 4-byte offsets)
+            bytes += pull ? 4ull * n + 4ull * ex + ex / 8 + 12ull * q + 4ull * words
+                          : 12ull * fsize + 8ull * ex + 16ull * q;
+            reached += q;
+            if (tid == 0 && level <= kTraceLen) {
+                trace->tr_t[level - 1] = wall_clock64();
+                trace->tr_mode[level - 1] = (int8_t)(pull ? kPull : kPush);
+                trace->tr_n[level - 1] = (uint32_t)q;
+                trace->tr_e[level - 1] = (unsigned long long)scq;
+                trace->tr_scan[level - 1] = (unsigned long long)ex;
+            }
+        }
         // Next level's frontier; clear the old one for reuse.
         uint32_t *t = front;
         front = next;
@@ -301,6 +322,52 @@ __device__ __forceinline__ void bfs_one_graph(const Desc &d, int32_t src,
         }
         __syncthreads();
     }
+    if (TRACE && tid == 0) {
+        trace->t_start = t_start;
+        trace->t_end = wall_clock64();
+        trace->epoch = level;
+        trace->push_epochs = (int32_t)st.pushes;
+        trace->pull_epochs = (int32_t)st.pulls;
+        trace->reached = reached;
+        trace->alg_bytes = bytes;
+        trace->done = 1;
+        trace[0].steps = 1;
+        trace[1].steps = 0;
+    }
+}
+
+// One BFS of a small graph by one workgroup in one launch: its levels take a
+// few microseconds each, where the epoch loop's two launches take a dozen
+// (Kronecker, 4096 vertices: 175 -> 84 us a query with its result fetched).
+constexpr int kSmallBlock = 1024;
+constexpr int kSmallHeavy = 1024;
+__global__ __launch_bounds__(kSmallBlock) void bfs_small_kernel(
+    const uint32_t *__restrict__ off, const int32_t *__restrict__ adj, int32_t n, int64_t m,
+    int32_t src, int32_t *__restrict__ depth, int32_t *__restrict__ parents, int alpha, int beta,
+    StepCtl *ctl) {
+    extern __shared__ uint32_t lds_bm[];
+    __shared__ int32_t heavy[kSmallHeavy];
+    __shared__ int s_nheavy;
+    __shared__ long long s_red[kSmallBlock / kWave];
+    ManyStats st{0, 0, 0};
+    const Desc d{0, 0, 0, n, 0, m};
+    bfs_one_graph<kSmallBlock, false, true>(d, src, off, adj, depth, parents, lds_bm,
+                                            (n + 31) / 32, alpha, beta, 8, kSmallHeavy, heavy,
+                                            &s_nheavy, s_red, st, ctl);
+}
+
+bool bfs_is_small(const hc_graph_s *g) {
+    return !g->off64 && g->n <= kBfsSmallNodes && g->m <= kBfsSmallEdges && g->row0 == 0 &&
+           g->rows == g->n;
+}
+
+int launch_bfs_small(const hc_graph_s *g, int32_t src, int32_t *depth, int32_t *parents,
+                     int alpha, int beta, StepCtl *ctl, hipStream_t s) {
+    const size_t lds = sizeof(uint32_t) * 3 * (size_t)((g->n + 31) / 32);
+    bfs_small_kernel<<<1, kSmallBlock, lds, s>>>(static_cast<const uint32_t *>(g->d_off), g->d_adj,
+                                                 g->n, g->m, src, depth, parents, alpha, beta, ctl);
+    HC_HIP(hipGetLastError());
+    return HC_OK;
 }
 
 template <int BLOCK>

@@ -58,3 +58,25 @@ def test_flat_rows_read_ahead(hc, gpu, oracle, monkeypatch, degree, wide):
     dst = rng.integers(0, n - 1000, degree * n).astype(np.int32)
     g = hc.HostGraph.from_edges(src, dst, n)
     _check(hc, oracle, g, [int(src[0])], directions=(0, 1))
+
+
+@pytest.mark.parametrize("n", [1, 2, 31, 32, 33, 1023, 1025, 8193, 32767, 32768, 32769])
+def test_small_graphs_around_the_one_workgroup_limit(hc, gpu, oracle, n):
+    """Graphs of up to 2^15 vertices run as one workgroup: its levels, trace and
+    totals are those of the epoch loop."""
+    rng = np.random.default_rng(n)
+    src = rng.integers(0, n, 6 * n).astype(np.int32)
+    dst = rng.integers(0, n, 6 * n).astype(np.int32)
+    hub = np.zeros(min(n, 3000), np.int32)
+    g = hc.HostGraph.from_edges(np.concatenate([src, hub]),
+                                np.concatenate([dst, rng.permutation(n)[:hub.size].astype(np.int32)]),
+                                n)
+    _check(hc, oracle, g, [0, n // 2, n - 1])
+    with hc.DeviceGraph(g) as dg:
+        one = hc.bfs(dg, n // 2)
+        hc.set_tuning("profile.kernel_events", 1)  # the epoch loop
+        loop = hc.bfs(dg, n // 2)
+        hc.reset_tuning()
+        assert np.array_equal(one.values, loop.values)
+        for key in ("epochs", "push_epochs", "pull_epochs", "reached"):
+            assert one.stats[key] == loop.stats[key], key
