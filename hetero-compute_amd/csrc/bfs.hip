@@ -1135,7 +1135,7 @@ static int run_bfs_loop(hc_graph_s *g, int32_t src, int32_t *depth,
     if (direction == 0 && bfs_is_small(g) && !tuning().kernel_events) {
         HC_TRY(launch_bfs_small(g, src, depth ? depth : ws->depth, parents, alpha, beta,
                                 ws->f.ctl, s));
-        StepCtl &c = *ws->f.h_ctl;
+        StepCtl &c = ws->f.h_ctl[1];
         HC_HIP(hipMemcpyAsync(&c, ws->f.ctl, sizeof(StepCtl), hipMemcpyDeviceToHost, s));
         HC_HIP(hipStreamSynchronize(s));
         fill_bfs_stats(c, 1, stats);
@@ -1170,11 +1170,9 @@ static int run_bfs_loop(hc_graph_s *g, int32_t src, int32_t *depth,
                       head4, ws->f.fb, ws->f.ctl, rl, grid, s, nstage, tuning().bu_stage_min,
                       lds_words, push_cap, tuning().bu_first == 2, &ws->f.kt};
     const long long cap = (long long)g->n + 2;  // levels <= n
-    float ms = 0;
     long long launches = 0;
     StepCtl fc;
-    HC_TRY(run_epoch_loop(&ws->f, s, cap, &BfsLaunch<OffT>::launch, &L, &ms,
-                          &launches, &fc));
+    HC_TRY(run_epoch_loop(&ws->f, s, cap, &BfsLaunch<OffT>::launch, &L, &launches, &fc));
     if (!fc.done) return fail(HC_ERR_HIP, "BFS loop did not finish in %lld epochs", launches);
     fill_bfs_stats(fc, (int32_t)(2 * launches), stats);
     if (stats) {

@@ -159,7 +159,7 @@ __device__ __forceinline__ void publish_done(const FrontierBufs &fb) {
 struct FrontierWs {
     FrontierBufs fb{};
     StepCtl *ctl = nullptr;
-    StepCtl *h_ctl = nullptr;  // pinned mirror for polling
+    StepCtl *h_ctl = nullptr;  // pinned: [0] its done word is polled, [1], [2] final headers
     void *dmem = nullptr;
     int64_t chunk_cap = 0;
     int32_t grid = 0;
@@ -689,8 +689,8 @@ int launch_bfs_small(const hc_graph_s *g, int32_t src, int32_t *depth, int32_t *
 // batch while the next one is queued.  final_ctl: the last header with the
 // trace of slot 0.
 int run_epoch_loop(FrontierWs *ws, hipStream_t s, long long cap,
-                   int (*launch_epoch)(void *, long long), void *arg, float *ms,
-                   long long *launches, StepCtl *final_ctl);
+                   int (*launch_epoch)(void *, long long), void *arg, long long *launches,
+                   StepCtl *final_ctl);
 
 // The newer header of the two slots at d (their step counts differ) with
 // the trace of slot 0.

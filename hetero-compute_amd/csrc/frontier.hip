@@ -54,7 +54,7 @@ int frontier_ws_alloc(hc_graph_s *g, FrontierWs *ws) {
     ws->dmem = base;
     ws->chunk_cap = cap;
     ws->grid = grid;
-    if (hipHostMalloc(reinterpret_cast<void **>(&ws->h_ctl), sizeof(StepCtl),
+    if (hipHostMalloc(reinterpret_cast<void **>(&ws->h_ctl), 3 * sizeof(StepCtl),
                       hipHostMallocDefault) != hipSuccess) {
         hipFree(base);
         ws->dmem = nullptr;
@@ -106,22 +106,25 @@ void frontier_ws_free(FrontierWs *ws) {
     ws->h_ctl = nullptr;
 }
 
+// The newer header of h[0] and h[1] with the trace of h[0].
+static void newer_ctl(const StepCtl *h, StepCtl *out) {
+    *out = h[0];
+    if (h[1].steps > h[0].steps)
+        std::memcpy(out, &h[1], sizeof(unsigned long long) * kCtlHeadWords);
+}
+
 int read_final_ctl(const StepCtl *d, StepCtl *out, hipStream_t s) {
     StepCtl h[2];
     HC_HIP(hipMemcpyAsync(h, d, 2 * sizeof(StepCtl), hipMemcpyDeviceToHost, s));
     HC_HIP(hipStreamSynchronize(s));
-    *out = h[0];
-    if (h[1].steps > h[0].steps)
-        std::memcpy(out, &h[1], sizeof(unsigned long long) * kCtlHeadWords);
+    newer_ctl(h, out);
     return HC_OK;
 }
 
 int run_epoch_loop(FrontierWs *ws, hipStream_t s, long long cap,
-                   int (*launch_epoch)(void *, long long), void *arg, float *ms,
-                   long long *launches, StepCtl *final_ctl) {
-    hipEvent_t ev0, ev1, evb[2];
-    HC_HIP(hipEventCreate(&ev0));
-    HC_HIP(hipEventCreate(&ev1));
+                   int (*launch_epoch)(void *, long long), void *arg, long long *launches,
+                   StepCtl *final_ctl) {
+    hipEvent_t evb[2];
     // The batch events only pace the host: no system-scope fence (an L2
     // writeback per batch); the done word is a system-scope store of its own.
     const unsigned pace = hipEventDisableTiming | hipEventDisableSystemFence;
@@ -129,7 +132,6 @@ int run_epoch_loop(FrontierWs *ws, hipStream_t s, long long cap,
     HC_HIP(hipEventCreateWithFlags(&evb[1], pace));
     StepCtl *h = ws->h_ctl;
     h->done = 0;
-    HC_HIP(hipEventRecord(ev0, s));
     // Batches of two epochs: the host reads the done flag after batch b-1 has
     // finished while batch b is queued, so at most ~4 epochs are enqueued past
     // the last one (they return at once) and the device never waits on a poll.
@@ -153,12 +155,16 @@ int run_epoch_loop(FrontierWs *ws, hipStream_t s, long long cap,
         }
         b++;
     }
-    HC_HIP(hipEventRecord(ev1, s));
-    HC_HIP(hipEventSynchronize(ev1));
-    HC_HIP(hipEventElapsedTime(ms, ev0, ev1));
-    rc = rc != HC_OK ? rc : read_final_ctl(ws->ctl, final_ctl, s);
-    hipEventDestroy(ev0);
-    hipEventDestroy(ev1);
+    // One wait for the launches queued past the end and the final headers,
+    // copied to pinned memory (through pageable memory the copy alone took 24
+    // us, and an event before it another 9).
+    if (rc == HC_OK &&
+        (hipMemcpyAsync(ws->h_ctl + 1, ws->ctl, 2 * sizeof(StepCtl), hipMemcpyDeviceToHost, s) !=
+             hipSuccess ||
+         hipStreamSynchronize(s) != hipSuccess))
+        rc = fail(HC_ERR_HIP, "reading the control block failed");
+    if (rc == HC_OK) newer_ctl(ws->h_ctl + 1, final_ctl);
+    else (void)hipStreamSynchronize(s);
     hipEventDestroy(evb[0]);
     hipEventDestroy(evb[1]);
     *launches = epochs;

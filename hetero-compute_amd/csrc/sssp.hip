@@ -1554,11 +1554,9 @@ static int run_sssp_loop(hc_graph_s *g, int32_t src, const int32_t *init_dist,
     // re-pushes: a generous bound); the cap bounds a faulty loop.
     const long long bound = delta > 0 ? 64LL * (g->n + 1) + 4096 : (long long)g->n;
     const long long cap = (max_epochs > 0 ? std::min<long long>(max_epochs, bound) : bound) + 2;
-    float ms = 0;
     long long launches = 0;
     StepCtl fc;
-    HC_TRY(run_epoch_loop(&ws->f, s, cap, &SsspLaunch<OffT>::launch, &L, &ms,
-                          &launches, &fc));
+    HC_TRY(run_epoch_loop(&ws->f, s, cap, &SsspLaunch<OffT>::launch, &L, &launches, &fc));
     if (!fc.done && max_epochs <= 0)
         return fail(HC_ERR_HIP, "SSSP loop did not converge in %lld epochs", launches);
     if (stats) {
