@@ -338,6 +338,11 @@ __device__ __forceinline__ T ldnt(const T *p) {
     return __builtin_nontemporal_load(p);
 }
 
+template <typename T>
+__device__ __forceinline__ void stnt(T *p, T v) {
+    __builtin_nontemporal_store(v, p);
+}
+
 __device__ __forceinline__ uint64_t lanemask_lt() {
     return (uint64_t(1) << lane_id()) - 1;
 }
@@ -482,6 +487,7 @@ struct DeviceState {
     int cus = 0;
     double clock_khz = 100000.0;  // device wall clock rate
     size_t hbm = 0;
+    size_t max_lds = 64 * 1024;  // largest LDS of a workgroup
     hipStream_t stream = nullptr;  // library default stream
     bool ready = false;
 };

@@ -126,8 +126,6 @@ struct PrBufs {
     const double *inv_deg;
     float *hub_hi;         // per chunk partials
     float *hub_lo;
-    uint32_t *hub_cnt;     // per hub: chunks finished this epoch
-    double *hub_resid;     // per hub: |score' - score|
     double *partials;      // per workgroup residual partial
 };
 
@@ -157,91 +155,130 @@ struct PrEpoch {
 // Rule 0 returns |score' - score| (FP64); rule 1 keeps the old score unless
 // the new one moves it by more than 5e-8 (epoch_pr_pull_cpu_one_to_one,
 // src/kernels/cpu/pr.cuh:170-181) and returns 1 when it moved.
-__device__ __forceinline__ double pr_finalize(const PrEpoch &ep, const double *inv_deg,
-                                              int32_t u, KSum k) {
+__device__ __forceinline__ double pr_finalize(const PrEpoch &ep, int32_t u, KSum k, float s_old,
+                                              double inv_deg) {
     float sum = k.hi + k.lo;
     float s_new = __fadd_rn(ep.base, __fmul_rn(ep.damp, sum));
-    const float s_old = ep.s_in[u];
     if (ep.rule) {
         const bool moved = fabsf(__fsub_rn(s_new, s_old)) > 0.00000005f;
         const float s = moved ? s_new : s_old;
-        ep.s_out[u] = s;
-        ep.c_out[u] = (float)((double)s * inv_deg[u]);
+        stnt(&ep.s_out[u], s);
+        ep.c_out[u] = (float)((double)s * inv_deg);
         return moved ? 1.0 : 0.0;
     }
-    ep.s_out[u] = s_new;
-    ep.c_out[u] = (float)((double)s_new * inv_deg[u]);
+    stnt(&ep.s_out[u], s_new);
+    ep.c_out[u] = (float)((double)s_new * inv_deg);
     return fabs((double)s_new - (double)s_old);
 }
 
+__device__ __forceinline__ double pr_finalize(const PrEpoch &ep, const double *inv_deg,
+                                              int32_t u, KSum k) {
+    return pr_finalize(ep, u, k, ep.s_in[u], inv_deg[u]);
+}
+
+constexpr int64_t kPrHubMin = 2048;  // edges a row has at least to be cut into chunks
+// A sweep runs in workgroups of 16 wavefronts, one per CU where the LDS copy
+// of the hubs' contributions takes most of its LDS; each wavefront takes rows
+// and chunks by itself.
+//
+// The gathers bound it: those that reach L2 come at 262 G/s at most, those
+// that miss it at 65 G/s (a line each), while the ids stream in at
+// about 1000 G/s.
+// So LDS takes as many as it can.  Kronecker, 16M vertices, 512M edges, 7
+// sweeps: 22.4 ms with none staged, 19.4 with 20K entries, 18.0 with 39K (and
+// 19.4 before, in four 256-thread workgroups per CU with 8K entries each).
+// 262144 vertices, 8M edges: 450 us with none, 380 with 39K.
+constexpr int kPrBlock = 1024;
+constexpr int kPrWaves = kPrBlock / kWave;
+
+// The rows of class c, kWave / G of them per wavefront and unit; unit k0 and
+// every `waves`-th after it.  The next unit's rows and offsets are read before
+// this unit's edges, and the old scores and degrees beside them, so that a unit
+// waits for its ids and its gathers only.
 template <int G, typename OffT>
-__device__ __forceinline__ void pr_group(const PlanDev &p, int c, int k,
-                                         const GraphView<OffT> &g,
-                                         const Staged<float> &cr,
-                                         const PrEpoch &ep, const PrBufs &b,
-                                         double &racc) {
-    constexpr int PER = kBlock / G;
-    const int gid = threadIdx.x / G, lane = threadIdx.x % G;
-    const int idx = k * PER + gid;
-    if (idx < p.cnt[c]) {
-        int32_t u = p.list[c] ? p.list[c][idx] : p.beg[c] + idx;
-        KSum s = row_ksum<G>(g, cr, g.rbeg(u), g.rend(u), lane);
+__device__ __forceinline__ void pr_rows(const PlanDev &p, int c, int &start, int wave, int waves,
+                                        const GraphView<OffT> &g, const Staged<float> &cr,
+                                        const PrEpoch &ep, const PrBufs &b, double &racc) {
+    constexpr int R = kWave / G;
+    const int cnt = p.cnt[c], units = (cnt + R - 1) / R;
+    const int32_t *list = p.list[c];
+    const int32_t beg = p.beg[c];
+    int k = wave - start % waves;
+    if (k < 0) k += waves;
+    start += units;
+    const int lane = lane_id() % G, row = lane_id() / G;
+    int32_t u = -1;
+    OffT rb = 0, re = 0;
+    if (k < units && k * R + row < cnt) {
+        u = list ? list[k * R + row] : beg + k * R + row;
+        rb = g.rbeg(u);
+        re = g.rend(u);
+    }
+    for (; k < units; k += waves) {
+        int32_t nu = -1;
+        OffT nb = 0, ne = 0;
+        const int nk = k + waves;
+        if (nk < units && nk * R + row < cnt) {
+            nu = list ? list[nk * R + row] : beg + nk * R + row;
+            nb = g.rbeg(nu);
+            ne = g.rend(nu);
+        }
+        float s_old = 0.0f;
+        double inv = 0.0;
+        if (lane == 0 && u >= 0) {
+            s_old = ldnt(&ep.s_in[u]);
+            inv = ldnt(&b.inv_deg[u]);
+        }
+        KSum s = row_ksum<G>(g, cr, rb, re, lane);
         if (G > 1) s = group_ksum<G>(s);
-        if (lane == 0) racc += pr_finalize(ep, b.inv_deg, u, s);
+        if (lane == 0 && u >= 0) racc += pr_finalize(ep, u, s, s_old, inv);
+        u = nu;
+        rb = nb;
+        re = ne;
     }
 }
 
-// One Jacobi sweep over the plan units and the zero-degree vertices.
+// One Jacobi sweep over the plan's rows and the zero-degree vertices.
 // Returns this thread's residual contribution (hub residuals go to
-// b.hub_resid instead, so the total does not depend on which workgroup
-// finishes a hub).
+// b.hub_resid instead).
 // contrib is read-only within a sweep, so the LDS snapshot of its hub entries
 // (staged from ep.c_in) is exact.
 template <typename OffT>
-__device__ double pr_sweep(const PlanDev &p, const GraphView<OffT> &g,
-                           const PrEpoch &ep, const PrBufs &b, int32_t nstage,
-                           float *lds) {
-    const Staged<float> cr = stage(ep.c_in, nstage, lds);
+__device__ __forceinline__ double pr_sweep(const PlanDev &p, const GraphView<OffT> &g,
+                                           const PrEpoch &ep, const PrBufs &b, int32_t nstage,
+                                           float *lds) {
+#pragma unroll 8
+    for (int i = threadIdx.x; i < nstage; i += kPrBlock) lds[i] = ep.c_in[i];
+    __syncthreads();
+    const Staged<float> cr{ep.c_in, lds, nstage};
+    const int wave = blockIdx.x * kPrWaves + threadIdx.x / kWave;
+    const int waves = gridDim.x * kPrWaves;
+    for (int k = wave; k < p.cnt[0]; k += waves) {
+        const HubChunk h = p.chunks[k];
+        const KSum s = group_ksum<kWave>(row_ksum<kWave>(g, cr, OffT(h.b), OffT(h.e), lane_id()));
+        // Chunk partials are combined by the controller kernel.
+        if (lane_id() == 0) {
+            b.hub_hi[k] = s.hi;
+            b.hub_lo[k] = s.lo;
+        }
+    }
     double racc = 0.0;
-    const int gstride = gridDim.x * blockDim.x;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < p.zero_cnt; i += gstride) {
+    int start = p.cnt[0];
+    pr_rows<64>(p, 1, start, wave, waves, g, cr, ep, b, racc);
+    pr_rows<64>(p, 2, start, wave, waves, g, cr, ep, b, racc);
+    pr_rows<16>(p, 3, start, wave, waves, g, cr, ep, b, racc);
+    pr_rows<4>(p, 4, start, wave, waves, g, cr, ep, b, racc);
+    pr_rows<1>(p, 5, start, wave, waves, g, cr, ep, b, racc);
+    const int gstride = gridDim.x * kPrBlock;
+    for (int i = blockIdx.x * kPrBlock + threadIdx.x; i < p.zero_cnt; i += gstride) {
         int32_t u = p.zero_list ? p.zero_list[i] : p.zero_beg + i;
         racc += pr_finalize(ep, b.inv_deg, u, KSum{0.0f, 0.0f});
-    }
-    const int total = p.unit_start[kNumClasses];
-    for (int unit = blockIdx.x; unit < total; unit += gridDim.x) {
-        int c = 0;
-        while (unit >= p.unit_start[c + 1]) c++;
-        const int k = unit - p.unit_start[c];
-        if (c == 0) {
-            HubChunk h = p.chunks[k];
-            KSum s = block_ksum(row_ksum<kBlock>(g, cr, OffT(h.b), OffT(h.e),
-                                                 threadIdx.x));
-            // Chunk partials are combined by the controller kernel.
-            if (threadIdx.x == 0) {
-                b.hub_hi[k] = s.hi;
-                b.hub_lo[k] = s.lo;
-            }
-        } else if (c == 1) {
-            int32_t u = p.list[1] ? p.list[1][k] : p.beg[1] + k;
-            KSum s = block_ksum(row_ksum<kBlock>(g, cr, g.rbeg(u), g.rend(u),
-                                                 threadIdx.x));
-            if (threadIdx.x == 0) racc += pr_finalize(ep, b.inv_deg, u, s);
-        } else if (c == 2) {
-            pr_group<64>(p, c, k, g, cr, ep, b, racc);
-        } else if (c == 3) {
-            pr_group<16>(p, c, k, g, cr, ep, b, racc);
-        } else if (c == 4) {
-            pr_group<4>(p, c, k, g, cr, ep, b, racc);
-        } else {
-            pr_group<1>(p, c, k, g, cr, ep, b, racc);
-        }
     }
     return racc;
 }
 
 template <typename OffT>
-__global__ __launch_bounds__(kBlock) void pr_step_kernel(
+__global__ __launch_bounds__(kPrBlock) void pr_step_kernel(
     PlanDev p, GraphView<OffT> g, float *s0, float *s1, float *c0, float *c1,
     PrBufs b, PrCtl *ctl, float base, float damp, int32_t nstage) {
     extern __shared__ float s_stagef[];
@@ -253,38 +290,40 @@ __global__ __launch_bounds__(kBlock) void pr_step_kernel(
     if (threadIdx.x == 0) b.partials[blockIdx.x] = r;
 }
 
-// Hub vertices: combine their chunk partials in chunk order and finish
-// them; then the fixed-order residual total (workgroup partials, then hub
-// residuals).  One workgroup of kBlock threads; returns the total in every
-// thread.
+// Hub vertices: four lanes add up a hub's chunk partials, each every fourth
+// of them in chunk order, and their sums are combined in lane order; then the
+// fixed-order residual total (workgroup partials, then hub residuals).  One
+// workgroup of kPrBlock threads; returns the total in every thread.
 __device__ double pr_hubs_and_residual(const PlanDev &p, const PrEpoch &ep,
                                        const PrBufs &b, int nparts) {
-    for (int h = threadIdx.x; h < p.num_hubs; h += kBlock) {
-        const int32_t c0 = p.hub_chunk_start[h], c1 = p.hub_chunk_start[h + 1];
-        KSum tot{0.0f, 0.0f};
-        for (int32_t j = c0; j < c1; j++) tot = two_sum_combine(tot, KSum{b.hub_hi[j], b.hub_lo[j]});
-        b.hub_resid[h] = pr_finalize(ep, b.inv_deg, p.chunks[c0].u, tot);
-    }
-    __syncthreads();
-    __shared__ double s_tot[kBlock];
+    constexpr int G = 4;
     double t = 0.0;
-    for (int i = threadIdx.x; i < nparts; i += kBlock) t += b.partials[i];
-    for (int i = threadIdx.x; i < p.num_hubs; i += kBlock) t += b.hub_resid[i];
+    for (int i = threadIdx.x; i < nparts; i += kPrBlock) t += b.partials[i];
+    const int lane = threadIdx.x % G;
+    for (int h = threadIdx.x / G; h - int(threadIdx.x / G) < p.num_hubs; h += kPrBlock / G) {
+        const bool has = h < p.num_hubs;
+        const int32_t c0 = has ? p.hub_chunk_start[h] : 0;
+        const int32_t c1 = has ? p.hub_chunk_start[h + 1] : 0;
+        KSum tot{0.0f, 0.0f};
+        for (int32_t j = c0 + lane; j < c1; j += G)
+            tot = two_sum_combine(tot, KSum{b.hub_hi[j], b.hub_lo[j]});
+        tot = group_ksum<G>(tot);
+        if (has && lane == 0) t += pr_finalize(ep, b.inv_deg, p.chunks[c0].u, tot);
+    }
+    __shared__ double s_tot[kPrBlock];
     s_tot[threadIdx.x] = t;
     __syncthreads();
-    for (int s = kBlock / 2; s > 0; s >>= 1) {
+    for (int s = kPrBlock / 2; s > 0; s >>= 1) {
         if ((int)threadIdx.x < s) s_tot[threadIdx.x] += s_tot[threadIdx.x + s];
         __syncthreads();
     }
-    double r = s_tot[0];
-    __syncthreads();
-    return r;
+    return s_tot[0];
 }
 
 // Controller of the iteration loop (one workgroup).
-__global__ __launch_bounds__(kBlock) void pr_ctl_kernel(
+__global__ __launch_bounds__(kPrBlock) void pr_ctl_kernel(
     PlanDev p, float *s0, float *s1, float *c0, float *c1, PrBufs b, PrCtl *ctl,
-    float base, float damp, int nparts) {
+    float base, float damp, int nparts, int32_t *host_done) {
     if (ctl->done) return;
     const int it = ctl->iter;
     const bool odd = it & 1;
@@ -297,14 +336,26 @@ __global__ __launch_bounds__(kBlock) void pr_ctl_kernel(
         ctl->iter = it + 1;
         ctl->alg_bytes += ctl->epoch_bytes;
         ctl->t_end = wall_clock64();
-        if (converged || it + 1 >= ctl->max_iters) ctl->done = 1;
+        if (converged || it + 1 >= ctl->max_iters) {
+            ctl->done = 1;
+            __hip_atomic_store(host_done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
+}
+
+// The scores of the last iteration, to the caller.
+__global__ __launch_bounds__(kBlock) void pr_result_kernel(const PrCtl *ctl, const float *s0,
+                                                           const float *s1, float *scores,
+                                                           int32_t n) {
+    const float *s = (ctl->iter & 1) ? s1 : s0;
+    const int stride = gridDim.x * kBlock;
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) scores[i] = s[i];
 }
 
 template <typename OffT>
 __global__ __launch_bounds__(kBlock) void pr_init_kernel(
-    GraphView<OffT> g, float *s0, float *c0, double *inv_deg, uint32_t *hub_cnt,
-    int32_t num_hubs, PrCtl *ctl, int max_iters, double tol, double epoch_bytes, int rule) {
+    GraphView<OffT> g, float *s0, float *c0, double *inv_deg, PrCtl *ctl, int max_iters,
+    double tol, double epoch_bytes, int rule) {
     const int stride = gridDim.x * kBlock;
     const float init = 1.0f / (float)g.n;
     for (int u = blockIdx.x * kBlock + threadIdx.x; u < g.n; u += stride) {
@@ -314,7 +365,6 @@ __global__ __launch_bounds__(kBlock) void pr_init_kernel(
         s0[u] = init;
         c0[u] = (float)((double)init * inv);
     }
-    for (int h = blockIdx.x * kBlock + threadIdx.x; h < num_hubs; h += stride) hub_cnt[h] = 0;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         ctl->done = max_iters <= 0 ? 1 : 0;
         ctl->t_start = wall_clock64();
@@ -332,7 +382,7 @@ __global__ __launch_bounds__(kBlock) void pr_init_kernel(
 // Epoch API: one sweep over a plan; its finish kernel completes the hubs and
 // adds the fixed-order residual to *residual_out.
 template <typename OffT>
-__global__ __launch_bounds__(kBlock) void pr_epoch_kernel(PlanDev p, GraphView<OffT> g,
+__global__ __launch_bounds__(kPrBlock) void pr_epoch_kernel(PlanDev p, GraphView<OffT> g,
                                                           PrEpoch ep, PrBufs b,
                                                           int32_t nstage) {
     extern __shared__ float s_stagef[];
@@ -340,7 +390,7 @@ __global__ __launch_bounds__(kBlock) void pr_epoch_kernel(PlanDev p, GraphView<O
     if (threadIdx.x == 0) b.partials[blockIdx.x] = r;
 }
 
-__global__ __launch_bounds__(kBlock) void pr_epoch_finish_kernel(PlanDev p, PrEpoch ep,
+__global__ __launch_bounds__(kPrBlock) void pr_epoch_finish_kernel(PlanDev p, PrEpoch ep,
                                                                  PrBufs b, int nparts,
                                                                  double *residual_out) {
     const double r = pr_hubs_and_residual(p, ep, b, nparts);
@@ -437,11 +487,11 @@ struct PrWs {
     float *c[2] = {nullptr, nullptr};
     double *inv_deg = nullptr;
     float *hub_hi = nullptr, *hub_lo = nullptr;
-    uint32_t *hub_cnt = nullptr;
-    double *hub_resid = nullptr;
     double *partials = nullptr;
     PrCtl *ctl = nullptr;
-    int32_t chunk_cap = 0, hub_cap = 0, part_cap = 0;
+    PrCtl *h_ctl = nullptr;        // pinned: [0] its done word is polled, [1] the final state
+    int32_t *host_done = nullptr;  // h_ctl[0].done as the device sees it
+    int32_t chunk_cap = 0, part_cap = 0;
     void *dmem = nullptr;
 };
 
@@ -449,14 +499,15 @@ void free_pr_ws(hc_graph_s *g) {
     if (!g->ws_pr) return;
     auto *ws = static_cast<PrWs *>(g->ws_pr);
     if (ws->dmem) hipFree(ws->dmem);
+    if (ws->h_ctl) hipHostFree(ws->h_ctl);
     delete ws;
     g->ws_pr = nullptr;
 }
 
-static int get_pr_ws(hc_graph_s *g, int32_t chunks, int32_t hubs, PrWs **out) {
+static int get_pr_ws(hc_graph_s *g, int32_t chunks, PrWs **out) {
     auto *ws = static_cast<PrWs *>(g->ws_pr);
     const int32_t parts = grid_blocks();
-    if (ws && ws->chunk_cap >= chunks && ws->hub_cap >= hubs && ws->part_cap >= parts) {
+    if (ws && ws->chunk_cap >= chunks && ws->part_cap >= parts) {
         *out = ws;
         return HC_OK;
     }
@@ -466,13 +517,21 @@ static int get_pr_ws(hc_graph_s *g, int32_t chunks, int32_t hubs, PrWs **out) {
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
     size_t sz_f = al(sizeof(float) * n), sz_d = al(sizeof(double) * n);
     size_t sz_ch = al(sizeof(float) * std::max(chunks, 1));
-    size_t sz_h = al(sizeof(double) * std::max(hubs, 1));
     size_t sz_p = al(sizeof(double) * parts);
-    size_t total = 4 * sz_f + sz_d + 2 * sz_ch + 2 * sz_h + sz_p + al(sizeof(PrCtl));
+    size_t total = 4 * sz_f + sz_d + 2 * sz_ch + sz_p + al(sizeof(PrCtl));
     char *base = nullptr;
     if (hipMalloc(reinterpret_cast<void **>(&base), total) != hipSuccess) {
         delete ws;
         return fail(HC_ERR_OOM, "PageRank workspace of %zu bytes failed", total);
+    }
+    if (hipHostMalloc(reinterpret_cast<void **>(&ws->h_ctl), 2 * sizeof(PrCtl),
+                      hipHostMallocDefault) != hipSuccess ||
+        hipHostGetDevicePointer(reinterpret_cast<void **>(&ws->host_done), &ws->h_ctl->done, 0) !=
+            hipSuccess) {
+        hipFree(base);
+        if (ws->h_ctl) hipHostFree(ws->h_ctl);
+        delete ws;
+        return fail(HC_ERR_OOM, "pinned PageRank control block failed");
     }
     size_t o = 0;
     for (int i = 0; i < 2; i++) {
@@ -487,20 +546,56 @@ static int get_pr_ws(hc_graph_s *g, int32_t chunks, int32_t hubs, PrWs **out) {
     o += sz_ch;
     ws->hub_lo = reinterpret_cast<float *>(base + o);
     o += sz_ch;
-    ws->hub_cnt = reinterpret_cast<uint32_t *>(base + o);
-    o += sz_h;
-    ws->hub_resid = reinterpret_cast<double *>(base + o);
-    o += sz_h;
     ws->partials = reinterpret_cast<double *>(base + o);
     o += sz_p;
     ws->ctl = reinterpret_cast<PrCtl *>(base + o);
     ws->dmem = base;
     ws->chunk_cap = std::max(chunks, 1);
-    ws->hub_cap = std::max(hubs, 1);
     ws->part_cap = parts;
     g->ws_pr = ws;
     *out = ws;
     return HC_OK;
+}
+
+// Degree classes of a sweep: a wavefront takes a row or a chunk by itself, so
+// a row is cut into chunks once it would keep its wavefront longer than an
+// even share of all edges would, but not below kPrHubMin edges (8 trips),
+// since the one workgroup that adds up the chunks takes longer with each hub
+// (21 us a sweep with 2.3K of them).
+static PlanConfig pr_plan_config(const hc_graph_s *g) {
+    PlanConfig c = tuning().pull;
+    const int64_t share = g->m / (int64_t(kPrWaves) * device_state().cus);
+    const int64_t cut = std::max<int64_t>(share, kPrHubMin);
+    if (c.hub_threshold > cut) c.hub_threshold = cut;
+    if (c.block_threshold > c.hub_threshold) c.block_threshold = c.hub_threshold;
+    if (c.wave_threshold > c.block_threshold) c.wave_threshold = c.block_threshold;
+    if (c.g16_threshold > c.wave_threshold) c.g16_threshold = c.wave_threshold;
+    if (c.g4_threshold > c.g16_threshold) c.g4_threshold = c.g16_threshold;
+    c.hub_chunk = std::min<int64_t>(c.hub_chunk, std::max<int64_t>(c.hub_threshold, kPrHubMin));
+    return c;
+}
+
+// Launch shape of a sweep over [start, end): workgroups, and contributions
+// staged in LDS.
+struct PrShape {
+    int grid;
+    int32_t nstage;
+};
+
+static PrShape pr_shape(const hc_graph_s *g, int32_t start, int32_t end, const void *kernel) {
+    const DeviceState &d = device_state();
+    // Five times the entries of a 256-thread pull workgroup for one four times
+    // as wide: by default as many as fit.
+    int64_t ns = std::min<int64_t>(5ll * tuning().stage_pull, g->n);
+    ns = std::min<int64_t>(ns, ((int64_t)d.max_lds - 4096) / (int64_t)sizeof(float));
+    // Gathers a workgroup saves: its share of the range's edges, times the
+    // share of all edges that the first ns vertices have (on a graph of which
+    // only some rows are held, a quarter).  Copying an entry takes about a
+    // quarter of a gather's time.
+    const double edges = double(g->h_off[end - g->row0] - g->h_off[start - g->row0]) / d.cus;
+    const double part = g->rows < g->n ? 0.25 : g->m > 0 ? double(g->h_off[ns]) / g->m : 0.0;
+    if (edges * part < 0.25 * ns) ns = 0;
+    return {resident_grid(kernel, kPrBlock, ns * sizeof(float), grid_blocks()), (int32_t)ns};
 }
 
 static long long pr_epoch_bytes(const hc_graph_s *g, const PlanHost *ph) {
@@ -517,53 +612,65 @@ template <typename OffT>
 static int run_pr(hc_graph_s *g, float *scores, float damp, double tol,
                   int max_iters, int rule, hc_run_stats_t *stats, hipStream_t s) {
     const PlanHost *ph = nullptr;
-    HC_TRY(get_plan(g, 0, g->n, tuning().pull, &ph));
+    HC_TRY(get_plan(g, 0, g->n, pr_plan_config(g), &ph));
     PrWs *ws = nullptr;
-    HC_TRY(get_pr_ws(g, ph->dev.cnt[0], ph->dev.num_hubs, &ws));
+    HC_TRY(get_pr_ws(g, ph->dev.cnt[0], &ws));
     GraphView<OffT> v = view<OffT>(g);
-    const int32_t ns = std::min<int32_t>(tuning().stage_pull, g->n);
-    const int grid = resident_grid(reinterpret_cast<const void *>(&pr_step_kernel<OffT>), kBlock,
-                                   ns * sizeof(float), grid_blocks());
-    const int init_grid = std::max(1, std::min(grid, (g->n + kBlock - 1) / kBlock));
+    const PrShape sh = pr_shape(g, 0, g->n, reinterpret_cast<const void *>(&pr_step_kernel<OffT>));
+    const int grid = sh.grid;
+    const int32_t ns = sh.nstage;
+    const int init_grid = std::max(1, std::min(grid_blocks(), (g->n + kBlock - 1) / kBlock));
     const float base = (1.0f - damp) / (float)g->n;
     pr_init_kernel<OffT><<<init_grid, kBlock, 0, s>>>(
-        v, ws->s[0], ws->c[0], ws->inv_deg, ws->hub_cnt, ph->dev.num_hubs, ws->ctl,
-        max_iters, tol, (double)pr_epoch_bytes(g, ph), rule);
+        v, ws->s[0], ws->c[0], ws->inv_deg, ws->ctl, max_iters, tol, (double)pr_epoch_bytes(g, ph), rule);
     HC_HIP(hipGetLastError());
-    PrBufs b{ws->inv_deg, ws->hub_hi, ws->hub_lo, ws->hub_cnt, ws->hub_resid, ws->partials};
-    hipEvent_t e0, e1;
-    HC_HIP(hipEventCreate(&e0));
-    HC_HIP(hipEventCreate(&e1));
-    HC_HIP(hipEventRecord(e0, s));
+    PrBufs b{ws->inv_deg, ws->hub_hi, ws->hub_lo, ws->partials};
     ws->kt.reset();
-    for (int i = 0; i < max_iters; i++) {
-        timed_launch(&ws->kt, pr_step_kernel<OffT>, dim3(grid), dim3(kBlock),
-                     uint32_t(ns * sizeof(float)), s, ph->dev, v, ws->s[0], ws->s[1], ws->c[0],
-                     ws->c[1], b, ws->ctl, base, damp, ns);
-        pr_ctl_kernel<<<1, kBlock, 0, s>>>(ph->dev, ws->s[0], ws->s[1], ws->c[0],
-                                           ws->c[1], b, ws->ctl, base, damp, grid);
+    // Batches of two iterations: the host reads the done word after batch b-1
+    // has finished while batch b is queued.  With all max_iters queued at once
+    // the launches past the last iteration took 60 us of a run that stopped
+    // after 7 of 20.
+    PrCtl *h = ws->h_ctl;
+    h->done = 0;
+    hipEvent_t ev[2];
+    const unsigned pace = hipEventDisableTiming | hipEventDisableSystemFence;
+    HC_HIP(hipEventCreateWithFlags(&ev[0], pace));
+    HC_HIP(hipEventCreateWithFlags(&ev[1], pace));
+    int launched = 0;
+    hipError_t err = hipSuccess;
+    for (int batch = 0; launched < max_iters && err == hipSuccess; batch++) {
+        for (int i = 0; i < 2 && launched < max_iters; i++, launched++) {
+            timed_launch(&ws->kt, pr_step_kernel<OffT>, dim3(grid), dim3(kPrBlock),
+                         uint32_t(ns * sizeof(float)), s, ph->dev, v, ws->s[0], ws->s[1],
+                         ws->c[0], ws->c[1], b, ws->ctl, base, damp, ns);
+            pr_ctl_kernel<<<1, kPrBlock, 0, s>>>(ph->dev, ws->s[0], ws->s[1], ws->c[0], ws->c[1],
+                                                 b, ws->ctl, base, damp, grid, ws->host_done);
+        }
+        err = hipGetLastError();
+        if (err == hipSuccess) err = hipEventRecord(ev[batch & 1], s);
+        if (batch > 0 && err == hipSuccess) {
+            err = hipEventSynchronize(ev[(batch - 1) & 1]);
+            if (__atomic_load_n(&h->done, __ATOMIC_ACQUIRE)) break;
+        }
     }
-    HC_HIP(hipGetLastError());
-    HC_HIP(hipEventRecord(e1, s));
-    HC_HIP(hipEventSynchronize(e1));
-    float ms = 0;
-    HC_HIP(hipEventElapsedTime(&ms, e0, e1));
-    hipEventDestroy(e0);
-    hipEventDestroy(e1);
-    PrCtl c;
-    HC_HIP(hipMemcpyAsync(&c, ws->ctl, sizeof(PrCtl), hipMemcpyDeviceToHost, s));
-    HC_HIP(hipStreamSynchronize(s));
-    const float *final_s = (c.iter & 1) ? ws->s[1] : ws->s[0];
-    HC_HIP(hipMemcpyAsync(scores, final_s, sizeof(float) * g->n,
-                          hipMemcpyDeviceToDevice, s));
-    HC_HIP(hipStreamSynchronize(s));
+    if (err == hipSuccess) {
+        pr_result_kernel<<<init_grid, kBlock, 0, s>>>(ws->ctl, ws->s[0], ws->s[1], scores, g->n);
+        err = hipGetLastError();
+    }
+    if (err == hipSuccess)
+        err = hipMemcpyAsync(h + 1, ws->ctl, sizeof(PrCtl), hipMemcpyDeviceToHost, s);
+    const hipError_t waited = hipStreamSynchronize(s);
+    hipEventDestroy(ev[0]);
+    hipEventDestroy(ev[1]);
+    HC_HIP(err);
+    HC_HIP(waited);
+    const PrCtl c = h[1];
     if (stats) {
         std::memset(stats, 0, sizeof(*stats));
-        (void)ms;
         stats->ms = double(c.t_end - c.t_start) / device_state().clock_khz;
         stats->epochs = c.iter;
         stats->pull_epochs = c.iter;
-        stats->launches = max_iters;
+        stats->launches = launched;
         stats->reached = -1;
         stats->residual = c.residual;
         stats->alg_bytes = c.alg_bytes;
@@ -583,15 +690,17 @@ static int run_pr_pull(hc_graph_s *g, int mapping, const float *init, float *sco
                        double tol, int max_iters, int rule, int blocks, int threads,
                        hc_run_stats_t *stats, hipStream_t s) {
     const PlanHost *ph = nullptr;
-    if (mapping == HC_MAP_BUCKETED) HC_TRY(get_plan(g, 0, g->n, tuning().pull, &ph));
+    if (mapping == HC_MAP_BUCKETED) HC_TRY(get_plan(g, 0, g->n, pr_plan_config(g), &ph));
     PrWs *ws = nullptr;
-    HC_TRY(get_pr_ws(g, ph ? ph->dev.cnt[0] : 0, ph ? ph->dev.num_hubs : 0, &ws));
+    HC_TRY(get_pr_ws(g, ph ? ph->dev.cnt[0] : 0, &ws));
     GraphView<OffT> v = view<OffT>(g);
-    const int32_t ns = std::min<int32_t>(tuning().stage_pull, g->n);
+    int32_t ns = 0;
     int nb = blocks, nt = threads;
     if (mapping == HC_MAP_BUCKETED) {
-        nb = std::max(1, std::min(std::max(ph->total_units, 1), grid_blocks()));
-        nt = kBlock;
+        const PrShape sh =
+            pr_shape(g, 0, g->n, reinterpret_cast<const void *>(&pr_epoch_kernel<OffT>));
+        nb = sh.grid;
+        ns = sh.nstage;
     }
     double *dmem = nullptr;  // nb partials | the iteration's total
     HC_HIP(hipMalloc(&dmem, sizeof(double) * (nb + 1)));
@@ -624,15 +733,15 @@ static int run_pr_pull(hc_graph_s *g, int mapping, const float *init, float *sco
                                                                             partials);
                 break;
             default: {
-                PrBufs b{ws->inv_deg, ws->hub_hi, ws->hub_lo, ws->hub_cnt, ws->hub_resid, partials};
-                pr_epoch_kernel<OffT><<<nb, kBlock, ns * sizeof(float), s>>>(ph->dev, v, ep, b, ns);
+                PrBufs b{ws->inv_deg, ws->hub_hi, ws->hub_lo, partials};
+                pr_epoch_kernel<OffT><<<nb, kPrBlock, ns * sizeof(float), s>>>(ph->dev, v, ep, b, ns);
                 break;
             }
         }
         if (mapping == HC_MAP_BUCKETED) {
-            PrBufs b{ws->inv_deg, ws->hub_hi, ws->hub_lo, ws->hub_cnt, ws->hub_resid, partials};
+            PrBufs b{ws->inv_deg, ws->hub_hi, ws->hub_lo, partials};
             pr_pull_zero_kernel<<<1, 64, 0, s>>>(total);
-            pr_epoch_finish_kernel<<<1, kBlock, 0, s>>>(ph->dev, ep, b, nb, total);
+            pr_epoch_finish_kernel<<<1, kPrBlock, 0, s>>>(ph->dev, ep, b, nb, total);
         } else {
             pr_pull_total_kernel<<<1, kBlock, 0, s>>>(partials, nb, total);
         }
@@ -748,21 +857,22 @@ int hc_pr_pull_epoch(hc_graph_t g, int32_t start_id, int32_t end_id,
     GraphCall call(g);
     hipStream_t s = pick_stream(stream);
     const PlanHost *ph = nullptr;
-    HC_TRY(get_plan(g, start_id, end_id, tuning().pull, &ph));
+    HC_TRY(get_plan(g, start_id, end_id, pr_plan_config(g), &ph));
     PrWs *ws = nullptr;
-    HC_TRY(get_pr_ws(g, ph->dev.cnt[0], ph->dev.num_hubs, &ws));
-    PrBufs b{inv_degree, ws->hub_hi, ws->hub_lo, ws->hub_cnt, ws->hub_resid, ws->partials};
+    HC_TRY(get_pr_ws(g, ph->dev.cnt[0], &ws));
+    PrBufs b{inv_degree, ws->hub_hi, ws->hub_lo, ws->partials};
     PrEpoch ep{score_in, contrib, score_out, contrib_out,
                (1.0f - damping) / (float)g->n, damping, 0};
-    const int nb = std::max(1, std::min(std::max(ph->total_units, 1), grid_blocks()));
-    const int32_t ns = std::min<int32_t>(tuning().stage_pull, g->n);
-    if (g->off64)
-        pr_epoch_kernel<uint64_t><<<nb, kBlock, ns * sizeof(float), s>>>(
-            ph->dev, view<uint64_t>(g), ep, b, ns);
-    else
-        pr_epoch_kernel<uint32_t><<<nb, kBlock, ns * sizeof(float), s>>>(
-            ph->dev, view<uint32_t>(g), ep, b, ns);
-    pr_epoch_finish_kernel<<<1, kBlock, 0, s>>>(ph->dev, ep, b, nb, residual_out);
+    auto sweep = [&](auto off) {
+        using OffT = decltype(off);
+        const PrShape sh =
+            pr_shape(g, start_id, end_id, reinterpret_cast<const void *>(&pr_epoch_kernel<OffT>));
+        pr_epoch_kernel<OffT><<<sh.grid, kPrBlock, sh.nstage * sizeof(float), s>>>(
+            ph->dev, view<OffT>(g), ep, b, sh.nstage);
+        return sh.grid;
+    };
+    const int nb = g->off64 ? sweep(uint64_t(0)) : sweep(uint32_t(0));
+    pr_epoch_finish_kernel<<<1, kPrBlock, 0, s>>>(ph->dev, ep, b, nb, residual_out);
     HC_HIP(hipGetLastError());
     return HC_OK;
 }

@@ -434,6 +434,7 @@ int hc_init(int device) {
             s.clock_khz = khz;
     }
     s.hbm = prop.totalGlobalMem;
+    s.max_lds = prop.sharedMemPerBlock;
     if (!s.stream) HC_HIP(hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking));
     s.ready = true;
     return HC_OK;
