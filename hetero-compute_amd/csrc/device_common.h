@@ -138,7 +138,7 @@ struct Tuning {
     int bu_first = 2;      // BFS: rows probe the first-neighbour array (1: one-lane
                            // rows, 2: all rows)
     int bu_stage_min = 4096;  // BFS: unvisited lists shorter than this skip LDS staging
-    int compact_grid = 4096;  // workgroups of the frontier compaction launch (capped)
+    int compact_grid = 512;   // workgroups of the frontier compaction launch (capped)
     int loop_batch = 2;    // epochs the host enqueues per poll of the done flag
     int kernel_events = 0; // 1: time every launch of a loop's main kernel
     int multi_graph = 1;   // batched SSSP/BFS: relaunch an epoch hipGraph

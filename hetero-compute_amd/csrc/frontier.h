@@ -558,12 +558,14 @@ __device__ __forceinline__ void ctl_end(const StepCtl *s_c, StepCtl *cur, StepCt
 }
 
 // Bitmap -> degree-classed queues of parity (epoch & 1), run by the
-// between-epochs launch with the decided header c.  Each workgroup
-// takes a contiguous run of bitmap words, counts its vertices per class in
-// LDS and reserves its output with one atomic per class.
+// between-epochs launch with the decided header c.  Each workgroup takes its
+// share of the bitmap's lines, counts their vertices per class in LDS and
+// reserves its output with one atomic per class.
 // The launch is queued after every epoch but has compaction work only when
 // the direction turns to top-down; a smaller grid keeps its idle launches
-// cheap (tuning knob compact.grid: workgroups, at most the step grid).
+// cheap (tuning knob compact.grid: workgroups, at most the step grid; BFS on 8M
+// vertices: 315 us with 1024 and more, 310 with 512, 308 with 256, which leaves
+// the rebuild of the 16-bit mirror too few).
 inline int compact_grid(int step_grid) { return std::max(1, std::min(step_grid, tuning().compact_grid)); }
 
 // SSSP with a 16-bit distance mirror (`d16`): before every pull epoch the
@@ -585,36 +587,82 @@ __device__ void compact_body(const GraphView<OffT> &g, const FrontierBufs &fb,
     const uint32_t *bm = three_bitmaps ? fb.bm[k % 3] : fb.bm[k & 1];
     const int words = fb.words;
     const int64_t ck = ctl->chunk;
-    // Word w belongs to workgroup w % grid, so the hub words at the start
-    // of a degree-sorted bitmap spread over many workgroups.
+    // Lines of 16 words are dealt to the workgroups in turn, so the hubs at the
+    // start of a degree-sorted bitmap spread over many of them.
+    constexpr int kLine = 16;
     const int stride = gridDim.x;
-    const int rounds = (words - (int)blockIdx.x + stride * kBlock - 1) / (stride * kBlock);
+    const int lines = (words + kLine - 1) / kLine;
+    const int mine = lines > (int)blockIdx.x ? (lines - (int)blockIdx.x + stride - 1) / stride : 0;
+    const int rounds = (mine + kBlock / kLine - 1) / (kBlock / kLine);
     constexpr uint32_t kHubList = 256;
     __shared__ uint32_t s_cnt[5], s_base[5], s_nhub;
+    __shared__ uint32_t s_wave[kWavesPerBlock];
+    __shared__ uint16_t s_bit[kBlock * 32];  // set bits: thread << 5 | bit
+    __shared__ uint8_t s_class[kBlock * 32];
     __shared__ int32_t s_hub_v[kHubList];
     __shared__ uint32_t s_hub_at[kHubList], s_hub_pre[kHubList + 1];
     __shared__ long long s_hub_b[kHubList], s_hub_e[kHubList];
+    auto word_of = [&](int r, int t) {
+        return ((r * kBlock + t) / kLine * stride + (int)blockIdx.x) * kLine + t % kLine;
+    };
+    auto load_word = [&](int r) {
+        const int w = word_of(r, threadIdx.x);
+        return r < rounds && w < words ? bm[w] : 0u;
+    };
+    uint32_t ahead = load_word(0);
     for (int r = 0; r < rounds; r++) {
+        const uint32_t bits = ahead;
+        ahead = load_word(r + 1);
         if (threadIdx.x < 5) s_cnt[threadIdx.x] = 0;
         if (threadIdx.x == 0) s_nhub = 0;
+        // The set bits of the round as one list, a thread taking every
+        // kBlock-th of them.  With a thread per word, a dense word's vertices
+        // were a chain of up to 64 dependent loads (SSSP, Kronecker, 64K
+        // vertices, one compaction: 388 us a query, 378 so).
+        const uint32_t pop = __popc(bits);
+        uint32_t before = pop;
+#pragma unroll
+        for (int sh = 1; sh < kWave; sh <<= 1) {
+            const uint32_t o = __shfl_up(before, sh, kWave);
+            if (lane_id() >= sh) before += o;
+        }
+        if (lane_id() == kWave - 1) s_wave[threadIdx.x / kWave] = before;
         __syncthreads();
-        const int w = (int)blockIdx.x + (r * kBlock + (int)threadIdx.x) * stride;
-        uint32_t bits = (w < words) ? bm[w] : 0u;
+        uint32_t total = 0;
+        before -= pop;
+        for (int i = 0; i < kWavesPerBlock; i++) {
+            if (i < (int)threadIdx.x / kWave) before += s_wave[i];
+            total += s_wave[i];
+        }
+        for (uint32_t x = bits; x; x &= x - 1)
+            s_bit[before++] = uint16_t(threadIdx.x << 5 | (__ffs(x) - 1));
+        __syncthreads();
+        if (total == 0) continue;
+        auto vertex = [&](uint32_t j) {
+            const int e = s_bit[j];
+            return word_of(r, e >> 5) * 32 + (e & 31);
+        };
         // pass 1: count per class (class 3 counts chunks; slot 4 hubs)
-        uint32_t my[5] = {0, 0, 0, 0, 0};
-        for (uint32_t x = bits; x; x &= x - 1) {
-            int32_t v = w * 32 + __ffs(x) - 1;
-            int64_t d = int64_t(g.rend(v) - g.rbeg(v));
-            int c = degree_class(d, ctl->mid);
-            if (c < 3) {
-                my[c]++;
-            } else {
-                my[3] += (uint32_t)((d + ck - 1) / ck);
-                my[4]++;
+        for (uint32_t j0 = threadIdx.x; j0 < total; j0 += 4 * kBlock) {
+            int64_t d[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const uint32_t j = j0 + q * kBlock;
+                d[q] = -1;
+                if (j < total) {
+                    const int32_t v = vertex(j);
+                    d[q] = int64_t(g.rend(v) - g.rbeg(v));
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                if (d[q] < 0) continue;
+                const int c = degree_class(d[q], ctl->mid);
+                s_class[j0 + q * kBlock] = (uint8_t)c;
+                atomicAdd(&s_cnt[c], c < 3 ? 1u : (uint32_t)((d[q] + ck - 1) / ck));
+                if (c == 3) atomicAdd(&s_cnt[4], 1u);
             }
         }
-        uint32_t off[5];
-        for (int c = 0; c < 5; c++) off[c] = my[c] ? atomicAdd(&s_cnt[c], my[c]) : 0;
         __syncthreads();
         if (threadIdx.x < 5)
             s_base[threadIdx.x] = s_cnt[threadIdx.x]
@@ -624,16 +672,15 @@ __device__ void compact_body(const GraphView<OffT> &g, const FrontierBufs &fb,
         // pass 2: queue entries; hubs are listed with their chunk range and
         // their descriptors written by the whole workgroup below (serially
         // by the owning thread only past the list's capacity).
-        for (uint32_t x = bits; x; x &= x - 1) {
-            int32_t v = w * 32 + __ffs(x) - 1;
-            OffT b = g.rbeg(v), e = g.rend(v);
-            int64_t d = int64_t(e - b);
-            int c = degree_class(d, ctl->mid);
+        for (uint32_t j = threadIdx.x; j < total; j += kBlock) {
+            const int32_t v = vertex(j);
+            const int c = s_class[j];
             if (c < 3) {
-                fb.q[p][c][s_base[c] + off[c]++] = v;
+                fb.q[p][c][atomicAdd(&s_base[c], 1u)] = v;
             } else {
-                const uint32_t at = s_base[3] + off[3];
-                off[3] += (uint32_t)((d + ck - 1) / ck);
+                const OffT b = g.rbeg(v), e = g.rend(v);
+                const uint32_t at =
+                    atomicAdd(&s_base[3], (uint32_t)((int64_t(e - b) + ck - 1) / ck));
                 const uint32_t h = atomicAdd(&s_nhub, 1u);
                 if (h < kHubList) {
                     s_hub_v[h] = v;

@@ -260,7 +260,7 @@ int hc_graph_get_info(hc_graph_t g, hc_graph_info_t *out);
  *                          this reads the frontier bitmap without LDS
  *                          staging (4096)
  *   compact.grid           workgroups of the frontier compaction launch, at
- *                          most the step grid (4096)
+ *                          most the step grid (512)
  *   bu.first               bottom-up rows test their first neighbour from a
  *                          per-vertex array (n int32 per graph) before the
  *                          edge array: 1 one-lane rows, 2 all rows, 0 off (2)
