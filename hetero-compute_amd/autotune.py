@@ -72,7 +72,7 @@ KNOB_SPACE = {
         "bu.stage": [0, 2048, 8192, 15360],
         "bu.wave_threshold": [1024, 4096],
         "bu.g16_threshold": [128, 256, 512],
-        "bu.g4_threshold": [8, 16, 32, 64],
+        "bu.g4_threshold": [32, 64, 128, 256],
         "bu.remaining": [0, 1, 4],
         "bu.stage_min": [0, 256, 1024, 4096, 1 << 20],
         "bu.first": [0, 1, 2],
