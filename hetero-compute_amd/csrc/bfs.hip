@@ -1169,11 +1169,12 @@ static int run_bfs_loop(hc_graph_s *g, int32_t src, int32_t *depth,
     BfsLaunch<OffT> L{ph->dev, v, depth, parents, tuning().bu_first ? ws->first : nullptr,
                       head4, ws->f.fb, ws->f.ctl, rl, grid, s, nstage, tuning().bu_stage_min,
                       lds_words, push_cap, tuning().bu_first == 2, &ws->f.kt};
-    const long long cap = (long long)g->n + 2;  // levels <= n
+    // At most n levels, and a heavy top-down one takes two launch pairs.
+    const long long cap = 2 * (long long)g->n + 2;
     long long launches = 0;
     StepCtl fc;
     HC_TRY(run_epoch_loop(&ws->f, s, cap, &BfsLaunch<OffT>::launch, &L, &launches, &fc));
-    if (!fc.done) return fail(HC_ERR_HIP, "BFS loop did not finish in %lld epochs", launches);
+    if (!fc.done) return fail(HC_ERR_HIP, "BFS loop did not finish in %lld launch pairs", launches);
     fill_bfs_stats(fc, (int32_t)(2 * launches), stats);
     if (stats) {
         if (ws->f.kt.on) {

@@ -45,6 +45,23 @@ def test_heavy_top_down_epochs(hc, gpu, oracle, leaves):
     _check(hc, oracle, g, [0, int(dst[1][0])])
 
 
+@pytest.mark.parametrize("n", [4, 5, 9])
+def test_path_of_parallel_edges(hc, gpu, n):
+    """A path whose links are 2^19 + n parallel edges: every level after the
+    first is a heavy top-down epoch, so the loop takes two launch pairs for
+    nearly every vertex."""
+    k = (1 << 19) + n
+    rows = [[v for v in (u - 1, u + 1) if 0 <= v < n] for u in range(n)]
+    index = np.concatenate([[0], np.cumsum([k * len(r) for r in rows])]).astype(np.int64)
+    g = hc.HostGraph.from_csr(index, np.repeat(np.concatenate(rows), k).astype(np.int32))
+    with hc.DeviceGraph(g) as dg:
+        for s in (0, n - 1, n // 2):
+            b = hc.bfs(dg, s, direction=2)
+            assert b.values.tolist() == [abs(v - s) for v in range(n)]
+            assert b.parents.tolist() == [v - np.sign(v - s) for v in range(n)]
+            assert b.stats["epochs"] == max(s, n - 1 - s) + 1
+
+
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("degree", [1, 2, 3, 9])
 def test_flat_rows_read_ahead(hc, gpu, oracle, monkeypatch, degree, wide):
