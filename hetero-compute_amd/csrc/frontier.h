@@ -88,7 +88,7 @@ struct StepCtl {
     // cannot beat the row's distance from it, are not looked at).
     int32_t low;
     int32_t sorted;                // SSSP: sweeps run on the weight-sorted adjacency
-    // SSSP buckets (delta > 0): the current bucket holds the distances in
+    // SSSP buckets (delta > 0) there: the current bucket holds the distances in
     // [base, thresh).  Its push epochs (or, from a heavy frontier, sweeps over
     // the rows: a promotion epoch with settle 3) relax the edges that land in
     // it; when a frontier comes out empty, the bucket's distances are final
@@ -103,6 +103,14 @@ struct StepCtl {
     int32_t promotions;            // promotion epochs run
     long long bucket_e;            // degree sum of this bucket's frontiers
     long long done_e;              // and of the buckets before it
+    // Buckets on the plain CSR (push epochs only): a vertex lowered to a value
+    // at or above thresh goes to the far bitmap instead of the next frontier;
+    // when a frontier comes out empty thresh rises (by delta, doubled after a
+    // promotion that found nothing) and a promotion epoch makes the far
+    // vertices now below it the frontier.
+    int32_t far_step;              // the last rise of thresh
+    int32_t far_pad;
+    long long far_live;            // upper bound of the far vertices
     // Device wall clock (constant rate): start of the loop, end of the last
     // epoch, and end of each traced epoch.
     long long t_start;
@@ -143,6 +151,7 @@ struct FrontierBufs {
     int32_t *q[2][3];
     HubChunk *ch[2];
     uint32_t *bm[3];
+    uint32_t *far;             // SSSP buckets on the plain CSR: vertices waiting
     uint32_t (*cnt)[5];        // queue fill [parity][q0, q1, q2, chunks, hubs]
     int32_t words;             // bitmap words
     Partials part;             // counter set of the current epoch

@@ -323,17 +323,18 @@ constexpr int kPushTrip = 4;  // edges a lane of a push epoch has in flight
 // edge in flight per lane they would want a wavefront from 17 edges on.
 constexpr int32_t kPushMid = 64;
 
-// Edges of a push epoch: the CSR's two arrays, or the weight-sorted pairs.
-template <typename OffT>
+// Edges of a push epoch: the CSR's two arrays (FAR: with buckets), or the
+// weight-sorted pairs.
+template <typename OffT, bool FAR = false>
 struct CsrEdges {
-    static constexpr bool kSorted = false;
+    static constexpr bool kSorted = false, kFar = FAR;
     const int32_t *adj, *wt;
     __device__ __forceinline__ int2 get(OffT i) const { return int2{adj[i], wt[i]}; }
     __device__ __forceinline__ int32_t floor(int32_t) const { return 0; }
 };
 template <typename OffT>
 struct SortedEdges {
-    static constexpr bool kSorted = true;
+    static constexpr bool kSorted = true, kFar = false;
     SortedView v;
     __device__ __forceinline__ int2 get(OffT i) const { return v.e[i]; }
     __device__ __forceinline__ int32_t floor(int32_t w) const { return v.floor(w); }
@@ -344,7 +345,9 @@ struct SortedEdges {
 // staging slot -- and its latency bounds the epoch); a lowered neighbour joins
 // the next frontier.  Sorted edges: only those that land below `thresh` are
 // relaxed (buckets; HC_INF_DIST: all), and the scan stops at the first key
-// that cannot.  `lowest` is the smallest value written.
+// that cannot.  Buckets on the CSR: a neighbour lowered to thresh or more joins
+// the far bitmap instead (`nfar` counts those settings).  `lowest` is the
+// smallest value written.
 template <int G, typename ER, typename OffT>
 __device__ __forceinline__ void push_range(const GraphView<OffT> &g, const ER &er,
                                            int32_t *__restrict__ dist,
@@ -353,8 +356,9 @@ __device__ __forceinline__ void push_range(const GraphView<OffT> &g, const ER &e
                                            int nxt, uint32_t *wbm, int32_t u, OffT b,
                                            OffT e, int lane, uint32_t &cnt,
                                            unsigned long long &edges_acc, int32_t thresh,
-                                           int32_t &lowest) {
+                                           int32_t &lowest, uint32_t &nfar) {
     const int32_t du = dist[u];
+    const int32_t reach = ER::kSorted ? thresh : HC_INF_DIST;
     for (OffT i = b + OffT(lane); i < e; i += OffT(kPushTrip * G)) {
         int2 x[kPushTrip];
         bool in[kPushTrip];
@@ -364,12 +368,12 @@ __device__ __forceinline__ void push_range(const GraphView<OffT> &g, const ER &e
             in[r] = k < e;
             x[r] = in[r] ? er.get(k) : int2{0, 0};
         }
-        if (ER::kSorted && relax(du, er.floor(x[0].y)) >= thresh) break;
+        if (ER::kSorted && relax(du, er.floor(x[0].y)) >= reach) break;
         int32_t nd[kPushTrip], d[kPushTrip], old[kPushTrip];
 #pragma unroll
         for (int r = 0; r < kPushTrip; r++) {
             nd[r] = in[r] ? relax(du, x[r].y) : HC_INF_DIST;
-            d[r] = nd[r] < thresh ? dist[x[r].x] : 0;
+            d[r] = nd[r] < reach ? dist[x[r].x] : 0;
         }
 #pragma unroll
         for (int r = 0; r < kPushTrip; r++)
@@ -381,6 +385,11 @@ __device__ __forceinline__ void push_range(const GraphView<OffT> &g, const ER &e
             v[r] = x[r].x;
             lowered[r] = nd[r] < old[r];
             if (lowered[r]) lowest = min(lowest, nd[r]);
+            if (ER::kFar && lowered[r] && nd[r] >= thresh) {
+                atomicOr(&fb.far[v[r] >> 5], 1u << (v[r] & 31));
+                nfar++;
+                lowered[r] = false;
+            }
             if (!out.dedup && lowered[r]) {
                 // The first edge to set v's bit appends v, now.
                 const uint32_t bit = 1u << (v[r] & 31);
@@ -403,8 +412,9 @@ __device__ __forceinline__ void sssp_push_sweep(const GraphView<OffT> &g, const 
                                 const FrontierBufs &fb, StepCtl *ctl,
                                 const PushOut &out, int cur,
                                 int nxt, uint32_t *wbm, uint32_t &cnt,
-                                unsigned long long &edges_acc, int32_t &lowest) {
-    const int32_t thresh = ER::kSorted ? ctl->thresh : HC_INF_DIST;
+                                unsigned long long &edges_acc, int32_t &lowest,
+                                uint32_t &nfar) {
+    const int32_t thresh = ctl->thresh;
     const uint32_t nch = fb.cnt[cur][3], n0 = fb.cnt[cur][0],
                    n1 = fb.cnt[cur][1], n2 = fb.cnt[cur][2];
     const uint32_t u1 = nch + n0;
@@ -421,17 +431,17 @@ __device__ __forceinline__ void sssp_push_sweep(const GraphView<OffT> &g, const 
         if (unit < nch) {
             HubChunk h = fb.ch[cur][unit];
             push_range<kBlock>(g, er, dist, fb, ctl, out, nxt, wbm, h.u, OffT(h.b), OffT(h.e),
-                               threadIdx.x, cnt, edges_acc, thresh, lowest);
+                               threadIdx.x, cnt, edges_acc, thresh, lowest, nfar);
         } else if (unit < u1) {
             int32_t u = fb.q[cur][0][unit - nch];
             push_range<kBlock>(g, er, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u), g.rend(u),
-                               threadIdx.x, cnt, edges_acc, thresh, lowest);
+                               threadIdx.x, cnt, edges_acc, thresh, lowest, nfar);
         } else if (unit < u2) {
             uint32_t idx = (unit - u1) * kWavesPerBlock + threadIdx.x / kWave;
             if (idx < n1) {
                 int32_t u = fb.q[cur][1][idx];
                 push_range<kWave>(g, er, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u), g.rend(u),
-                                  lane_id(), cnt, edges_acc, thresh, lowest);
+                                  lane_id(), cnt, edges_acc, thresh, lowest, nfar);
             }
         } else {
             uint32_t idx = (unit - u2) * kSmallPerUnit + threadIdx.x / kSmallLanes;
@@ -439,8 +449,39 @@ __device__ __forceinline__ void sssp_push_sweep(const GraphView<OffT> &g, const 
                 int32_t u = fb.q[cur][2][idx];
                 push_range<kSmallLanes>(g, er, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u),
                                         g.rend(u), threadIdx.x % kSmallLanes, cnt,
-                                        edges_acc, thresh, lowest);
+                                        edges_acc, thresh, lowest, nfar);
             }
+        }
+    }
+}
+
+// Promotion epoch of the buckets on the CSR: every far vertex whose distance is
+// now below `thresh` leaves the far bitmap and is set in the changed bitmap
+// `wbm` (compacted into the next frontier's queues by the launch after);
+// `left` counts the vertices still far.  A thread owns one word of both
+// bitmaps.
+template <typename OffT>
+__device__ __forceinline__ void promote_far(const GraphView<OffT> &g, const int32_t *dist,
+                                            const FrontierBufs &fb, int32_t thresh, uint32_t *wbm,
+                                            uint32_t &cnt, unsigned long long &edges_acc,
+                                            uint32_t &left) {
+    for (int w = blockIdx.x * kBlock + threadIdx.x; w < fb.words; w += gridDim.x * kBlock) {
+        const uint32_t word = fb.far[w];
+        uint32_t now = 0;
+        for (uint32_t x = word; x; x &= x - 1) {
+            const int b = __ffs(x) - 1;
+            const int32_t v = w * 32 + b;
+            if (dist[v] < thresh) {
+                now |= 1u << b;
+                cnt++;
+                edges_acc += (unsigned long long)(g.rend(v) - g.rbeg(v));
+            } else {
+                left++;
+            }
+        }
+        if (now) {
+            fb.far[w] = word & ~now;
+            wbm[w] = now;  // cleared by the launch before; no other writer
         }
     }
 }
@@ -879,13 +920,49 @@ __global__ __launch_bounds__(kBlock) void sssp_step_kernel(
         __syncthreads();
         const PushOut out{s_stage, &s_out, (uint32_t)push_cap, defer_dedup ? wbm : nullptr};
         int32_t lowest = HC_INF_DIST;
+        uint32_t nfar = 0;
         sssp_push_sweep(g, CsrEdges<OffT>{g.adj, g.wt}, dist, fb, ctl, out, cur, nxt, wbm, cnt,
-                        eacc, lowest);
+                        eacc, lowest, nfar);
         const PushKept k = push_out_flush(out, g, fb, ctl, nxt);
         cnt += k.n;
         eacc += k.e;
     }
     write_partials(fb.part, cnt, eacc, gathered);
+}
+
+// The step of the buckets on the CSR: push and promotion epochs.
+template <typename OffT>
+__global__ __launch_bounds__(kBlock) void sssp_near_far_kernel(GraphView<OffT> g,
+                                                               int32_t *__restrict__ dist,
+                                                               FrontierBufs fb, StepCtl *ctl,
+                                                               int32_t push_cap,
+                                                               int defer_dedup) {
+    extern __shared__ int32_t s_stage[];
+    __shared__ uint32_t s_out;
+    if (ctl->done) return;
+    const int k = ctl->epoch;
+    const int cur = k & 1, nxt = cur ^ 1;
+    uint32_t *wbm = fb.bm[(k + 1) % 3];
+    uint32_t *cbm = fb.bm[(k + 2) % 3];
+    for (int w = blockIdx.x * kBlock + threadIdx.x; w < fb.words; w += gridDim.x * kBlock)
+        cbm[w] = 0;
+    // `nfar`: far settings of a push, vertices left far by a promotion.
+    uint32_t cnt = 0, nfar = 0;
+    unsigned long long eacc = 0;
+    if (ctl->mode == kPromote) {
+        promote_far(g, dist, fb, ctl->thresh, wbm, cnt, eacc, nfar);
+    } else {
+        if (threadIdx.x == 0) s_out = 0;
+        __syncthreads();
+        const PushOut out{s_stage, &s_out, (uint32_t)push_cap, defer_dedup ? wbm : nullptr};
+        int32_t lowest = HC_INF_DIST;
+        sssp_push_sweep(g, CsrEdges<OffT, true>{g.adj, g.wt}, dist, fb, ctl, out, cur, nxt, wbm,
+                        cnt, eacc, lowest, nfar);
+        const PushKept kept = push_out_flush(out, g, fb, ctl, nxt);
+        cnt += kept.n;
+        eacc += kept.e;
+    }
+    write_partials(fb.part, cnt, eacc, nfar);
 }
 
 // The step on the weight-sorted adjacency (the default): pull epochs or, with
@@ -922,8 +999,9 @@ __global__ __launch_bounds__(kBlock) void sssp_sorted_step_kernel(
     const RowBounds rb{ctl->low, ctl->base, ctl->thresh};
     if (mode == kPush && !(BUCKETS && ctl->settle)) {
         const PushOut out{s_stage, &s_out, (uint32_t)push_cap, defer_dedup ? wbm : nullptr};
+        uint32_t nfar = 0;
         sssp_push_sweep(g, SortedEdges<OffT>{sv}, dist, fb, ctl, out, cur, nxt, wbm, s.cnt,
-                        s.edges, s.lowest);
+                        s.edges, s.lowest, nfar);
         const PushKept kept = push_out_flush(out, g, fb, ctl, nxt);
         s.cnt += kept.n;
         s.edges += kept.e;
@@ -962,7 +1040,13 @@ __device__ void sssp_decide(StepCtl *c, StepCtl *trace,
     const int k = c->epoch;
     const int ran = c->mode;
     const int settled = c->settle;
-    if (ran == kPromote) {
+    if (ran == kPromote && !c->sorted) {
+        // far bitmap words, plus dist[v] and a bitmap entry per far vertex
+        c->alg_bytes += 4ull * (unsigned long long)((c->n + 31) / 32) + 8ull * (out_n + gathered);
+        c->promotions++;
+        c->far_live = (long long)gathered;
+        trace_epoch(c, trace, k, ran, out_n, out_e, 0);
+    } else if (ran == kPromote) {
         // dist per vertex; pair + gathered distance per relaxed edge and
         // offsets per row of a settling sweep; a bit per frontier vertex
         c->alg_bytes += (settled ? 8ull : 4ull) * (unsigned long long)c->n + 12ull * gathered +
@@ -980,6 +1064,7 @@ __device__ void sssp_decide(StepCtl *c, StepCtl *trace,
             trace_epoch(c, trace, k, ran, out_n, out_e, c->in_e);
         }
         c->push_epochs++;
+        if (!c->sorted) c->far_live += (long long)gathered;  // may repeat a vertex
     } else if (c->sorted) {
         // Offsets and own distances; id + weight + distance per edge relaxed.
         c->alg_bytes += (unsigned long long)c->sweep_bytes - 12ull * (unsigned long long)c->m +
@@ -1007,6 +1092,17 @@ __device__ void sssp_decide(StepCtl *c, StepCtl *trace,
     int next = ran;
     if (c->max_epochs > 0 && k + 1 >= c->max_epochs) {
         c->done = 1;
+    } else if (c->delta > 0 && !c->sorted) {
+        if (out_n != 0) {
+            next = kPush;
+        } else if (c->far_live > 0) {
+            const long long step = ran == kPromote ? 2ll * c->far_step : (long long)c->delta;
+            c->far_step = (int32_t)min(step, (long long)HC_INF_DIST);
+            c->thresh = (int32_t)min((long long)c->thresh + step, (long long)HC_INF_DIST);
+            next = kPromote;
+        } else {
+            c->done = 1;
+        }
     } else if (c->delta > 0) {
         c->settle = 0;
         if (out_n != 0) {
@@ -1104,6 +1200,7 @@ __global__ __launch_bounds__(kBlock) void sssp_init_kernel(
         fb.bm[0][w] = (!init_dist && w == (src >> 5)) ? (1u << (src & 31)) : 0u;
         fb.bm[1][w] = 0;
         fb.bm[2][w] = 0;
+        fb.far[w] = 0;
     }
     // Smallest initial distance (sssp_init_low_kernel's results lie in the
     // counter sets, one per workgroup of that launch).
@@ -1150,6 +1247,8 @@ __global__ __launch_bounds__(kBlock) void sssp_init_kernel(
         ctl->promotions = 0;
         ctl->bucket_e = 0;
         ctl->done_e = 0;
+        ctl->far_step = delta;
+        ctl->far_live = 0;
         ctl->reached = 0;
         ctl->alg_bytes = 0;
         ctl->t_start = wall_clock64();
@@ -1445,6 +1544,10 @@ struct SsspLaunch {
         if (a->sv.e) {
             if (a->buckets) a->template sorted_step<true>(fb, cur);
             else a->template sorted_step<false>(fb, cur);
+        } else if (a->buckets) {
+            timed_launch(a->kt, sssp_near_far_kernel<OffT>, dim3(a->grid), dim3(kBlock),
+                         uint32_t(a->lds_entries * sizeof(int32_t)), a->s, a->g, a->dist, fb, cur,
+                         a->push_cap, a->defer_dedup);
         } else if (a->d16) {
             if (a->cbk) a->template step<true, true>(fb, cur);
             else a->template step<true, false>(fb, cur);
@@ -1460,17 +1563,26 @@ struct SsspLaunch {
 };
 
 
-// Bucket width of the single-source loop (knob sssp.delta): 4 x the sampled
-// largest weight / mean degree on flat graphs (uniform 23, weights 1..255,
-// degree 32: widths 24 / 32 / 48 / 64 / 96 4.41 / 4.06 / 4.41 / 4.56 / 4.70
+// Bucket width of the single-source loop (knob sssp.delta).  Sorted adjacency: 4 x
+// the sampled largest weight / mean degree on flat graphs (uniform 23, weights
+// 1..255, degree 32: widths 24 / 32 / 48 / 64 / 96 4.41 / 4.06 / 4.41 / 4.56 / 4.70
 // ms), off on skewed ones, whose pull sweeps win (Kronecker 23: 1.36 ms
 // against 2.4 / 1.8 ms with widths 32 / 96).
-static int sssp_delta(hc_graph_s *g) {
+// Plain CSR: 2 x, on flat graphs of at least kNearFarMinEdges edges.  Buckets
+// save re-relaxations and cost epochs, so the line is where an epoch's work
+// outweighs its launches (plain loop against buckets; uniform graphs, 65 K
+// vertices, 2.1 M edges: 0.56 / 0.99 ms; 256 K, 7.9 M: 1.01 / 1.34; 4 M, 16.8 M:
+// 2.24 / 2.39; 1 M, 33.6 M: 2.28 / 2.15; 16 M, 67 M: 8.79 / 5.86; 8 M, 268 M:
+// 20.7 / 9.75; grids of 4.2 M, 16.8 M and 67 M edges: 26 / 55, 114 / 147, 579 /
+// 344).
+constexpr int64_t kNearFarMinEdges = int64_t(1) << 24;
+static int sssp_delta(hc_graph_s *g, bool sorted) {
     const int d = tuning().sssp_delta;
     if (d >= 0) return d;
     if (!g->weighted || g->m == 0 || g->max_weight <= 0 || !flat_graph(g)) return 0;
+    if (!sorted && g->m < kNearFarMinEdges) return 0;
     const double mean_deg = (double)g->m / std::max(1, g->rows);
-    return (int)std::max(1.0, std::ceil(4.0 * g->max_weight / mean_deg));
+    return (int)std::max(1.0, std::ceil((sorted ? 4.0 : 2.0) * g->max_weight / mean_deg));
 }
 
 template <typename OffT>
@@ -1495,8 +1607,10 @@ static int run_sssp_loop(hc_graph_s *g, int32_t src, const int32_t *init_dist,
     // A pruned pull costs little more than its row heads: pull early
     // (Kronecker 23: alpha 4 / 8 / 16 / 32 1.72 / 1.39 / 1.36 / 1.35 ms).
     if (alpha <= 0) alpha = t.sssp_alpha > 0 ? t.sssp_alpha : (sorted ? 16 : flat_graph(g) ? 2 : 4);
+    // Buckets (sssp.delta): no pulls on the CSR.
+    const int delta = init_dist || direction == 1 ? 0 : sssp_delta(g, sorted);
     uint16_t *d16 = nullptr;
-    if (!sorted && (t.sssp_dist16 == 1 || (t.sssp_dist16 == 2 && flat_graph(g)))) {
+    if (!sorted && delta == 0 && (t.sssp_dist16 == 1 || (t.sssp_dist16 == 2 && flat_graph(g)))) {
         if (!ws->d16 && hipMalloc(&ws->d16, sizeof(uint16_t) * std::max(g->n, 1)) != hipSuccess)
             return fail(HC_ERR_OOM, "16-bit distance mirror allocation failed");
         d16 = ws->d16;
@@ -1507,11 +1621,9 @@ static int run_sssp_loop(hc_graph_s *g, int32_t src, const int32_t *init_dist,
     const int32_t lds_entries = std::max<int32_t>(nstage, push_cap);
     // Pull epochs gather column block by column block (not with filtering,
     // which tests a changed bit per neighbour before its gather).
-    // Buckets (sssp.delta): on the sorted adjacency.
-    const int delta = init_dist || direction == 1 || !sorted ? 0 : sssp_delta(g);
     const ColBlocks *cb = nullptr;
     const PlanHost *phb = nullptr;
-    if (!sorted && direction != 2 && tuning().sssp_filter != 1) {
+    if (!sorted && delta == 0 && direction != 2 && tuning().sssp_filter != 1) {
         HC_TRY(get_col_blocks(g, col_shift_for(g, flat_graph(g)), s, &cb));
         if (cb) {
             // Plain sweep for the light rows only.
@@ -1522,6 +1634,7 @@ static int run_sssp_loop(hc_graph_s *g, int32_t src, const int32_t *init_dist,
     const void *step_fn =
         sorted ? (delta > 0 ? reinterpret_cast<const void *>(&sssp_sorted_step_kernel<OffT, true>)
                             : reinterpret_cast<const void *>(&sssp_sorted_step_kernel<OffT, false>))
+        : delta > 0 ? reinterpret_cast<const void *>(&sssp_near_far_kernel<OffT>)
         : d16 ? (cb ? reinterpret_cast<const void *>(&sssp_step_kernel<OffT, true, true>)
                   : reinterpret_cast<const void *>(&sssp_step_kernel<OffT, true, false>))
             : (cb ? reinterpret_cast<const void *>(&sssp_step_kernel<OffT, false, true>)

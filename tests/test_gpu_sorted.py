@@ -123,6 +123,53 @@ def test_flat_buckets_cover_every_settling_path(hc, gpu, oracle):
                     assert np.array_equal(hc.sssp(dg, s, direction=2).values, ref), (top, delta)
 
 
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("knob,value", [("sssp.sorted", 0), ("sssp.filter", 1), ("sssp.dist16", 1),
+                                        ("pull.col_shift", 10)])
+def test_buckets_without_the_copy(hc, gpu, oracle, monkeypatch, knob, value, wide):
+    """sssp.delta holds on the plain CSR too (no copy, or a knob that asks for a
+    plain sweep): vertices past the threshold wait in the far set and are
+    promoted, hubs and zero weights among them, and no epoch pulls."""
+    if wide:
+        monkeypatch.setenv("HC_FORCE_OFF64", "1")
+    rng = np.random.default_rng(8)
+    n = 20000
+    src, dst = rng.integers(0, n - 300, 6 * n), rng.integers(0, n - 300, 6 * n)
+    for top in (3, 255, (1 << 30) - 2):
+        w = rng.integers(0, top + 1, src.size).astype(np.int32)
+        flat = hc.HostGraph.from_edges(src.astype(np.int32), dst.astype(np.int32), n, weights=w)
+        for g in (flat, _stars(hc, DEGREES, top, 1)):
+            with hc.DeviceGraph(g) as dg:
+                dg.set_tuning(knob, value)
+                for s in (0, g.num_nodes // 3):
+                    ref = oracle.sssp_dijkstra(g.index, g.neighbors, g.weights, s)
+                    for delta in (max(1, top // 8), top, 0):
+                        dg.set_tuning("sssp.delta", delta)
+                        for direction in (0, 2, 1):
+                            r = hc.sssp(dg, s, direction=direction)
+                            assert np.array_equal(r.values, ref), (top, delta, direction)
+                            modes = {e["mode"] for e in hc.epoch_trace(dg, "sssp")}
+                            buckets = delta > 0 and direction != 1
+                            assert ("promote" in modes) == (buckets and int(
+                                (ref < hc.INF_DIST).sum() and ref[ref < hc.INF_DIST].max()) >= delta)
+                            if buckets:
+                                assert r.stats["pull_epochs"] == 0
+
+
+def test_default_buckets_without_the_copy(hc, gpu):
+    """A flat graph of more than 2^24 edges has buckets by default on the plain
+    CSR as well, a smaller one does not."""
+    for degree, buckets in ((9, True), (7, False)):
+        g = hc.HostGraph.generate("uniform", 20, degree, weighted=True, seed=3)
+        assert (g.num_edges >= 1 << 24) == buckets
+        with hc.DeviceGraph(g) as dg:
+            s = int(g.pick_sources(1)[0])
+            ref = hc.sssp(dg, s).values
+            dg.set_tuning("sssp.sorted", 0)
+            assert np.array_equal(hc.sssp(dg, s).values, ref)
+            assert ("promote" in {e["mode"] for e in hc.epoch_trace(dg, "sssp")}) == buckets
+
+
 @pytest.mark.parametrize("max_weight,delta", [(0, -1), (255, -1), (255, 40), (70000, 9000)])
 @pytest.mark.parametrize("seed", [0, 1])
 def test_batched_sweeps_exact(hc, gpu, oracle, max_weight, delta, seed):
