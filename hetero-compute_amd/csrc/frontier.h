@@ -88,28 +88,28 @@ struct StepCtl {
     // cannot beat the row's distance from it, are not looked at).
     int32_t low;
     int32_t sorted;                // SSSP: sweeps run on the weight-sorted adjacency
-    // SSSP buckets (delta > 0) there: the current bucket holds the distances in
-    // [base, thresh).  Its push epochs (or, from a heavy frontier, sweeps over
-    // the rows: a promotion epoch with settle 3) relax the edges that land in
-    // it; when a frontier comes out empty, the bucket's distances are final
-    // and its remaining edges are settled, by a push from its vertices
-    // (settle 2) or by a sweep over the rows above it (a promotion epoch with
-    // settle 1), and a promotion epoch makes the vertices of the next bucket
-    // the frontier.
+    // SSSP buckets (delta > 0): the current bucket holds the distances in
+    // [base, thresh); everything below is final and its edges are relaxed.
+    // A light bucket (far_on; all of them on the plain CSR) relaxes every edge
+    // of its vertices at once, by pushes, and a vertex lowered to thresh or
+    // more joins the far bitmap; a promotion epoch takes the next bucket from
+    // there.  A heavy one, on the weight-sorted adjacency, relaxes the edges
+    // that land in it, by pushes or (from a heavy frontier) sweeps over the
+    // rows, a promotion epoch with settle 3; when its frontier comes out empty
+    // its other edges are settled by a push from its vertices (settle 2) or by
+    // a sweep over the rows above it, which takes the next bucket as well (a
+    // promotion epoch with settle 1), and after a push the next bucket is taken
+    // by a scan of the distances (settle 4: the scan also sets the far bitmap,
+    // for light buckets from here on).
     int32_t base;
     int32_t thresh;
     int32_t delta;
     int32_t settle;
     int32_t promotions;            // promotion epochs run
+    int32_t far_on;
     long long bucket_e;            // degree sum of this bucket's frontiers
     long long done_e;              // and of the buckets before it
-    // Buckets on the plain CSR (push epochs only): a vertex lowered to a value
-    // at or above thresh goes to the far bitmap instead of the next frontier;
-    // when a frontier comes out empty thresh rises (by delta, doubled after a
-    // promotion that found nothing) and a promotion epoch makes the far
-    // vertices now below it the frontier.
-    int32_t far_step;              // the last rise of thresh
-    int32_t far_pad;
+    long long prev_e, prev2_e;     // and of the last and last but one that were not empty
     long long far_live;            // upper bound of the far vertices
     // Device wall clock (constant rate): start of the loop, end of the last
     // epoch, and end of each traced epoch.
@@ -151,7 +151,7 @@ struct FrontierBufs {
     int32_t *q[2][3];
     HubChunk *ch[2];
     uint32_t *bm[3];
-    uint32_t *far;             // SSSP buckets on the plain CSR: vertices waiting
+    uint32_t *far;             // SSSP buckets: vertices waiting for a later one
     uint32_t (*cnt)[5];        // queue fill [parity][q0, q1, q2, chunks, hubs]
     int32_t words;             // bitmap words
     Partials part;             // counter set of the current epoch

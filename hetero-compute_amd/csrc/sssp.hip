@@ -323,8 +323,8 @@ constexpr int kPushTrip = 4;  // edges a lane of a push epoch has in flight
 // edge in flight per lane they would want a wavefront from 17 edges on.
 constexpr int32_t kPushMid = 64;
 
-// Edges of a push epoch: the CSR's two arrays (FAR: with buckets), or the
-// weight-sorted pairs.
+// Edges of a push epoch: the CSR's two arrays, or the weight-sorted pairs (FAR:
+// with buckets).
 template <typename OffT, bool FAR = false>
 struct CsrEdges {
     static constexpr bool kSorted = false, kFar = FAR;
@@ -332,9 +332,9 @@ struct CsrEdges {
     __device__ __forceinline__ int2 get(OffT i) const { return int2{adj[i], wt[i]}; }
     __device__ __forceinline__ int32_t floor(int32_t) const { return 0; }
 };
-template <typename OffT>
+template <typename OffT, bool FAR>
 struct SortedEdges {
-    static constexpr bool kSorted = true, kFar = false;
+    static constexpr bool kSorted = true, kFar = FAR;
     SortedView v;
     __device__ __forceinline__ int2 get(OffT i) const { return v.e[i]; }
     __device__ __forceinline__ int32_t floor(int32_t w) const { return v.floor(w); }
@@ -343,11 +343,10 @@ struct SortedEdges {
 // Relaxes the out-edges [b, e) of u (G lanes, kPushTrip edges a lane in
 // flight: a trip is a chain of dependent accesses -- pair, distance, minimum,
 // staging slot -- and its latency bounds the epoch); a lowered neighbour joins
-// the next frontier.  Sorted edges: only those that land below `thresh` are
-// relaxed (buckets; HC_INF_DIST: all), and the scan stops at the first key
-// that cannot.  Buckets on the CSR: a neighbour lowered to thresh or more joins
-// the far bitmap instead (`nfar` counts those settings).  `lowest` is the
-// smallest value written.
+// the next frontier.  Sorted edges: only those that land below `reach` are
+// relaxed (HC_INF_DIST: all), and the scan stops at the first key that cannot.
+// Buckets: a neighbour lowered to `thresh` or more joins the far bitmap instead
+// (`nfar` counts those settings).  `lowest` is the smallest value written.
 template <int G, typename ER, typename OffT>
 __device__ __forceinline__ void push_range(const GraphView<OffT> &g, const ER &er,
                                            int32_t *__restrict__ dist,
@@ -355,10 +354,9 @@ __device__ __forceinline__ void push_range(const GraphView<OffT> &g, const ER &e
                                            const PushOut &out,
                                            int nxt, uint32_t *wbm, int32_t u, OffT b,
                                            OffT e, int lane, uint32_t &cnt,
-                                           unsigned long long &edges_acc, int32_t thresh,
-                                           int32_t &lowest, uint32_t &nfar) {
+                                           unsigned long long &edges_acc, int32_t reach,
+                                           int32_t thresh, int32_t &lowest, uint32_t &nfar) {
     const int32_t du = dist[u];
-    const int32_t reach = ER::kSorted ? thresh : HC_INF_DIST;
     for (OffT i = b + OffT(lane); i < e; i += OffT(kPushTrip * G)) {
         int2 x[kPushTrip];
         bool in[kPushTrip];
@@ -414,7 +412,8 @@ __device__ __forceinline__ void sssp_push_sweep(const GraphView<OffT> &g, const 
                                 int nxt, uint32_t *wbm, uint32_t &cnt,
                                 unsigned long long &edges_acc, int32_t &lowest,
                                 uint32_t &nfar) {
-    const int32_t thresh = ctl->thresh;
+    const int32_t thresh = ER::kFar ? ctl->thresh : HC_INF_DIST;
+    const int32_t reach = ER::kSorted && !ctl->far_on ? thresh : HC_INF_DIST;
     const uint32_t nch = fb.cnt[cur][3], n0 = fb.cnt[cur][0],
                    n1 = fb.cnt[cur][1], n2 = fb.cnt[cur][2];
     const uint32_t u1 = nch + n0;
@@ -431,17 +430,17 @@ __device__ __forceinline__ void sssp_push_sweep(const GraphView<OffT> &g, const 
         if (unit < nch) {
             HubChunk h = fb.ch[cur][unit];
             push_range<kBlock>(g, er, dist, fb, ctl, out, nxt, wbm, h.u, OffT(h.b), OffT(h.e),
-                               threadIdx.x, cnt, edges_acc, thresh, lowest, nfar);
+                               threadIdx.x, cnt, edges_acc, reach, thresh, lowest, nfar);
         } else if (unit < u1) {
             int32_t u = fb.q[cur][0][unit - nch];
             push_range<kBlock>(g, er, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u), g.rend(u),
-                               threadIdx.x, cnt, edges_acc, thresh, lowest, nfar);
+                               threadIdx.x, cnt, edges_acc, reach, thresh, lowest, nfar);
         } else if (unit < u2) {
             uint32_t idx = (unit - u1) * kWavesPerBlock + threadIdx.x / kWave;
             if (idx < n1) {
                 int32_t u = fb.q[cur][1][idx];
                 push_range<kWave>(g, er, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u), g.rend(u),
-                                  lane_id(), cnt, edges_acc, thresh, lowest, nfar);
+                                  lane_id(), cnt, edges_acc, reach, thresh, lowest, nfar);
             }
         } else {
             uint32_t idx = (unit - u2) * kSmallPerUnit + threadIdx.x / kSmallLanes;
@@ -449,39 +448,8 @@ __device__ __forceinline__ void sssp_push_sweep(const GraphView<OffT> &g, const 
                 int32_t u = fb.q[cur][2][idx];
                 push_range<kSmallLanes>(g, er, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u),
                                         g.rend(u), threadIdx.x % kSmallLanes, cnt,
-                                        edges_acc, thresh, lowest, nfar);
+                                        edges_acc, reach, thresh, lowest, nfar);
             }
-        }
-    }
-}
-
-// Promotion epoch of the buckets on the CSR: every far vertex whose distance is
-// now below `thresh` leaves the far bitmap and is set in the changed bitmap
-// `wbm` (compacted into the next frontier's queues by the launch after);
-// `left` counts the vertices still far.  A thread owns one word of both
-// bitmaps.
-template <typename OffT>
-__device__ __forceinline__ void promote_far(const GraphView<OffT> &g, const int32_t *dist,
-                                            const FrontierBufs &fb, int32_t thresh, uint32_t *wbm,
-                                            uint32_t &cnt, unsigned long long &edges_acc,
-                                            uint32_t &left) {
-    for (int w = blockIdx.x * kBlock + threadIdx.x; w < fb.words; w += gridDim.x * kBlock) {
-        const uint32_t word = fb.far[w];
-        uint32_t now = 0;
-        for (uint32_t x = word; x; x &= x - 1) {
-            const int b = __ffs(x) - 1;
-            const int32_t v = w * 32 + b;
-            if (dist[v] < thresh) {
-                now |= 1u << b;
-                cnt++;
-                edges_acc += (unsigned long long)(g.rend(v) - g.rbeg(v));
-            } else {
-                left++;
-            }
-        }
-        if (now) {
-            fb.far[w] = word & ~now;
-            wbm[w] = now;  // cleared by the launch before; no other writer
         }
     }
 }
@@ -501,6 +469,14 @@ constexpr long long kSettleShare = 2;
 // Within a bucket, a frontier of more than m / kBucketSweep edges is relaxed
 // by a sweep over the rows instead of a push.
 constexpr long long kBucketSweep = 8;
+// A bucket whose frontiers hold more than kLightEdges + n / 8 edges is heavy: it
+// is worth two or three passes over the vertices and their launches, which a
+// light one is not (3D grid of 256^3 vertices, weights 1..3, about 500 buckets:
+// 30.9 ms with the limit at kLightEdges + n / 32, 16.6 at n / 8, 36.2 with
+// none light).  On graphs without locality a bucket holds up to forty times as
+// many as the one before it, and most of the last light one's edges are relaxed
+// for nothing (uniform, 8M vertices: 40 us), so growth counts.
+constexpr long long kLightEdges = 1ll << 18;
 
 // What a sorted sweep does with a row.
 enum RowJob {
@@ -515,8 +491,9 @@ struct RowSums {
     uint32_t cnt = 0;                  // rows put into the next frontier
     unsigned long long edges = 0;      // and their degree sum
     uint32_t gathered = 0;             // edges relaxed
-    uint32_t left = 0;                 // kRowSettle: rows reached and left at or above thresh
-    int32_t lowest = HC_INF_DIST;      // smallest value written (kRowSettle: left at or above thresh)
+    uint32_t left = 0;                 // promotions: rows reached and left at or above thresh;
+                                       // pushes: settings of the far bitmap
+    int32_t lowest = HC_INF_DIST;      // smallest value written (promotions: left at or above thresh)
 };
 
 // One trip of sorted_row_min: R edges a lane from edge i.  False when the
@@ -823,11 +800,45 @@ __device__ __forceinline__ void sorted_sweep(const PlanDev &p, const RowBounds &
     }
 }
 
-// Promotion without a settling sweep: the vertices in [base, thresh) become
-// the frontier.  A wavefront owns two words of the bitmap.
+// Promotion from the far bitmap: the far vertices in the new bucket [base, thresh)
+// become the frontier (bits of `wbm`, compacted into its queues by the launch
+// after), and those below it leave the bitmap, since they were lowered into an
+// earlier bucket meanwhile and relaxed there.  A thread owns one word of both
+// bitmaps.
 template <typename OffT>
-__device__ __forceinline__ void promote_scan(const RowBounds &ct, const GraphView<OffT> &g, const int32_t *dist,
-                             uint32_t *wbm, RowSums &s) {
+__device__ __forceinline__ void promote_far(const RowBounds &ct, const GraphView<OffT> &g,
+                                            const int32_t *dist, uint32_t *far, int32_t words,
+                                            uint32_t *wbm, RowSums &s) {
+    for (int w = blockIdx.x * kBlock + threadIdx.x; w < words; w += gridDim.x * kBlock) {
+        const uint32_t word = far[w];
+        uint32_t gone = 0, now = 0;
+        for (uint32_t x = word; x; x &= x - 1) {
+            const int b = __ffs(x) - 1;
+            const int32_t v = w * 32 + b;
+            const int32_t d = dist[v];
+            if (d >= ct.thresh) {
+                s.left++;
+                s.lowest = min(s.lowest, d);
+                continue;
+            }
+            gone |= 1u << b;
+            if (d < ct.base) continue;
+            now |= 1u << b;
+            s.cnt++;
+            s.edges += (unsigned long long)(g.rend(v) - g.rbeg(v));
+        }
+        if (gone) far[w] = word & ~gone;
+        if (now) wbm[w] = now;  // cleared by the launch before; no other writer
+    }
+}
+
+// Promotion by a scan: the vertices in [base, thresh) become the frontier, and
+// with `far` (or nullptr) those above it its bitmap.  A wavefront owns two words
+// of the bitmaps.
+template <typename OffT>
+__device__ __forceinline__ void promote_scan(const RowBounds &ct, const GraphView<OffT> &g,
+                                             const int32_t *dist, uint32_t *far, uint32_t *wbm,
+                                             RowSums &s) {
     const int64_t stride = (int64_t)gridDim.x * kBlock;
     for (int64_t i0 = (int64_t)blockIdx.x * kBlock; i0 < g.n; i0 += stride) {
         const int64_t i = i0 + threadIdx.x;
@@ -835,13 +846,19 @@ __device__ __forceinline__ void promote_scan(const RowBounds &ct, const GraphVie
         const int32_t u = (int32_t)(in ? i : 0);
         const int32_t d = in ? dist[u] : HC_INF_DIST;
         const bool hit = in && d >= ct.base && d < ct.thresh;
+        const bool later = d >= ct.thresh && d < HC_INF_DIST;
         const uint64_t m = __ballot(hit);
         if (hit) {
             s.cnt++;
             s.edges += (unsigned long long)(g.rend(u) - g.rbeg(u));
-        } else if (d >= ct.thresh && d < HC_INF_DIST) {
+        } else if (later) {
             s.left++;
             s.lowest = min(s.lowest, d);
+        }
+        if (far) {
+            const uint64_t f = __ballot(later);
+            if (in && lane_id() == 0) far[u >> 5] = uint32_t(f);
+            if (in && lane_id() == 32) far[u >> 5] = uint32_t(f >> 32);
         }
         // (the epoch before cleared the bitmap)
         if (lane_id() == 0 && uint32_t(m)) wbm[u >> 5] = uint32_t(m);
@@ -930,7 +947,26 @@ __global__ __launch_bounds__(kBlock) void sssp_step_kernel(
     write_partials(fb.part, cnt, eacc, gathered);
 }
 
-// The step of the buckets on the CSR: push and promotion epochs.
+// `left` and `lowest` of a workgroup, cleared by thread 0 before a barrier.
+struct RowSumsLds {
+    uint32_t left;
+    int32_t lowest;
+    __device__ __forceinline__ void clear() {
+        left = 0;
+        lowest = HC_INF_DIST;
+    }
+};
+
+__device__ __forceinline__ void write_row_sums(const Partials &part, const RowSums &s,
+                                               RowSumsLds &lds) {
+    if (s.left) atomicAdd(&lds.left, s.left);
+    if (s.lowest < HC_INF_DIST) atomicMin(&lds.lowest, s.lowest);
+    __syncthreads();
+    write_partials(part, s.cnt, s.edges, s.gathered, lds.left, 0,
+                   (unsigned long long)(HC_INF_DIST - lds.lowest));
+}
+
+// The step of the buckets on the plain CSR: push and promotion epochs.
 template <typename OffT>
 __global__ __launch_bounds__(kBlock) void sssp_near_far_kernel(GraphView<OffT> g,
                                                                int32_t *__restrict__ dist,
@@ -939,6 +975,7 @@ __global__ __launch_bounds__(kBlock) void sssp_near_far_kernel(GraphView<OffT> g
                                                                int defer_dedup) {
     extern __shared__ int32_t s_stage[];
     __shared__ uint32_t s_out;
+    __shared__ RowSumsLds s_sums;
     if (ctl->done) return;
     const int k = ctl->epoch;
     const int cur = k & 1, nxt = cur ^ 1;
@@ -946,23 +983,24 @@ __global__ __launch_bounds__(kBlock) void sssp_near_far_kernel(GraphView<OffT> g
     uint32_t *cbm = fb.bm[(k + 2) % 3];
     for (int w = blockIdx.x * kBlock + threadIdx.x; w < fb.words; w += gridDim.x * kBlock)
         cbm[w] = 0;
-    // `nfar`: far settings of a push, vertices left far by a promotion.
-    uint32_t cnt = 0, nfar = 0;
-    unsigned long long eacc = 0;
-    if (ctl->mode == kPromote) {
-        promote_far(g, dist, fb, ctl->thresh, wbm, cnt, eacc, nfar);
-    } else {
-        if (threadIdx.x == 0) s_out = 0;
-        __syncthreads();
-        const PushOut out{s_stage, &s_out, (uint32_t)push_cap, defer_dedup ? wbm : nullptr};
-        int32_t lowest = HC_INF_DIST;
-        sssp_push_sweep(g, CsrEdges<OffT, true>{g.adj, g.wt}, dist, fb, ctl, out, cur, nxt, wbm,
-                        cnt, eacc, lowest, nfar);
-        const PushKept kept = push_out_flush(out, g, fb, ctl, nxt);
-        cnt += kept.n;
-        eacc += kept.e;
+    if (threadIdx.x == 0) {
+        s_out = 0;
+        s_sums.clear();
     }
-    write_partials(fb.part, cnt, eacc, nfar);
+    __syncthreads();
+    RowSums s;
+    if (ctl->mode == kPromote) {
+        const RowBounds rb{ctl->low, ctl->base, ctl->thresh};
+        promote_far(rb, g, dist, fb.far, fb.words, wbm, s);
+    } else {
+        const PushOut out{s_stage, &s_out, (uint32_t)push_cap, defer_dedup ? wbm : nullptr};
+        sssp_push_sweep(g, CsrEdges<OffT, true>{g.adj, g.wt}, dist, fb, ctl, out, cur, nxt, wbm,
+                        s.cnt, s.edges, s.lowest, s.left);
+        const PushKept kept = push_out_flush(out, g, fb, ctl, nxt);
+        s.cnt += kept.n;
+        s.edges += kept.e;
+    }
+    write_row_sums(fb.part, s, s_sums);
 }
 
 // The step on the weight-sorted adjacency (the default): pull epochs or, with
@@ -979,8 +1017,8 @@ __global__ __launch_bounds__(kBlock) void sssp_sorted_step_kernel(
     PlanDev p, GraphView<OffT> g, SortedView sv, int32_t *__restrict__ dist, FrontierBufs fb,
     StepCtl *ctl, int32_t push_cap, int defer_dedup) {
     extern __shared__ int32_t s_stage[];
-    __shared__ uint32_t s_out, s_left;
-    __shared__ int32_t s_lowest;
+    __shared__ uint32_t s_out;
+    __shared__ RowSumsLds s_sums;
     if (ctl->done) return;
     const int mode = ctl->mode;
     const int k = ctl->epoch;
@@ -991,17 +1029,15 @@ __global__ __launch_bounds__(kBlock) void sssp_sorted_step_kernel(
         cbm[w] = 0;
     if (threadIdx.x == 0) {
         s_out = 0;
-        s_left = 0;
-        s_lowest = HC_INF_DIST;
+        s_sums.clear();
     }
     __syncthreads();
     RowSums s;
     const RowBounds rb{ctl->low, ctl->base, ctl->thresh};
     if (mode == kPush && !(BUCKETS && ctl->settle)) {
         const PushOut out{s_stage, &s_out, (uint32_t)push_cap, defer_dedup ? wbm : nullptr};
-        uint32_t nfar = 0;
-        sssp_push_sweep(g, SortedEdges<OffT>{sv}, dist, fb, ctl, out, cur, nxt, wbm, s.cnt,
-                        s.edges, s.lowest, nfar);
+        sssp_push_sweep(g, SortedEdges<OffT, BUCKETS>{sv}, dist, fb, ctl, out, cur, nxt, wbm, s.cnt,
+                        s.edges, s.lowest, s.left);
         const PushKept kept = push_out_flush(out, g, fb, ctl, nxt);
         s.cnt += kept.n;
         s.edges += kept.e;
@@ -1011,20 +1047,22 @@ __global__ __launch_bounds__(kBlock) void sssp_sorted_step_kernel(
         sorted_sweep<kRowScatter>(p, rb, g, sv, dist, wbm, s);
     } else if (ctl->settle == 3) {
         sorted_sweep<kRowBucket>(p, rb, g, sv, dist, wbm, s);
-    } else if (ctl->settle) {
+    } else if (ctl->settle == 1) {
         sorted_sweep<kRowSettle>(p, rb, g, sv, dist, wbm, s);
+    } else if (ctl->far_on && ctl->settle == 0) {
+        promote_far(rb, g, dist, fb.far, fb.words, wbm, s);
     } else {
-        promote_scan(rb, g, dist, wbm, s);
+        promote_scan(rb, g, dist, ctl->settle ? fb.far : nullptr, wbm, s);
     }
-    if (s.left) atomicAdd(&s_left, s.left);
-    if (s.lowest < HC_INF_DIST) atomicMin(&s_lowest, s.lowest);
-    __syncthreads();
-    write_partials(fb.part, s.cnt, s.edges, s.gathered, s_left, 0,
-                   (unsigned long long)(HC_INF_DIST - s_lowest));
+    write_row_sums(fb.part, s, s_sums);
 }
 
 // Next bucket: the vertices in [base, base + delta) at least.
 __device__ __forceinline__ void next_bucket(StepCtl *c, int32_t base) {
+    if (c->bucket_e > 0) {
+        c->prev2_e = c->prev_e;
+        c->prev_e = c->bucket_e;
+    }
     c->base = base;
     c->thresh = (int32_t)min((long long)base + c->delta, (long long)HC_INF_DIST);
     c->bucket_e = 0;
@@ -1040,11 +1078,11 @@ __device__ void sssp_decide(StepCtl *c, StepCtl *trace,
     const int k = c->epoch;
     const int ran = c->mode;
     const int settled = c->settle;
-    if (ran == kPromote && !c->sorted) {
+    if (ran == kPromote && c->far_on && settled == 0) {
         // far bitmap words, plus dist[v] and a bitmap entry per far vertex
-        c->alg_bytes += 4ull * (unsigned long long)((c->n + 31) / 32) + 8ull * (out_n + gathered);
+        c->alg_bytes += 4ull * (unsigned long long)((c->n + 31) / 32) + 8ull * (out_n + left);
         c->promotions++;
-        c->far_live = (long long)gathered;
+        c->far_live = (long long)left;
         trace_epoch(c, trace, k, ran, out_n, out_e, 0);
     } else if (ran == kPromote) {
         // dist per vertex; pair + gathered distance per relaxed edge and
@@ -1052,6 +1090,7 @@ __device__ void sssp_decide(StepCtl *c, StepCtl *trace,
         c->alg_bytes += (settled ? 8ull : 4ull) * (unsigned long long)c->n + 12ull * gathered +
                         8ull * out_n;
         c->promotions++;
+        c->far_live = (long long)left;
         trace_epoch(c, trace, k, ran, out_n, out_e, gathered);
     } else if (ran == kPush) {
         // offsets + dist[u] per frontier vertex; id + weight + dist[v] per
@@ -1064,7 +1103,7 @@ __device__ void sssp_decide(StepCtl *c, StepCtl *trace,
             trace_epoch(c, trace, k, ran, out_n, out_e, c->in_e);
         }
         c->push_epochs++;
-        if (!c->sorted) c->far_live += (long long)gathered;  // may repeat a vertex
+        c->far_live += (long long)left;  // far settings (may repeat a vertex)
     } else if (c->sorted) {
         // Offsets and own distances; id + weight + distance per edge relaxed.
         c->alg_bytes += (unsigned long long)c->sweep_bytes - 12ull * (unsigned long long)c->m +
@@ -1092,27 +1131,32 @@ __device__ void sssp_decide(StepCtl *c, StepCtl *trace,
     int next = ran;
     if (c->max_epochs > 0 && k + 1 >= c->max_epochs) {
         c->done = 1;
-    } else if (c->delta > 0 && !c->sorted) {
-        if (out_n != 0) {
-            next = kPush;
-        } else if (c->far_live > 0) {
-            const long long step = ran == kPromote ? 2ll * c->far_step : (long long)c->delta;
-            c->far_step = (int32_t)min(step, (long long)HC_INF_DIST);
-            c->thresh = (int32_t)min((long long)c->thresh + step, (long long)HC_INF_DIST);
-            next = kPromote;
-        } else {
-            c->done = 1;
-        }
     } else if (c->delta > 0) {
         c->settle = 0;
+        const long long light = kLightEdges + c->n / 8;
         if (out_n != 0) {
+            // Heavy: past the limit, or about to be if it outgrows the bucket
+            // before it as that one did the one before.
+            if (c->sorted && (c->bucket_e + (long long)out_e > light ||
+                              (ran == kPromote && c->prev_e > light * c->prev2_e / c->prev_e)))
+                c->far_on = 0;
             // The bucket goes on: by a sweep of the rows above its lowest
             // pending value while the frontier is heavy, else by a push.
             c->low = ran == kPromote && settled != 3 ? c->base : lowest;
             next = kPush;
-            if (c->direction != 2 && (long long)out_e > c->m / kBucketSweep) {
+            if (!c->far_on && c->direction != 2 && (long long)out_e > c->m / kBucketSweep) {
                 c->settle = 3;
                 next = kPromote;
+            }
+        } else if (c->far_on) {
+            // The bucket is complete, or was empty: on to the next width, or
+            // to the smallest far distance.
+            c->done_e += c->bucket_e;
+            if (c->far_live == 0) {
+                c->done = 1;
+            } else {
+                next = kPromote;
+                next_bucket(c, ran == kPromote ? lowest : c->thresh);
             }
         } else if ((ran == kPush && !settled) || settled == 3) {
             // The bucket is complete.  A sweep over the rows above it costs
@@ -1132,6 +1176,10 @@ __device__ void sssp_decide(StepCtl *c, StepCtl *trace,
                 next = kPush;
             }
         } else if (ran == kPush) {
+            if (c->bucket_e < light / 4) {
+                c->settle = 4;
+                c->far_on = 1;
+            }
             next = kPromote;
             next_bucket(c, c->thresh);
         } else if (left != 0) {
@@ -1247,7 +1295,8 @@ __global__ __launch_bounds__(kBlock) void sssp_init_kernel(
         ctl->promotions = 0;
         ctl->bucket_e = 0;
         ctl->done_e = 0;
-        ctl->far_step = delta;
+        ctl->prev_e = ctl->prev2_e = m > 0 ? m : 1;
+        ctl->far_on = delta > 0;
         ctl->far_live = 0;
         ctl->reached = 0;
         ctl->alg_bytes = 0;

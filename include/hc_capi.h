@@ -292,17 +292,15 @@ int hc_graph_get_info(hc_graph_t g, hc_graph_info_t *out);
  *                          largest weight / mean degree on flat graphs, off
  *                          on skewed ones.  Results do not depend on it
  *   sssp.delta             hc_sssp: distances become final in buckets of this
- *                          width.  On the weight-sorted adjacency push epochs
- *                          relax only the edges that land in the current
- *                          bucket, and a promotion epoch settles the bucket's
- *                          other edges and starts the next one; on the plain
- *                          CSR (no pulls then) vertices lowered past the bucket
- *                          wait in a far set, from which a promotion epoch
- *                          takes the next one.  0 off; -1 (default) 4 x the
- *                          graph's sampled largest weight / mean degree on
- *                          flat graphs (2 x on the plain CSR, from 2^24 edges),
- *                          off on skewed ones and with direction 1.  Results
- *                          do not depend on it
+ *                          width.  Vertices lowered past the bucket wait in a
+ *                          far set, from which a promotion epoch takes the
+ *                          next one (no pulls); on the weight-sorted adjacency
+ *                          a bucket of many edges relaxes only those that land
+ *                          in it and settles the others at its end.  0 off;
+ *                          -1 (default) 4 x the graph's sampled largest weight
+ *                          / mean degree on flat graphs (2 x on the plain CSR,
+ *                          from 2^24 edges), off on skewed ones and with
+ *                          direction 1.  Results do not depend on it
  *   multi.push_div         batched sweep: an epoch whose flagged vertices
  *                          hold at most m / this edges (none more than
  *                          1024) pushes from them with atomicMin instead of

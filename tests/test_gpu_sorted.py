@@ -123,6 +123,36 @@ def test_flat_buckets_cover_every_settling_path(hc, gpu, oracle):
                     assert np.array_equal(hc.sssp(dg, s, direction=2).values, ref), (top, delta)
 
 
+@pytest.mark.parametrize("top", [3, 255, 100000])
+def test_buckets_turn_light_and_heavy(hc, gpu, oracle, top):
+    """Two dense cores joined by a long path, with a tail and unreached vertices
+    behind: buckets start light (the far set), turn heavy in a core (scans and
+    sweeps), light again on the path, and heavy in the second core."""
+    rng = np.random.default_rng(top)
+    core, path = 12000, 600
+    src, dst = [], []
+    for base in (0, core + path):
+        src.append(base + rng.integers(0, core, 10 * core))
+        dst.append(base + rng.integers(0, core, 10 * core))
+    for first in (core - 1, 2 * core + path - 1):
+        src.append(first + np.arange(path))
+        dst.append(first + 1 + np.arange(path))
+    src, dst = np.concatenate(src), np.concatenate(dst)
+    n = 2 * (core + path) + 500
+    w = rng.integers(1, top + 1, src.size).astype(np.int32)
+    for relabel in (False, True):
+        g = hc.HostGraph.from_edges(src.astype(np.int32), dst.astype(np.int32), n, weights=w,
+                                    relabel=relabel)
+        with hc.DeviceGraph(g) as dg:
+            for s in (0, int(g.pick_sources(1)[0]), n // 2):
+                ref = oracle.sssp_dijkstra(g.index, g.neighbors, g.weights, s)
+                for delta in (-1, max(1, top // 20), top, 20 * top):
+                    dg.set_tuning("sssp.delta", delta)
+                    for direction in (0, 2):
+                        got = hc.sssp(dg, s, direction=direction).values
+                        assert np.array_equal(got, ref), (s, delta, direction)
+
+
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("knob,value", [("sssp.sorted", 0), ("sssp.filter", 1), ("sssp.dist16", 1),
                                         ("pull.col_shift", 10)])
