@@ -542,10 +542,10 @@ struct SortedView {
         return (k < kSortKeys - 1 ? k : kSortKeys - 1) << shift;
     }
 };
-// One copy for a graph and every share of it, built on first use.
+// One copy for a graph and every share of it, built on first use (and tried
+// again on the next one where there was no memory for it).
 struct SortedSlot {
     std::mutex mu;
-    bool tried = false;
     SortedAdj adj;
     ~SortedSlot();
 };

@@ -266,11 +266,9 @@ int get_sorted(hc_graph_s *g, hipStream_t s, SortedView *out) {
         return HC_OK;
     SortedSlot &slot = *g->sortslot;
     std::lock_guard<std::mutex> lk(slot.mu);
-    if (!slot.tried) {
+    if (!slot.adj.e)
         HC_TRY(g->off64 ? build_sorted<uint64_t>(g, s, &slot.adj)
                         : build_sorted<uint32_t>(g, s, &slot.adj));
-        slot.tried = true;
-    }
     *out = SortedView{slot.adj.e, slot.adj.shift};
     return HC_OK;
 }

@@ -200,6 +200,31 @@ def test_default_buckets_without_the_copy(hc, gpu):
             assert ("promote" in {e["mode"] for e in hc.epoch_trace(dg, "sssp")}) == buckets
 
 
+def test_copy_is_built_once_there_is_memory(hc, gpu):
+    """With the device's memory taken the queries run on the plain CSR; the first
+    one after it is given back builds the copy."""
+    g = hc.HostGraph.generate("uniform", 19, 16, weighted=True, seed=6)
+    s = int(g.pick_sources(1)[0])
+    with hc.DeviceGraph(g) as dg:
+        dg.set_tuning("sssp.sorted", 0)
+        ref = hc.sssp(dg, s).values
+        dg.reset_tuning()
+        hold = []
+        try:
+            while (free := hc.mem_get_info()[0]) > 96 << 20:
+                hold.append(hc.DeviceArray(min(free - (64 << 20), 8 << 30) // 4, np.int32))
+            print("held", sum(a.nbytes for a in hold) >> 20, "MiB", flush=True)
+            short = hc.mem_get_info()[0]
+            assert np.array_equal(hc.sssp(dg, s).values, ref)
+            assert short - hc.mem_get_info()[0] < 8 * g.num_edges
+        finally:
+            for a in hold:
+                a.free()
+        free = hc.mem_get_info()[0]
+        assert np.array_equal(hc.sssp(dg, s).values, ref)
+        assert free - hc.mem_get_info()[0] >= 8 * g.num_edges
+
+
 @pytest.mark.parametrize("max_weight,delta", [(0, -1), (255, -1), (255, 40), (70000, 9000)])
 @pytest.mark.parametrize("seed", [0, 1])
 def test_batched_sweeps_exact(hc, gpu, oracle, max_weight, delta, seed):
