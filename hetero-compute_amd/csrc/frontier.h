@@ -436,7 +436,9 @@ __device__ __forceinline__ void write_source_chunks(const GraphView<OffT> &g,
 
 // Workgroup sums of three per-thread counters plus three per-workgroup values
 // (x, y: added, z: maximum; taken from thread 0), put into this workgroup's
-// counter group.
+// counter group.  TWO: s holds two counters of 32 bits, also for the whole
+// workgroup, the upper one for y.
+template <bool TWO = false>
 __device__ __forceinline__ void write_partials(const Partials &part, uint32_t n,
                                                unsigned long long e,
                                                unsigned long long s,
@@ -464,6 +466,10 @@ __device__ __forceinline__ void write_partials(const Partials &part, uint32_t n,
             v[0] += s_n[i];
             v[1] += s_e[i];
             v[2] += s_s[i];
+        }
+        if (TWO) {
+            v[4] = v[2] >> 32;
+            v[2] &= 0xffffffffull;
         }
         unsigned long long *g = part.acc + (blockIdx.x % kSumGroups) * kSumStride;
         for (int k = 0; k < kMaxSlot; k++)

@@ -346,7 +346,9 @@ struct SortedEdges {
 // the next frontier.  Sorted edges: only those that land below `reach` are
 // relaxed (HC_INF_DIST: all), and the scan stops at the first key that cannot.
 // Buckets: a neighbour lowered to `thresh` or more joins the far bitmap instead
-// (`nfar` counts those settings).  `lowest` is the smallest value written.
+// (`nfar` counts those settings).  `lowest` is the smallest value written;
+// `pairs` and `gathered` count the edges and distances read where the scan may
+// stop early.
 template <int G, typename ER, typename OffT>
 __device__ __forceinline__ void push_range(const GraphView<OffT> &g, const ER &er,
                                            int32_t *__restrict__ dist,
@@ -355,7 +357,8 @@ __device__ __forceinline__ void push_range(const GraphView<OffT> &g, const ER &e
                                            int nxt, uint32_t *wbm, int32_t u, OffT b,
                                            OffT e, int lane, uint32_t &cnt,
                                            unsigned long long &edges_acc, int32_t reach,
-                                           int32_t thresh, int32_t &lowest, uint32_t &nfar) {
+                                           int32_t thresh, int32_t &lowest, uint32_t &nfar,
+                                           uint32_t &pairs, uint32_t &gathered) {
     const int32_t du = dist[u];
     for (OffT i = b + OffT(lane); i < e; i += OffT(kPushTrip * G)) {
         int2 x[kPushTrip];
@@ -366,12 +369,14 @@ __device__ __forceinline__ void push_range(const GraphView<OffT> &g, const ER &e
             in[r] = k < e;
             x[r] = in[r] ? er.get(k) : int2{0, 0};
         }
+        if (ER::kSorted && ER::kFar) pairs += (uint32_t)min((e - 1 - i) / OffT(G) + 1, OffT(kPushTrip));
         if (ER::kSorted && relax(du, er.floor(x[0].y)) >= reach) break;
         int32_t nd[kPushTrip], d[kPushTrip], old[kPushTrip];
 #pragma unroll
         for (int r = 0; r < kPushTrip; r++) {
             nd[r] = in[r] ? relax(du, x[r].y) : HC_INF_DIST;
             d[r] = nd[r] < reach ? dist[x[r].x] : 0;
+            if (ER::kSorted && ER::kFar) gathered += nd[r] < reach ? 1u : 0u;
         }
 #pragma unroll
         for (int r = 0; r < kPushTrip; r++)
@@ -411,7 +416,7 @@ __device__ __forceinline__ void sssp_push_sweep(const GraphView<OffT> &g, const 
                                 const PushOut &out, int cur,
                                 int nxt, uint32_t *wbm, uint32_t &cnt,
                                 unsigned long long &edges_acc, int32_t &lowest,
-                                uint32_t &nfar) {
+                                uint32_t &nfar, uint32_t &pairs, uint32_t &gathered) {
     const int32_t thresh = ER::kFar ? ctl->thresh : HC_INF_DIST;
     const int32_t reach = ER::kSorted && !ctl->far_on ? thresh : HC_INF_DIST;
     const uint32_t nch = fb.cnt[cur][3], n0 = fb.cnt[cur][0],
@@ -430,17 +435,20 @@ __device__ __forceinline__ void sssp_push_sweep(const GraphView<OffT> &g, const 
         if (unit < nch) {
             HubChunk h = fb.ch[cur][unit];
             push_range<kBlock>(g, er, dist, fb, ctl, out, nxt, wbm, h.u, OffT(h.b), OffT(h.e),
-                               threadIdx.x, cnt, edges_acc, reach, thresh, lowest, nfar);
+                               threadIdx.x, cnt, edges_acc, reach, thresh, lowest, nfar,
+                               pairs, gathered);
         } else if (unit < u1) {
             int32_t u = fb.q[cur][0][unit - nch];
             push_range<kBlock>(g, er, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u), g.rend(u),
-                               threadIdx.x, cnt, edges_acc, reach, thresh, lowest, nfar);
+                               threadIdx.x, cnt, edges_acc, reach, thresh, lowest, nfar,
+                               pairs, gathered);
         } else if (unit < u2) {
             uint32_t idx = (unit - u1) * kWavesPerBlock + threadIdx.x / kWave;
             if (idx < n1) {
                 int32_t u = fb.q[cur][1][idx];
                 push_range<kWave>(g, er, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u), g.rend(u),
-                                  lane_id(), cnt, edges_acc, reach, thresh, lowest, nfar);
+                                  lane_id(), cnt, edges_acc, reach, thresh, lowest, nfar,
+                               pairs, gathered);
             }
         } else {
             uint32_t idx = (unit - u2) * kSmallPerUnit + threadIdx.x / kSmallLanes;
@@ -448,7 +456,8 @@ __device__ __forceinline__ void sssp_push_sweep(const GraphView<OffT> &g, const 
                 int32_t u = fb.q[cur][2][idx];
                 push_range<kSmallLanes>(g, er, dist, fb, ctl, out, nxt, wbm, u, g.rbeg(u),
                                         g.rend(u), threadIdx.x % kSmallLanes, cnt,
-                                        edges_acc, reach, thresh, lowest, nfar);
+                                        edges_acc, reach, thresh, lowest, nfar,
+                               pairs, gathered);
             }
         }
     }
@@ -490,7 +499,8 @@ enum RowJob {
 struct RowSums {
     uint32_t cnt = 0;                  // rows put into the next frontier
     unsigned long long edges = 0;      // and their degree sum
-    uint32_t gathered = 0;             // edges relaxed
+    uint32_t pairs = 0;                // sorted edges read
+    uint32_t gathered = 0;             // distances read for them
     uint32_t left = 0;                 // promotions: rows reached and left at or above thresh;
                                        // pushes: settings of the far bitmap
     int32_t lowest = HC_INF_DIST;      // smallest value written (promotions: left at or above thresh)
@@ -537,13 +547,18 @@ __device__ __forceinline__ bool sorted_trip(const SortedView &sv, const int32_t 
 template <int G, typename OffT>
 __device__ __forceinline__ int32_t sorted_row_min(const SortedView &sv, const int32_t *dist,
                                                   OffT b, OffT e, int lane, int32_t cur,
-                                                  int32_t low, uint32_t &gathered) {
+                                                  int32_t low, uint32_t &pairs,
+                                                  uint32_t &gathered) {
     int32_t best = cur, m = HC_INF_DIST;
-    if (!sorted_trip<G, 2>(sv, dist, b, e, lane, low, best, m, gathered)) return m;
-    // (8-byte offsets take the registers of the longer trip)
-    constexpr int R = sizeof(OffT) == 8 ? 2 : 4;
-    for (OffT i = b + OffT(2 * G); i < e; i += OffT(R * G))
-        if (!sorted_trip<G, R>(sv, dist, i, e, lane, low, best, m, gathered)) break;
+    OffT i = b + OffT(2 * G);
+    if (sorted_trip<G, 2>(sv, dist, b, e, lane, low, best, m, gathered)) {
+        // (8-byte offsets take the registers of the longer trip)
+        constexpr int R = sizeof(OffT) == 8 ? 2 : 4;
+        bool more = true;
+        for (; more && i < e; i += OffT(R * G))
+            more = sorted_trip<G, R>(sv, dist, i, e, lane, low, best, m, gathered);
+    }
+    if (lane == 0) pairs += (uint32_t)(min(i, e) - b);
     return m;
 }
 
@@ -552,9 +567,10 @@ __device__ __forceinline__ int32_t sorted_row_min(const SortedView &sv, const in
 template <int G, typename OffT>
 __device__ __forceinline__ void scatter_row(const SortedView &sv, int32_t *dist, OffT b, OffT e,
                                             int lane, int32_t du, int32_t thresh,
-                                            uint32_t &gathered) {
+                                            uint32_t &pairs, uint32_t &gathered) {
     for (OffT i = b + OffT(lane); i < e; i += OffT(G)) {
         const int2 x = sv.e[i];
+        pairs++;
         const int32_t nd = relax(du, x.y);
         if (nd < thresh || nd >= HC_INF_DIST) continue;
         gathered++;
@@ -658,11 +674,11 @@ __device__ __forceinline__ void sorted_block(const RowHead<OffT> &h, int j0, int
     if (G == 1) {
         if (want) {
             if (JOB == kRowScatter) {
-                scatter_row<1>(sv, dist, h.b, h.e, 0, h.cur, ct.thresh, s.gathered);
+                scatter_row<1>(sv, dist, h.b, h.e, 0, h.cur, ct.thresh, s.pairs, s.gathered);
             } else {
                 const int32_t top = row_top<JOB>(ct, h.cur);
                 const int32_t m =
-                    sorted_row_min<1>(sv, dist, h.b, h.e, 0, top, ct.low, s.gathered);
+                    sorted_row_min<1>(sv, dist, h.b, h.e, 0, top, ct.low, s.pairs, s.gathered);
                 if (m < top) dist[h.u] = m;
                 hit = row_done<JOB>(ct, h.cur, top, m, (unsigned long long)(h.e - h.b), s);
             }
@@ -686,11 +702,11 @@ __device__ __forceinline__ void sorted_block(const RowHead<OffT> &h, int j0, int
             bool ghit = false;
             if (have) {
                 if (JOB == kRowScatter) {
-                    scatter_row<G>(sv, dist, b, e, lane % G, cur, ct.thresh, s.gathered);
+                    scatter_row<G>(sv, dist, b, e, lane % G, cur, ct.thresh, s.pairs, s.gathered);
                 } else {
                     const int32_t top = row_top<JOB>(ct, cur);
                     const int32_t m = sorted_row_min<G>(sv, dist, b, e, lane % G, top, ct.low,
-                                                        s.gathered);
+                                                        s.pairs, s.gathered);
                     if (SHARED) {
                         if (lane == 0) shared_done<JOB>(ct, g, dist, wbm, u, cur, top, m, s);
                     } else if (lane % G == 0) {
@@ -937,9 +953,9 @@ __global__ __launch_bounds__(kBlock) void sssp_step_kernel(
         __syncthreads();
         const PushOut out{s_stage, &s_out, (uint32_t)push_cap, defer_dedup ? wbm : nullptr};
         int32_t lowest = HC_INF_DIST;
-        uint32_t nfar = 0;
+        uint32_t nfar = 0, pairs = 0;
         sssp_push_sweep(g, CsrEdges<OffT>{g.adj, g.wt}, dist, fb, ctl, out, cur, nxt, wbm, cnt,
-                        eacc, lowest, nfar);
+                        eacc, lowest, nfar, pairs, gathered);
         const PushKept k = push_out_flush(out, g, fb, ctl, nxt);
         cnt += k.n;
         eacc += k.e;
@@ -962,8 +978,9 @@ __device__ __forceinline__ void write_row_sums(const Partials &part, const RowSu
     if (s.left) atomicAdd(&lds.left, s.left);
     if (s.lowest < HC_INF_DIST) atomicMin(&lds.lowest, s.lowest);
     __syncthreads();
-    write_partials(part, s.cnt, s.edges, s.gathered, lds.left, 0,
-                   (unsigned long long)(HC_INF_DIST - lds.lowest));
+    write_partials<true>(part, s.cnt, s.edges,
+                         (unsigned long long)s.pairs << 32 | s.gathered, lds.left, 0,
+                         (unsigned long long)(HC_INF_DIST - lds.lowest));
 }
 
 // The step of the buckets on the plain CSR: push and promotion epochs.
@@ -995,7 +1012,7 @@ __global__ __launch_bounds__(kBlock) void sssp_near_far_kernel(GraphView<OffT> g
     } else {
         const PushOut out{s_stage, &s_out, (uint32_t)push_cap, defer_dedup ? wbm : nullptr};
         sssp_push_sweep(g, CsrEdges<OffT, true>{g.adj, g.wt}, dist, fb, ctl, out, cur, nxt, wbm,
-                        s.cnt, s.edges, s.lowest, s.left);
+                        s.cnt, s.edges, s.lowest, s.left, s.pairs, s.gathered);
         const PushKept kept = push_out_flush(out, g, fb, ctl, nxt);
         s.cnt += kept.n;
         s.edges += kept.e;
@@ -1037,7 +1054,7 @@ __global__ __launch_bounds__(kBlock) void sssp_sorted_step_kernel(
     if (mode == kPush && !(BUCKETS && ctl->settle)) {
         const PushOut out{s_stage, &s_out, (uint32_t)push_cap, defer_dedup ? wbm : nullptr};
         sssp_push_sweep(g, SortedEdges<OffT, BUCKETS>{sv}, dist, fb, ctl, out, cur, nxt, wbm, s.cnt,
-                        s.edges, s.lowest, s.left);
+                        s.edges, s.lowest, s.left, s.pairs, s.gathered);
         const PushKept kept = push_out_flush(out, g, fb, ctl, nxt);
         s.cnt += kept.n;
         s.edges += kept.e;
@@ -1073,7 +1090,12 @@ __device__ __forceinline__ void next_bucket(StepCtl *c, int32_t base) {
 __device__ void sssp_decide(StepCtl *c, StepCtl *trace,
                             const unsigned long long (&sums)[kSumSlots]) {
     const unsigned long long out_n = sums[0], out_e = sums[1], gathered = sums[2];
-    const unsigned long long left = sums[3];
+    const unsigned long long left = sums[3], pairs = sums[4];
+    // Sorted sweeps: offsets and distance of every row, and the pairs and
+    // distances read.
+    const unsigned long long rows =
+        (unsigned long long)c->sweep_bytes - 12ull * (unsigned long long)c->m;
+    const unsigned long long looked = 8ull * pairs + 4ull * gathered;
     const int32_t lowest = HC_INF_DIST - (int32_t)sums[kMaxSlot];
     const int k = c->epoch;
     const int ran = c->mode;
@@ -1085,31 +1107,27 @@ __device__ void sssp_decide(StepCtl *c, StepCtl *trace,
         c->far_live = (long long)left;
         trace_epoch(c, trace, k, ran, out_n, out_e, 0);
     } else if (ran == kPromote) {
-        // dist per vertex; pair + gathered distance per relaxed edge and
-        // offsets per row of a settling sweep; a bit per frontier vertex
-        c->alg_bytes += (settled ? 8ull : 4ull) * (unsigned long long)c->n + 12ull * gathered +
-                        8ull * out_n;
+        // dist per vertex; of a settling sweep also the offsets, and pairs and
+        // distances read; a bit per frontier vertex
+        c->alg_bytes += (settled == 1 || settled == 3 ? rows : 4ull * (unsigned long long)c->n) +
+                        looked + 8ull * out_n;
         c->promotions++;
         c->far_live = (long long)left;
-        trace_epoch(c, trace, k, ran, out_n, out_e, gathered);
+        trace_epoch(c, trace, k, ran, out_n, out_e, pairs);
     } else if (ran == kPush) {
-        // offsets + dist[u] per frontier vertex; id + weight + dist[v] per
-        // edge; dist write + bitmap/queue entry per improved vertex.
-        if (settled) {
-            c->alg_bytes += 8ull * (unsigned long long)c->n + 12ull * gathered;
-            trace_epoch(c, trace, k, ran, out_n, out_e, gathered);
-        } else {
-            c->alg_bytes += 12ull * c->in_n + 12ull * c->in_e + 8ull * out_n;
-            trace_epoch(c, trace, k, ran, out_n, out_e, c->in_e);
-        }
+        // offsets + dist[u] per frontier vertex (per row when settling); id +
+        // weight + dist[v] per edge, in a heavy bucket as far as read; dist
+        // write + bitmap/queue entry per improved vertex.
+        const bool all = !c->sorted || c->delta == 0;
+        c->alg_bytes += (settled ? rows : 12ull * c->in_n) + (all ? 12ull * c->in_e : looked) +
+                        8ull * out_n;
+        trace_epoch(c, trace, k, ran, out_n, out_e, all ? (unsigned long long)c->in_e : pairs);
         c->push_epochs++;
         c->far_live += (long long)left;  // far settings (may repeat a vertex)
     } else if (c->sorted) {
-        // Offsets and own distances; id + weight + distance per edge relaxed.
-        c->alg_bytes += (unsigned long long)c->sweep_bytes - 12ull * (unsigned long long)c->m +
-                        12ull * gathered + 8ull * out_n;
+        c->alg_bytes += rows + looked + 8ull * out_n;
         c->pull_epochs++;
-        trace_epoch(c, trace, k, ran, out_n, out_e, gathered);
+        trace_epoch(c, trace, k, ran, out_n, out_e, pairs);
     } else {
         // Offsets, ids and own distances always; weight + distance per
         // gathered edge; one bit per tested neighbour when filtering.

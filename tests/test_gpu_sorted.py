@@ -200,6 +200,31 @@ def test_default_buckets_without_the_copy(hc, gpu):
             assert ("promote" in {e["mode"] for e in hc.epoch_trace(dg, "sssp")}) == buckets
 
 
+def test_sorted_sweeps_count_what_they_read(hc, gpu):
+    """The trace and the byte count hold the pairs read, whether or not a distance
+    is read for them: a star whose leaves lie at 1..200 is read once to lower the
+    leaves and once more, but for the lightest, to find nothing; a heavy bucket's
+    pushes read part of their frontier's edges."""
+    d = 200
+    g = hc.HostGraph.from_edges(np.zeros(d, np.int32), 1 + np.arange(d, dtype=np.int32), d + 1,
+                                weights=1 + np.arange(d, dtype=np.int32))
+    with hc.DeviceGraph(g) as dg:
+        r = hc.sssp(dg, 0, direction=1)
+        tr = hc.epoch_trace(dg, "sssp")
+        assert [(e["frontier"], e["scanned"]) for e in tr] == [(d, d), (0, d - 1)]
+        rows = 4 * (d + 2) + 4 * (d + 1)
+        assert r.stats["alg_bytes"] == 2 * rows + 8 * (2 * d - 1) + 4 * d + 8 * d
+    g = hc.HostGraph.generate("uniform", 16, 24, weighted=True, seed=2)
+    with hc.DeviceGraph(g) as dg:
+        dg.set_tuning("sssp.delta", 16)
+        hc.sssp(dg, int(g.pick_sources(1)[0]))
+        tr = hc.epoch_trace(dg, "sssp")
+        pushes = [(e["scanned"], p["frontier_edges"]) for p, e in zip(tr, tr[1:])
+                  if e["mode"] == "push" and p["frontier"] > 0]
+        assert all(0 < got <= edges for got, edges in pushes)
+        assert any(got < 0.8 * edges for got, edges in pushes)
+
+
 def test_copy_is_built_once_there_is_memory(hc, gpu):
     """With the device's memory taken the queries run on the plain CSR; the first
     one after it is given back builds the copy."""
