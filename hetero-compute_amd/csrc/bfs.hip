@@ -1019,9 +1019,6 @@ void free_bfs_ws(hc_graph_s *g) {
     g->ws_bfs = nullptr;
 }
 
-// Below this the edge array stays in cache anyway.
-constexpr int32_t kHead4MinNodes = 1 << 19;
-
 static int get_bfs_ws(hc_graph_s *g, BfsWs **out, hipStream_t s) {
     // The partial slots are sized for the launch grid; re-allocate when the
     // tuned grid changes.

@@ -737,6 +737,11 @@ __device__ void compact_body(const GraphView<OffT> &g, const FrontierBufs &fb,
     }
 }
 
+// Flat graphs of at least this many vertices keep each row's first four
+// neighbours beside the edge array for bottom-up levels; below, the edge array
+// stays in cache anyway.
+constexpr int32_t kHead4MinNodes = 1 << 19;
+
 // Graphs of up to this size run a direction-optimizing BFS as one workgroup
 // (many.hip): launch_bfs_small enqueues it; ctl[0] receives the final header
 // and the trace.

@@ -80,7 +80,9 @@ int64_t share_workspace_bound(int64_t n, int64_t m) {
                              4 * 4 * words + (int64_t)sizeof(unsigned long long) *
                              kSumWords * kSumSets + 64 * 1024;
     const int64_t sssp = frontier + 2 * n;                    // + 16-bit mirror
-    const int64_t bfs = frontier + 8 * n + 4 * (3 * (int64_t)grid_blocks() + 1);  // + depth, first
+    // + depth, first, and the first four neighbours
+    const int64_t bfs = frontier + 8 * n + (n >= kHead4MinNodes ? 16 * n : 0) +
+                        4 * (3 * (int64_t)grid_blocks() + 1);
     const int64_t multi = 3 * 4 * ((n + 3) / 4) + 4096;        // change flags
     // Bit-parallel batched BFS: seen and three frontier masks (8 bytes per
     // vertex each), three vertex lists, counters.

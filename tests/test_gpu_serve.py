@@ -132,6 +132,17 @@ def test_memory_budget_evicts_dynamic_graphs(hc, gpu, oracle, graphs):
         assert np.array_equal(m, ref)
 
 
+def test_charge_covers_the_head_array(hc, gpu):
+    """Flat graphs of at least 2^19 vertices keep 16 bytes per vertex and slot for
+    bottom-up levels; the charge has room for them."""
+    def path(n):
+        v = np.arange(n - 1, dtype=np.int32)
+        return hc.HostGraph.from_edges(v, v + 1, n)
+    with hc.Server(slots=2) as srv:
+        small, large = (srv.graph_bytes(path((1 << 19) + d), True) for d in (-1, 0))
+    assert large - small >= 2 * 16 << 19
+
+
 def test_below_batch_threshold_runs_single_source(hc, gpu, oracle, graphs):
     """Fewer waiting queries of one graph and kind than the batching
     threshold run one at a time on the single-source loops: with the BFS
