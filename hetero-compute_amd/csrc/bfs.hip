@@ -24,7 +24,7 @@
 #include <cstring>
 #include <vector>
 
-#include "frontier.h"
+#include "one_graph.h"
 
 namespace hc {
 
@@ -1121,6 +1121,47 @@ static void fill_bfs_stats(const StepCtl &fc, int32_t launches, hc_run_stats_t *
     stats->launches = launches;
     stats->reached = (int64_t)fc.reached;
     stats->alg_bytes = (double)fc.alg_bytes;
+}
+
+// Graphs of up to this size run a direction-optimizing BFS as one workgroup in
+// one launch: its levels take a few microseconds each, where the epoch loop's
+// two launches take a dozen (Kronecker, 4096 vertices: 173 -> 80 us a query with
+// its result fetched, and 74 with the final header in pinned memory).  ctl[0]
+// receives the final header and the trace.  (The kernel stands in this file
+// because a file's code is loaded when the first of its kernels runs, and the
+// many-graph one's holds a 32 MiB array: the first query of a process took 15 ms
+// there and takes 1.4 here.)
+constexpr int32_t kBfsSmallNodes = 1 << 15;
+constexpr int64_t kBfsSmallEdges = int64_t(1) << 20;
+constexpr int kSmallBlock = 1024;
+constexpr int kSmallHeavy = 1024;
+__global__ __launch_bounds__(kSmallBlock) void bfs_small_kernel(
+    const uint32_t *__restrict__ off, const int32_t *__restrict__ adj, int32_t n, int64_t m,
+    int32_t src, int32_t *__restrict__ depth, int32_t *__restrict__ parents, int alpha, int beta,
+    StepCtl *ctl) {
+    extern __shared__ uint32_t lds_bm[];
+    __shared__ int32_t heavy[kSmallHeavy];
+    __shared__ int s_nheavy;
+    __shared__ long long s_red[kSmallBlock / kWave];
+    ManyStats st{0, 0, 0};
+    const Desc d{0, 0, 0, n, 0, m};
+    bfs_one_graph<kSmallBlock, false, true>(d, src, off, adj, depth, parents, lds_bm,
+                                            (n + 31) / 32, alpha, beta, 8, kSmallHeavy, heavy,
+                                            &s_nheavy, s_red, st, ctl);
+}
+
+static bool bfs_is_small(const hc_graph_s *g) {
+    return !g->off64 && g->n <= kBfsSmallNodes && g->m <= kBfsSmallEdges && g->row0 == 0 &&
+           g->rows == g->n;
+}
+
+static int launch_bfs_small(const hc_graph_s *g, int32_t src, int32_t *depth, int32_t *parents,
+                     int alpha, int beta, StepCtl *ctl, hipStream_t s) {
+    const size_t lds = sizeof(uint32_t) * 3 * (size_t)((g->n + 31) / 32);
+    bfs_small_kernel<<<1, kSmallBlock, lds, s>>>(static_cast<const uint32_t *>(g->d_off), g->d_adj,
+                                                 g->n, g->m, src, depth, parents, alpha, beta, ctl);
+    HC_HIP(hipGetLastError());
+    return HC_OK;
 }
 
 template <typename OffT>

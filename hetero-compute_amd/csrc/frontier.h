@@ -742,15 +742,6 @@ __device__ void compact_body(const GraphView<OffT> &g, const FrontierBufs &fb,
 // stays in cache anyway.
 constexpr int32_t kHead4MinNodes = 1 << 19;
 
-// Graphs of up to this size run a direction-optimizing BFS as one workgroup
-// (many.hip): launch_bfs_small enqueues it; ctl[0] receives the final header
-// and the trace.
-constexpr int32_t kBfsSmallNodes = 1 << 15;
-constexpr int64_t kBfsSmallEdges = int64_t(1) << 20;
-bool bfs_is_small(const hc_graph_s *g);
-int launch_bfs_small(const hc_graph_s *g, int32_t src, int32_t *depth, int32_t *parents,
-                     int alpha, int beta, StepCtl *ctl, hipStream_t s);
-
 // Host loop shared by SSSP and BFS: enqueue `launch_epoch(arg, k)` for
 // epochs k = 0, 1, ... in batches and poll the done flag of the previous
 // batch while the next one is queued.  final_ctl: the last header with the

@@ -5,6 +5,10 @@ and bottom-up rows whose scan ends at, or just past, the neighbours read ahead
 valid, and bottom-up the first frontier neighbour."""
 from __future__ import annotations
 
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -97,3 +101,29 @@ def test_small_graphs_around_the_one_workgroup_limit(hc, gpu, oracle, n):
         assert np.array_equal(one.values, loop.values)
         for key in ("epochs", "push_epochs", "pull_epochs", "reached"):
             assert one.stats[key] == loop.stats[key], key
+
+
+FIRST_QUERY = """
+import importlib, sys
+sys.path.insert(0, sys.argv[1])
+hc = importlib.import_module("hetero-compute_amd")
+hc.check(hc.lib().hc_init(0))
+g = hc.HostGraph.generate("kron", 12, 16, weighted=False, seed=1)
+dg = hc.DeviceGraph(g)
+out = hc.DeviceArray(g.num_nodes, "int32")
+hc.synchronize()
+free, _ = hc.mem_get_info()
+hc.bfs(dg, 0, want_parents=False, depth_out=out, fetch=False)
+print("took", free - hc.mem_get_info()[0])
+"""
+
+
+def test_first_small_query_of_a_process_takes_little_memory(hc, gpu):
+    """A small graph's query loads the BFS loop's code only, not the many-graph
+    launch's with its 32 MiB scratch array (which is no part of a server's
+    budget either)."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(hc.__file__)))
+    run = subprocess.run([sys.executable, "-c", FIRST_QUERY, root], capture_output=True, text=True,
+                         timeout=100)
+    assert run.returncode == 0, run.stderr[-2000:]
+    assert int(run.stdout.split()[-1]) < 32 << 20
