@@ -176,7 +176,8 @@ __device__ __forceinline__ double pr_finalize(const PrEpoch &ep, const double *i
     return pr_finalize(ep, u, k, ep.s_in[u], inv_deg[u]);
 }
 
-constexpr int64_t kPrHubMin = 2048;  // edges a row has at least to be cut into chunks
+constexpr int64_t kPrHubMin = 1024;  // edges a row has at least to be cut into chunks
+constexpr int64_t kPrChunkMin = 2048;
 // A sweep runs in workgroups of 16 wavefronts, one per CU where the LDS copy
 // of the hubs' contributions takes most of its LDS; each wavefront takes rows
 // and chunks by itself.
@@ -239,8 +240,8 @@ __device__ __forceinline__ void pr_rows(const PlanDev &p, int c, int &start, int
 }
 
 // One Jacobi sweep over the plan's rows and the zero-degree vertices.
-// Returns this thread's residual contribution (hub residuals go to
-// b.hub_resid instead).
+// Returns this thread's residual contribution (the hubs' is added where their
+// chunks are).
 // contrib is read-only within a sweep, so the LDS snapshot of its hub entries
 // (staged from ep.c_in) is exact.
 template <typename OffT>
@@ -557,21 +558,28 @@ static int get_pr_ws(hc_graph_s *g, int32_t chunks, PrWs **out) {
     return HC_OK;
 }
 
-// Degree classes of a sweep: a wavefront takes a row or a chunk by itself, so
-// a row is cut into chunks once it would keep its wavefront longer than an
-// even share of all edges would, but not below kPrHubMin edges (8 trips),
+// Degree classes of a sweep over [start, end): a wavefront takes a row or a chunk
+// by itself, so a row is cut into chunks once it would keep its wavefront longer
+// than an even share of the range's edges would, but not below kPrHubMin edges,
 // since the one workgroup that adds up the chunks takes longer with each hub
-// (21 us a sweep with 2.3K of them).
-static PlanConfig pr_plan_config(const hc_graph_s *g) {
+// (21 us a sweep with 2.3K of them).  Kronecker in no order of degree, 1M
+// vertices, a 64th of the rows: 82 us with the share of the whole graph, 34 so
+// (38 with a workgroup per such row).  A chunk is a quarter of such a share, from
+// kPrChunkMin edges on (1M vertices as above, whole, 31M edges: 281 us a sweep
+// with chunks of 4096, 260 with 2048; 4M vertices, 128M edges: 1370 and 1362, in
+// order of degree 518 and 538).
+static PlanConfig pr_plan_config(const hc_graph_s *g, int32_t start, int32_t end) {
     PlanConfig c = tuning().pull;
-    const int64_t share = g->m / (int64_t(kPrWaves) * device_state().cus);
+    const int64_t edges = g->h_off[end - g->row0] - g->h_off[start - g->row0];
+    const int64_t share = edges / (int64_t(kPrWaves) * device_state().cus);
     const int64_t cut = std::max<int64_t>(share, kPrHubMin);
     if (c.hub_threshold > cut) c.hub_threshold = cut;
     if (c.block_threshold > c.hub_threshold) c.block_threshold = c.hub_threshold;
     if (c.wave_threshold > c.block_threshold) c.wave_threshold = c.block_threshold;
     if (c.g16_threshold > c.wave_threshold) c.g16_threshold = c.wave_threshold;
     if (c.g4_threshold > c.g16_threshold) c.g4_threshold = c.g16_threshold;
-    c.hub_chunk = std::min<int64_t>(c.hub_chunk, std::max<int64_t>(c.hub_threshold, kPrHubMin));
+    c.hub_chunk = std::min<int64_t>({c.hub_chunk, std::max<int64_t>(share / 4, kPrChunkMin),
+                                     std::max<int64_t>(c.hub_threshold, kPrHubMin)});
     return c;
 }
 
@@ -612,7 +620,7 @@ template <typename OffT>
 static int run_pr(hc_graph_s *g, float *scores, float damp, double tol,
                   int max_iters, int rule, hc_run_stats_t *stats, hipStream_t s) {
     const PlanHost *ph = nullptr;
-    HC_TRY(get_plan(g, 0, g->n, pr_plan_config(g), &ph));
+    HC_TRY(get_plan(g, 0, g->n, pr_plan_config(g, 0, g->n), &ph));
     PrWs *ws = nullptr;
     HC_TRY(get_pr_ws(g, ph->dev.cnt[0], &ws));
     GraphView<OffT> v = view<OffT>(g);
@@ -690,7 +698,7 @@ static int run_pr_pull(hc_graph_s *g, int mapping, const float *init, float *sco
                        double tol, int max_iters, int rule, int blocks, int threads,
                        hc_run_stats_t *stats, hipStream_t s) {
     const PlanHost *ph = nullptr;
-    if (mapping == HC_MAP_BUCKETED) HC_TRY(get_plan(g, 0, g->n, pr_plan_config(g), &ph));
+    if (mapping == HC_MAP_BUCKETED) HC_TRY(get_plan(g, 0, g->n, pr_plan_config(g, 0, g->n), &ph));
     PrWs *ws = nullptr;
     HC_TRY(get_pr_ws(g, ph ? ph->dev.cnt[0] : 0, &ws));
     GraphView<OffT> v = view<OffT>(g);
@@ -857,7 +865,7 @@ int hc_pr_pull_epoch(hc_graph_t g, int32_t start_id, int32_t end_id,
     GraphCall call(g);
     hipStream_t s = pick_stream(stream);
     const PlanHost *ph = nullptr;
-    HC_TRY(get_plan(g, start_id, end_id, pr_plan_config(g), &ph));
+    HC_TRY(get_plan(g, start_id, end_id, pr_plan_config(g, start_id, end_id), &ph));
     PrWs *ws = nullptr;
     HC_TRY(get_pr_ws(g, ph->dev.cnt[0], &ws));
     PrBufs b{inv_degree, ws->hub_hi, ws->hub_lo, ws->partials};

@@ -63,3 +63,34 @@ def test_row_counts_and_stops(hc, gpu, oracle, n):
             assert abs(r.stats["residual"] - np.abs(ref - prev).sum()) <= 2 * L1_TOL
             assert it == 20 if tol < 0 else r.stats["residual"] < tol or it == 20
         assert np.array_equal(hc.pagerank(dg).values, hc.pagerank(dg).values)
+
+
+@pytest.mark.parametrize("held", [False, True])
+@pytest.mark.parametrize("shuffle", [False, True])
+def test_epochs_over_ranges(hc, gpu, shuffle, held):
+    """One epoch range by range, of the whole graph or of a handle that holds the
+    range's rows only: rows are cut into chunks by the range's own edges.  Each
+    score is rounded six times (see L1_TOL)."""
+    rng = np.random.default_rng(4)
+    g = _stars(hc, [1, 5, 24, 192, 1023, 1024, 1025, 2047, 2049, 4097, 8193, 20000], 20000, rng,
+               shuffle)
+    n = g.num_nodes
+    contrib = (rng.random(n) / n).astype(np.float32)
+    s_in = rng.random(n).astype(np.float32)
+    inv = 1.0 / np.maximum(1, np.diff(g.index))
+    sums = np.add.reduceat(np.append(contrib[g.neighbors].astype(np.float64), 0.0), g.index[:-1])
+    ref = np.float32(0.15) / n + np.float32(0.85) * np.where(np.diff(g.index) > 0, sums, 0.0)
+    bufs = [hc.DeviceArray.from_host(x) for x in (s_in, contrib, inv)]
+    s_out, c_out = (hc.DeviceArray.from_host(np.zeros(n, np.float32)) for _ in range(2))
+    whole = None if held else hc.DeviceGraph(g)
+    cuts = [0, 1, 6, 12, 13, 500, n // 2, n // 2 + 64, n]
+    resid = 0.0
+    for a, b in zip(cuts, cuts[1:]):
+        dg = hc.DeviceGraph(g, a, b) if held else whole
+        resid += hc.pr_pull_epoch(dg, a, b, 0.85, *bufs, s_out, c_out)
+        if held:
+            dg.free()
+    got = s_out.get().astype(np.float64)
+    assert (np.abs(got - ref) <= 6 * 2.0**-24 * ref).all()
+    assert np.abs(c_out.get() - got * inv).max() <= 2.0**-24 * (got * inv).max()
+    assert abs(resid - np.abs(got - s_in).sum()) <= 1e-9 * resid
