@@ -170,6 +170,53 @@ constexpr int kMsGroup = 16;
 constexpr int kMsTrip = 4;                      // edges a lane has in flight
 constexpr int kMsChunk = kMsGroup * kMsTrip;
 constexpr int kMsPer = kMsWindow / kBlock;
+// A list of no more edges than this, and of no more than kMsFewMean a vertex (a
+// hub's would be one wavefront's: Kronecker 256K vertices, four sources, 398 ->
+// 494 us), skips the windows, whose offsets, barriers and search make a longer
+// chain than the edges do (grid of 256^2 vertices, one source, 510 levels: 16.9
+// us a push with them, 10.4 without).
+constexpr unsigned long long kMsFewMean = 16;
+constexpr unsigned long long kMsFewEdges = 8192;
+
+// Exclusive chunk offsets of a window's n vertices in s_pre, P of them per thread
+// (as few as cover n: they are a chain of loads, and a deep graph's short lists
+// wait for it); returns their sum.
+template <int P, typename OffT>
+__device__ __forceinline__ uint32_t ms_window_offsets(const GraphView<OffT> &g, const int32_t *wl,
+                                                      int n, uint32_t *s_pre, uint32_t *s_wave) {
+    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    uint32_t mine[P], t = 0;
+#pragma unroll
+    for (int k = 0; k < P; k++) {
+        const int i = threadIdx.x * P + k;
+        uint32_t ch = 0;
+        if (i < n) {
+            const int32_t u = wl[i];
+            ch = (uint32_t)((g.rend(u) - g.rbeg(u) + OffT(kMsChunk - 1)) / OffT(kMsChunk));
+        }
+        mine[k] = t;
+        t += ch;
+    }
+    uint32_t incl = t;
+#pragma unroll
+    for (int s = 1; s < kWave; s <<= 1) {
+        const uint32_t o = __shfl_up(incl, s, kWave);
+        if (lane >= s) incl += o;
+    }
+    __syncthreads();  // the window before is done with s_pre
+    if (lane == kWave - 1) s_wave[wave] = incl;
+    __syncthreads();
+    uint32_t before = incl - t, total = 0;
+    for (int w = 0; w < kWavesPerBlock; w++) {
+        if (w < wave) before += s_wave[w];
+        total += s_wave[w];
+    }
+#pragma unroll
+    for (int k = 0; k < P; k++)
+        if (threadIdx.x * P + k < (unsigned)kMsWindow) s_pre[threadIdx.x * P + k] = before + mine[k];
+    __syncthreads();
+    return total;
+}
 
 // Workgroups per window of a push from `len` vertices with `deg` edges.
 __host__ __device__ inline int ms_push_share(unsigned long long len, unsigned long long deg,
@@ -199,45 +246,84 @@ __global__ __launch_bounds__(kBlock) void ms_push_kernel(MsBufs b, GraphView<Off
     // length read here is level L-1's, final since its commit.
     const unsigned long long len = b.cnt[cu].len;
     const int per = ms_push_share(len, b.cnt[cu].deg, gridDim.x);
-    const unsigned long long wins = (len + kMsWindow - 1) / kMsWindow;
+    const bool few = b.cnt[cu].deg <= min(kMsFewEdges, kMsFewMean * len);
+    const unsigned long long wins = few ? 0 : (len + kMsWindow - 1) / kMsWindow;
     const int lane = lane_id(), wave = threadIdx.x / kWave;
     MsStage st{s_stage[wave], 0};
     unsigned long long deg_acc = 0, edges = 0;
+    // The next masks of a trip's targets (-1: none) of a frontier vertex with
+    // mask fu.
+    auto take = [&](const int32_t (&v)[kMsTrip], uint64_t fu) {
+                    uint64_t bits[kMsTrip], have[kMsTrip];
+#pragma unroll
+                    for (int r = 0; r < kMsTrip; r++) {
+                        bits[r] = v[r] >= 0 ? fu & ~b.seen[v[r]] : 0;
+                        have[r] = v[r] >= 0 ? nxt[v[r]] : 0;
+                    }
+                    bool fresh[kMsTrip];
+#pragma unroll
+                    for (int r = 0; r < kMsTrip; r++) {
+                        edges += v[r] >= 0;
+                        // An atomic only when it adds a bit the next mask lacks.
+                        fresh[r] = (bits[r] & ~have[r]) != 0 &&
+                                   atomicOr((unsigned long long *)&nxt[v[r]],
+                                            (unsigned long long)bits[r]) == 0;
+                    }
+#pragma unroll
+                    for (int r = 0; r < kMsTrip; r++) {
+                        if (fresh[r]) deg_acc += (unsigned long long)(g.rend(v[r]) - g.rbeg(v[r]));
+                        ms_stage_append(st, fresh[r], v[r]);
+                    }
+        if (st.n > kMsStage - kMsTrip * kWave) ms_stage_flush(st, nq, c);
+    };
+    if (few) {
+        // A few edges: four lanes a vertex, and the wavefront together for what
+        // a vertex has beyond kMsChunk.
+        constexpr int G = 4, PER = kWave / G;
+        const unsigned long long waves = (unsigned long long)gridDim.x * kWavesPerBlock;
+        for (unsigned long long q0 =
+                 (blockIdx.x * (unsigned long long)kWavesPerBlock + wave) * PER;
+             q0 < len; q0 += waves * PER) {
+            const bool ok = q0 + lane / G < len;
+            const int32_t u = ok ? list[q0 + lane / G] : 0;
+            const OffT ub = ok ? g.rbeg(u) : OffT(0), ue = ok ? g.rend(u) : OffT(0);
+            const uint64_t fu = ok ? cur[u] : 0;
+            const OffT mid = min(ue, ub + OffT(kMsChunk));
+            for (OffT t = 0; t < OffT(kMsChunk); t += OffT(kMsTrip * G)) {
+                if (__ballot(ub + t < mid) == 0) break;
+                int32_t v[kMsTrip];
+#pragma unroll
+                for (int r = 0; r < kMsTrip; r++) {
+                    const OffT k = ub + t + OffT(r * G + lane % G);
+                    v[r] = k < mid ? ldnt(&g.adj[k]) : -1;
+                }
+                take(v, fu);
+            }
+            for (uint64_t hv = __ballot(lane % G == 0 && mid < ue); hv; hv &= hv - 1) {
+                const int l = __ffsll((unsigned long long)hv) - 1;
+                const OffT e = __shfl(ue, l);
+                const uint64_t hfu = (uint64_t)__shfl((unsigned long long)fu, l);
+                for (OffT i = __shfl(mid, l); i < e; i += OffT(kMsTrip * kWave)) {
+                    int32_t v[kMsTrip];
+#pragma unroll
+                    for (int r = 0; r < kMsTrip; r++) {
+                        const OffT k = i + OffT(r * kWave + lane);
+                        v[r] = k < e ? ldnt(&g.adj[k]) : -1;
+                    }
+                    take(v, hfu);
+                }
+            }
+        }
+    }
     const int sub = blockIdx.x % per;
     for (unsigned long long win = blockIdx.x / per; win < wins; win += gridDim.x / per) {
         if (blockIdx.x / per >= gridDim.x / per) break;  // past the last full share
         const int n = (int)min((unsigned long long)kMsWindow, len - win * kMsWindow);
         const int32_t *wl = list + win * kMsWindow;
-        // Exclusive chunk offsets of the window's vertices, kMsPer per thread.
-        uint32_t mine[kMsPer], t = 0;
-#pragma unroll
-        for (int k = 0; k < kMsPer; k++) {
-            const int i = threadIdx.x * kMsPer + k;
-            uint32_t ch = 0;
-            if (i < n) {
-                const int32_t u = wl[i];
-                ch = (uint32_t)((g.rend(u) - g.rbeg(u) + OffT(kMsChunk - 1)) / OffT(kMsChunk));
-            }
-            mine[k] = t;
-            t += ch;
-        }
-        uint32_t incl = t;
-#pragma unroll
-        for (int s = 1; s < kWave; s <<= 1) {
-            const uint32_t o = __shfl_up(incl, s, kWave);
-            if (lane >= s) incl += o;
-        }
-        __syncthreads();  // the window before is done with s_pre
-        if (lane == kWave - 1) s_wave[wave] = incl;
-        __syncthreads();
-        uint32_t before = incl - t, total = 0;
-        for (int w = 0; w < kWavesPerBlock; w++) {
-            if (w < wave) before += s_wave[w];
-            total += s_wave[w];
-        }
-#pragma unroll
-        for (int k = 0; k < kMsPer; k++) s_pre[threadIdx.x * kMsPer + k] = before + mine[k];
-        __syncthreads();
+        uint32_t total;
+        if (n <= kBlock) total = ms_window_offsets<1>(g, wl, n, s_pre, s_wave);
+        else if (n <= 4 * kBlock) total = ms_window_offsets<4>(g, wl, n, s_pre, s_wave);
+        else total = ms_window_offsets<kMsPer>(g, wl, n, s_pre, s_wave);
         // Chunks in rounds of the wavefront's groups (the same count in all
         // its lanes).
         constexpr int kGroups = kWave / kMsGroup;
@@ -267,27 +353,7 @@ __global__ __launch_bounds__(kBlock) void ms_push_kernel(MsBufs b, GraphView<Off
 #pragma unroll
                 for (int r = 0; r < kMsTrip; r++) v[r] = -1;
             }
-            uint64_t bits[kMsTrip], have[kMsTrip];
-#pragma unroll
-            for (int r = 0; r < kMsTrip; r++) {
-                bits[r] = v[r] >= 0 ? fu & ~b.seen[v[r]] : 0;
-                have[r] = v[r] >= 0 ? nxt[v[r]] : 0;
-            }
-            bool fresh[kMsTrip];
-#pragma unroll
-            for (int r = 0; r < kMsTrip; r++) {
-                edges += v[r] >= 0;
-                // An atomic only when it adds a bit the next mask lacks.
-                fresh[r] = (bits[r] & ~have[r]) != 0 &&
-                           atomicOr((unsigned long long *)&nxt[v[r]],
-                                    (unsigned long long)bits[r]) == 0;
-            }
-#pragma unroll
-            for (int r = 0; r < kMsTrip; r++) {
-                if (fresh[r]) deg_acc += (unsigned long long)(g.rend(v[r]) - g.rbeg(v[r]));
-                ms_stage_append(st, fresh[r], v[r]);
-            }
-            if (st.n > kMsStage - kMsTrip * kWave) ms_stage_flush(st, nq, c);
+            take(v, fu);
         }
     }
     ms_stage_flush(st, nq, c);
@@ -583,11 +649,14 @@ __global__ __launch_bounds__(kBlock) void ms_pull_cb_kernel(MsBufs b, GraphView<
 }
 
 // Commit of level L: depth entries of the new bits, seen updated.  A
-// wavefront takes 64 listed vertices: their masks are read at once, a lane
-// each, then their rows are written one after another, lane q source q's
-// entry (with a vertex per wavefront the chain list, mask, row bounded the
-// level: 420 us for 2.3 M vertices of Kronecker 22).  Resets the counters of
+// wavefront takes up to 64 listed vertices, as many as give every wavefront
+// some: their masks are read at once, a lane each, then their rows are written
+// one after another, lane q source q's entry (with a vertex per wavefront the
+// chain list, mask, row bounded a long level: 420 us for 2.3 M vertices of
+// Kronecker 22; with 64 a short one of some hundred vertices took 8 us, and 4
+// so).  Resets the counters of
 // buffer (L+1) % 3, which level L+1 fills.
+constexpr int kMsCommitMin = 4;
 __global__ __launch_bounds__(kBlock) void ms_commit_kernel(MsBufs b, int L) {
     const int nx = L % 3;
     const uint64_t *nxt = b.fr[nx];
@@ -595,11 +664,13 @@ __global__ __launch_bounds__(kBlock) void ms_commit_kernel(MsBufs b, int L) {
     const unsigned long long len = b.cnt[nx].len;
     const int lane = lane_id();
     unsigned long long bits = 0;
-    const unsigned long long step = (unsigned long long)gridDim.x * kBlock;
-    for (unsigned long long i0 = blockIdx.x * (unsigned long long)kBlock +
-                                 (threadIdx.x / kWave) * kWave;
-         i0 < len; i0 += step) {
-        const int n = (int)min((unsigned long long)kWave, len - i0);
+    const unsigned long long waves = (unsigned long long)gridDim.x * kWavesPerBlock;
+    const unsigned long long per =
+        min((unsigned long long)kWave, max((unsigned long long)kMsCommitMin, len / 256));
+    for (unsigned long long i0 = (blockIdx.x * (unsigned long long)kWavesPerBlock +
+                                  threadIdx.x / kWave) * per;
+         i0 < len; i0 += waves * per) {
+        const int n = (int)min(per, len - i0);
         int32_t v = 0;
         uint64_t nb = 0;
         if (lane < n) {

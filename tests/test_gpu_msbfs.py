@@ -70,3 +70,29 @@ def test_push_windows(hc, gpu, oracle, size):
         r = hc.bfs_multi(dg, sources)
         for q, s in enumerate(sources):
             assert np.array_equal(r.values[q], oracle.bfs_depth(g.index, g.neighbors, s)), q
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("leaves", [1, 61, 62, 63, 190, 255, 256, 257, 1100])
+def test_short_lists(hc, gpu, oracle, monkeypatch, leaves, wide):
+    """A ladder of 40 rungs of 80 vertices whose every tenth rung has one vertex
+    with `leaves` leaves: lists of some hundred edges, rows on both sides of a
+    group's 64 edges and of a wavefront's 256 beyond them, and of the mean up to
+    which a list is short."""
+    if wide:
+        monkeypatch.setenv("HC_FORCE_OFF64", "1")
+    width, rungs = 80, 40
+    v = np.arange(width * (rungs - 1))
+    hubs = width * np.arange(0, rungs, 10) + 7
+    n = width * rungs + leaves * hubs.size
+    src = np.concatenate([v, v, np.repeat(hubs, leaves)])
+    dst = np.concatenate([v + width, v // width * width + width + (v + 1) % width,
+                          width * rungs + np.arange(leaves * hubs.size)])
+    p = np.random.default_rng(leaves).permutation(n)
+    g = hc.HostGraph.from_edges(p[src].astype(np.int32), p[dst].astype(np.int32), n)
+    hc.set_tuning("msbfs.alpha", 1)
+    with hc.DeviceGraph(g) as dg:
+        for sources in ([p[0]], p[[7, 8, n - 1]], p[:64]):
+            r = hc.bfs_multi(dg, sources)
+            for q, s in enumerate(sources):
+                assert np.array_equal(r.values[q], oracle.bfs_depth(g.index, g.neighbors, int(s)))
