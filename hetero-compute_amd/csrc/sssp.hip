@@ -1690,7 +1690,13 @@ static int run_sssp_loop(hc_graph_s *g, int32_t src, const int32_t *init_dist,
     // which tests a changed bit per neighbour before its gather).
     const ColBlocks *cb = nullptr;
     const PlanHost *phb = nullptr;
-    if (!sorted && delta == 0 && direction != 2 && tuning().sssp_filter != 1) {
+    // A loop that pulls only its few heavy epochs gains nothing from the blocks of
+    // a small graph, and the first query would build them (uniform, 2M vertices,
+    // 8.4 M edges, weights 1..3: 1.01 ms a query either way, the first 2.37 ms
+    // with and 2.07 without).
+    const bool blocks = t.pull_col_shift > 0 || init_dist || direction == 1 ||
+                        g->m >= kSortedMinEdges;
+    if (!sorted && delta == 0 && direction != 2 && tuning().sssp_filter != 1 && blocks) {
         HC_TRY(get_col_blocks(g, col_shift_for(g, flat_graph(g)), s, &cb));
         if (cb) {
             // Plain sweep for the light rows only.
