@@ -123,8 +123,14 @@ def run_graph(hc, kind, scale, degree, steps, warmup, seed, tuned=None):
 
 def kernel_roofline(hc, res, algo, count):
     """Average launch duration and algorithmic bytes of the step kernel
-    (sssp_step_kernel / bfs_step_kernel) from HIP events around each launch."""
+    (bfs_step_kernel; sssp_sorted_step_kernel where the weight-sorted adjacency
+    is used, else sssp_step_kernel) from HIP events around each launch."""
     dg = res["dg"]
+    kernel = f"{algo}_step_kernel"
+    if algo == "sssp":
+        sort = hc.get_tuning("sssp.sorted")
+        if sort == 2 or (sort == 1 and dg.info()["num_edges"] >= 1 << 23):
+            kernel = "sssp_sorted_step_kernel"
     n = res["n"]
     buf = hc.DeviceArray(n, np.int32)
     hc.set_tuning("profile.kernel_events", 1)
@@ -147,7 +153,7 @@ def kernel_roofline(hc, res, algo, count):
     achieved = per_launch / avg_s / 1e9
     return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
-            "kernel": f"{algo}_step_kernel", "avg_launch_us": round(avg_s * 1e6, 2),
+            "kernel": kernel, "avg_launch_us": round(avg_s * 1e6, 2),
             "alg_bytes_per_launch": round(per_launch, 1), "launches_timed": k_launch,
             "sources_timed": count}
 
@@ -897,13 +903,16 @@ def main():
     # the headline itself).  The dominant kernel (the algorithm with the
     # larger share of device time on the headline graph) is `roofline`.
     rooflines = {}
+    main_rf = {}
     for kind, r in results.items():
         for a in ("sssp", "bfs"):
             rf = kernel_roofline(hc, r, a, min(args.steps, args.roofline_sources))
             rf["traffic"] = committed_traffic(rf["kernel"], f"{kind}{args.scale}")
             rooflines[f"{rf['kernel']}_{kind}{args.scale}"] = rf
+            if kind == main_kind:
+                main_rf[a] = rf
     algo = "sssp" if R["sssp_ms"].sum() >= R["bfs_ms"].sum() else "bfs"
-    roofline = dict(rooflines[f"{algo}_step_kernel_{main_kind}{args.scale}"])
+    roofline = dict(main_rf[algo])
     if pr is not None:
         rooflines[f"pr_step_kernel_kron{args.pr_scale}"] = pr["roofline"]
 
