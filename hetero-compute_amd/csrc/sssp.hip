@@ -511,7 +511,7 @@ struct RowSums {
 template <int G, int R, typename OffT>
 __device__ __forceinline__ bool sorted_trip(const SortedView &sv, const int32_t *dist, OffT i,
                                             OffT e, int lane, int32_t low, int32_t &best,
-                                            int32_t &m, uint32_t &gathered) {
+                                            int32_t &m, uint32_t &pairs, uint32_t &gathered) {
     int2 x[R];
     bool in[R];
 #pragma unroll
@@ -519,6 +519,7 @@ __device__ __forceinline__ bool sorted_trip(const SortedView &sv, const int32_t 
         const OffT k = i + OffT(r * G + lane);
         in[r] = k < e;
         x[r] = in[r] ? sv.e[k] : int2{0, 0};
+        pairs += in[r] ? 1u : 0u;
     }
     int32_t d[R];
 #pragma unroll
@@ -550,15 +551,11 @@ __device__ __forceinline__ int32_t sorted_row_min(const SortedView &sv, const in
                                                   int32_t low, uint32_t &pairs,
                                                   uint32_t &gathered) {
     int32_t best = cur, m = HC_INF_DIST;
-    OffT i = b + OffT(2 * G);
-    if (sorted_trip<G, 2>(sv, dist, b, e, lane, low, best, m, gathered)) {
-        // (8-byte offsets take the registers of the longer trip)
-        constexpr int R = sizeof(OffT) == 8 ? 2 : 4;
-        bool more = true;
-        for (; more && i < e; i += OffT(R * G))
-            more = sorted_trip<G, R>(sv, dist, i, e, lane, low, best, m, gathered);
-    }
-    if (lane == 0) pairs += (uint32_t)(min(i, e) - b);
+    if (!sorted_trip<G, 2>(sv, dist, b, e, lane, low, best, m, pairs, gathered)) return m;
+    // (8-byte offsets take the registers of the longer trip)
+    constexpr int R = sizeof(OffT) == 8 ? 2 : 4;
+    for (OffT i = b + OffT(2 * G); i < e; i += OffT(R * G))
+        if (!sorted_trip<G, R>(sv, dist, i, e, lane, low, best, m, pairs, gathered)) break;
     return m;
 }
 
