@@ -532,7 +532,10 @@ constexpr int kSortKeys = 64;
 // 0.40 -> 0.33 ms a query, but 0.53 -> 0.98 ms the first; 31 M edges: 1.13 ->
 // 0.50 ms, the first 1.83 -> 1.85 ms).
 constexpr int64_t kSortedMinEdges = int64_t(1) << 23;
-constexpr int64_t kSortedMinBatchEdges = int64_t(1) << 20;  // batched sweeps
+// Batched sweeps: 64 sources, uniform graphs of 0.5, 1.05 and 2.1 M edges, 1.29,
+// 2.03 and 2.62 ms a batch on the plain CSR, 1.39, 2.06 and 2.61 so; Kronecker, 0.4
+// and 1.8 M edges: 3.29 and 3.03 against 1.43 and 1.22.
+constexpr int64_t kSortedMinBatchEdges = int64_t(1) << 20;
 struct SortedView {
     const int2 *e;
     int32_t shift;

@@ -226,8 +226,9 @@ int hc_graph_get_info(hc_graph_t g, hc_graph_info_t *out);
  *                          of at least 2^23 edges (or where sssp.delta sets
  *                          buckets), 2 on all, 0 on none.  The plain CSR is
  *                          used all the same when there is no memory for the
- *                          copy, and when sssp.filter, sssp.dist16 = 1 or
- *                          pull.col_shift > 0 asks for another sweep (1)
+ *                          copy (the next query tries again), and when
+ *                          sssp.filter, sssp.dist16 = 1 or pull.col_shift > 0
+ *                          asks for another sweep (1)
  *   sssp.grid_per_cu       cap on workgroups per CU of the SSSP loop (4)
  *   sssp.filter            1: SSSP pull epochs gather only neighbours whose
  *                          distance changed in the previous epoch; k >= 2:
@@ -320,6 +321,8 @@ int hc_graph_get_info(hc_graph_t g, hc_graph_info_t *out);
  *                          plus K (n+1) offsets; at most 32 blocks); 0 off,
  *                          6..30 on every graph, -1 (default) automatic:
  *                          flat graphs only, four blocks of >= 2^20 vertices
+ *                          (hc_sssp on the plain CSR: from 2^23 edges, or with
+ *                          direction 1)
  *   cb.min_slice           rows of degree above this x blocks are swept block
  *                          by block, lighter rows once over the plain CSR (4)
  *   cb.g4_slice / cb.g16_slice / cb.wave_slice / cb.block_slice   mean

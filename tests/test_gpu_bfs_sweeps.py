@@ -31,10 +31,13 @@ def _check(hc, oracle, g, sources, directions=(0, 1, 2)):
             assert 1 + sum(e["frontier"] for e in tr) == reached
 
 
+@pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("leaves", [5000, 560000, 900000])
-def test_heavy_top_down_epochs(hc, gpu, oracle, leaves):
+def test_heavy_top_down_epochs(hc, gpu, oracle, monkeypatch, leaves, wide):
     """Twelve hubs over a pool of leaves and a tail behind the leaves: the
     second epoch pushes 12 * leaves / 8 edges, many to the same leaves."""
+    if wide:
+        monkeypatch.setenv("HC_FORCE_OFF64", "1")
     rng = np.random.default_rng(leaves)
     hubs, tail = 12, 70
     per = leaves // 8
