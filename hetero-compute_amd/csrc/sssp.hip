@@ -1157,7 +1157,8 @@ __device__ void sssp_decide(StepCtl *c, StepCtl *trace,
             // Heavy: past the limit, or about to be if it outgrows the bucket
             // before it as that one did the one before.
             if (c->sorted && (c->bucket_e + (long long)out_e > light ||
-                              (ran == kPromote && c->prev_e > light * c->prev2_e / c->prev_e)))
+                              (ran == kPromote && (double)c->prev_e * (double)c->prev_e >
+                                                      (double)light * (double)c->prev2_e)))
                 c->far_on = 0;
             // The bucket goes on: by a sweep of the rows above its lowest
             // pending value while the frontier is heavy, else by a push.
@@ -1314,7 +1315,7 @@ __global__ __launch_bounds__(kBlock) void sssp_init_kernel(
         ctl->promotions = 0;
         ctl->bucket_e = 0;
         ctl->done_e = 0;
-        ctl->prev_e = ctl->prev2_e = m > 0 ? m : 1;
+        ctl->prev_e = ctl->prev2_e = m;
         ctl->far_on = delta > 0;
         ctl->far_live = 0;
         ctl->reached = 0;

@@ -123,13 +123,17 @@ def test_flat_buckets_cover_every_settling_path(hc, gpu, oracle):
                     assert np.array_equal(hc.sssp(dg, s, direction=2).values, ref), (top, delta)
 
 
+@pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("top", [3, 255, 100000])
-def test_buckets_turn_light_and_heavy(hc, gpu, oracle, top):
-    """Two dense cores joined by a long path, with a tail and unreached vertices
-    behind: buckets start light (the far set), turn heavy in a core (scans and
-    sweeps), light again on the path, and heavy in the second core."""
+def test_buckets_turn_light_and_heavy(hc, gpu, oracle, monkeypatch, top, wide):
+    """Two dense cores of 800K edges joined by a long path, with a tail and
+    unreached vertices behind: buckets start light (the far set), turn heavy in a
+    core (scans and sweeps), light again on the path, and heavy in the second
+    core."""
+    if wide:
+        monkeypatch.setenv("HC_FORCE_OFF64", "1")
     rng = np.random.default_rng(top)
-    core, path = 12000, 600
+    core, path = 40000, 600
     src, dst = [], []
     for base in (0, core + path):
         src.append(base + rng.integers(0, core, 10 * core))
